@@ -688,7 +688,7 @@ static int ensure_grid(bbfmm_amd_plan *p)
     // the MFMA forms on the plan's width (the particle-row form's vectors)
     const int gv = form != BBFMM_M2L_PLAIN ? p->width : p->nrhs;
     BB_TRY(grid_m2l_create(&p->grid, p->r, p->maxlev, gv, form, p->h_K.data(), p->stream, minlev, variant,
-                           variant_up, upper_split));
+                           variant_up, upper_split, p->d_Kc));
     p->grid_form = form;
     p->grid_minlev = minlev;
     p->grid_variant = variant;
@@ -1218,8 +1218,10 @@ extern "C" int bbfmm_amd_plan_tune(bbfmm_amd_plan *p, int reps, double *table, i
           for (int u : {1, 4, 5})
             if (u != v) cands.push_back({M2L_SCHEME_IJ, v, kMinLev, u});
     } else if (p->r == 32) {
-      for (int sw : sws)
+      for (int sw : sws) {
+        if (p->form == BBFMM_M2L_FP32MFMA) cands.push_back({M2L_SCHEME_IJ, 0, sw, 0});  // a block shape neither of 2, 3
         for (int v = 2; v <= 3; v++) cands.push_back({M2L_SCHEME_IJ, v, sw, 0});
+      }
     } else {
       for (int sw : sws) cands.push_back({M2L_SCHEME_IJ, 0, sw, 0});
     }
@@ -1872,7 +1874,7 @@ extern "C" int m2l_drv(int r, real *L, real *K, real *M, int minlev, int maxlev,
     else if (scheme == M2L_SCHEME_SI) rc = launch_m2l_sibling(m, nullptr);
     else if (scheme == M2L_SCHEME_CL && r <= kClusterMaxRank) rc = launch_m2l_cluster(m, nullptr);
     else {
-      rc = grid_m2l_create(&p.grid, r, maxlev, 1, BBFMM_M2L_PLAIN, p.h_K.data(), nullptr, minlev, 0);
+      rc = grid_m2l_create(&p.grid, r, maxlev, 1, BBFMM_M2L_PLAIN, p.h_K.data(), nullptr, minlev, 0, 0, 1, p.d_Kc);
       if (rc == BBFMM_OK) rc = grid_m2l_run(p.grid, p.d_M, dL, ncell, nullptr, nullptr);
     }
     if (rc != BBFMM_OK) break;

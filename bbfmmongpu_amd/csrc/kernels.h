@@ -136,11 +136,15 @@ struct GridM2L;  // defined in m2l_grid.hip
 // for the levels above the deepest (then two launches); upper_split: that
 // launch takes each class group's steps in this many parts (1..16), one
 // block each, whose partial sums are added afterwards
+// K_dev: the same column-major operators on the device (optional; then the
+// host copy is not uploaded again by the full-precision forms)
 int grid_m2l_create(GridM2L **g, int r, int maxlev, int nrhs, int form, const real *K_colmajor_host,
-                    hipStream_t s, int minlev, int variant, int variant_upper = 0, int upper_split = 1);
+                    hipStream_t s, int minlev, int variant, int variant_upper = 0, int upper_split = 1,
+                    const real *K_dev = nullptr);
 void grid_m2l_destroy(GridM2L *g);
-// flat = 1: the split-BF16 source-stationary kernel reads through pointers
-// (its form for grids of 2 GB and more) whatever the grid size
+// flat = 1: the split-BF16 source-stationary kernel and the full-precision
+// kernel read through pointers (their form for grids of 2 GB and more, and
+// for grids whose planes leave 32-bit offsets) whatever the grid size
 void grid_m2l_set_flat(GridM2L *g, int flat);
 // records `mid` (if not null) between the scatter into the grids and the M2L kernel
 // deep_in_grid: the deepest level's multipoles are already in the grids

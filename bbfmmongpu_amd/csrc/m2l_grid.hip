@@ -18,10 +18,11 @@
 // vectors widen every product.  One launch covers all levels.
 //
 // Forms:
-//   PLAIN   real-precision FMAs on the vector ALUs (drop-in parity);
+//   PLAIN   the build's precision on the matrix unit (fp32 or fp64 operands
+//           and sums), any rank 1..512;
 //   BF16X2  K and M split into bf16 hi + lo, three MFMA products
 //           (hi*hi + hi*lo + lo*hi) accumulated in fp32 (fp32 build);
-//   FP32    v_mfma_f32_32x32x2_f32 (fp32 build);
+//   FP32    the same kernel on the vectors of the particle-row form (fp32 build);
 //   FP16X3  K and M each split into three fp16 terms t1 + t2 + t3 (about 33
 //           bits), six MFMA products (t1t1, t1t2, t2t1, t1t3, t2t2, t3t1)
 //           accumulated in fp32 (fp32 build).  fp16 has a narrow exponent
@@ -30,9 +31,8 @@
 //           largest entry (measured on the device each solve); all sources
 //           of a field cell lie on its level, so the product is unscaled
 //           exactly in the epilogue.
-// MFMA forms use r = 32 (one 32 x 32 output tile per 32 columns); FP32 also
-// r = 256.  PLAIN takes any rank 1..512 (r = 32 and 256 with the rank fixed
-// at compile time).
+// The split forms use r = 32 (one 32 x 32 output tile per 32 columns), FP32
+// r = 32 and 256.
 #include "common.h"
 #include "kernels.h"
 
@@ -78,6 +78,11 @@ struct GridArgs {
   int nsplit;
   int up_cell0, up_ncell;
   float *Lx;
+  // full-precision kernel (k_m2l_real): rank in tiles of 16; a block's row
+  // tiles, column tiles and waves (offset slices); row groups of a column
+  // group; 1: buffer loads
+  int kt, rt, ct, ws, nrg, buf;
+  size_t plane;  // reals of one coefficient plane of the grids
 };
 
 constexpr int kSteps = 208;  // 8 source classes x 26 non-zero parent shifts
@@ -188,10 +193,10 @@ __global__ void __launch_bounds__(256) k_level_absmax(GridArgs g, const real *__
 // ---------------------------------------------------------------- scatter
 // M [rhs][ncell][r] -> per-class grids [slot][rhs][r]; one thread per
 // (cell, rhs, 8 consecutive coefficients).
-template <int FORM, int CW = 8>
+template <int FORM>
 __global__ void k_grid_scatter(GridArgs g, const real *__restrict__ M)
 {
-  static_assert(CW == 8 || FORM == BBFMM_M2L_PLAIN, "the MFMA grids take 8 coefficients per thread");
+  constexpr int CW = 8;
   const int chunks = g.r / CW;
   const long long total = (long long)(g.levsta[g.maxlev + 1] - g.levsta[g.minlev]) * g.nrhs * chunks;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -219,7 +224,7 @@ __global__ void k_grid_scatter(GridArgs g, const real *__restrict__ M)
     }
     *reinterpret_cast<bf16x8 *>((__bf16 *)g.Mg0 + dst) = hi;
     *reinterpret_cast<bf16x8 *>((__bf16 *)g.Mg1 + dst) = lo;
-  } else if (FORM == BBFMM_M2L_FP16X3) {
+  } else {  // FP16X3
     const float sc = ldexpf(1.0f, fp16_scale_exp(g.lvl_max[l]));
     f16x8 t1, t2, t3;
 #pragma unroll
@@ -233,10 +238,6 @@ __global__ void k_grid_scatter(GridArgs g, const real *__restrict__ M)
     *reinterpret_cast<f16x8 *>((_Float16 *)g.Mg0 + dst) = t1;
     *reinterpret_cast<f16x8 *>((_Float16 *)g.Mg1 + dst) = t2;
     *reinterpret_cast<f16x8 *>((_Float16 *)g.Mg2 + dst) = t3;
-  } else {
-    real *d = (real *)g.Mg0 + dst;
-#pragma unroll
-    for (int e = 0; e < CW; e++) d[e] = src[e];
   }
 }
 
@@ -357,29 +358,6 @@ __global__ void __launch_bounds__(256) k_m2l_mfma(GridArgs g)
           acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks][1], b[ks][1], acc[t], 0, 0, 0);
           acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[ks][2], b[ks][0], acc[t], 0, 0, 0);
         }
-      }
-    } else {
-      // FP32: lane holds k = 16*half + ks for ks = 0..15; A: [k][lane][16]
-      const f32x4 *Ka = (const f32x4 *)g.Ka + ((size_t)k * 64 + lane) * 4;
-      f32x4 a[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) a[q] = Ka[q];
-      const float *Mf = (const float *)g.Mg0;
-#pragma unroll
-      for (int t = 0; t < TPW; t++) {
-        const size_t o = ((size_t)(off + base[t]) * g.nrhs + rhs[t]) * 32 + half * 16;
-        const f32x4 *bp = (const f32x4 *)(Mf + o);
-        f32x4 b[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          b[q] = bp[q];
-          if (!valid[t]) b[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-#pragma unroll
-          for (int w = 0; w < 4; w++)
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q][w], b[q][w], acc[t], 0, 0, 0);
       }
     }
   }
@@ -899,312 +877,292 @@ __global__ void __launch_bounds__(256) k_m2l_add_parts(GridArgs g)
   *Lp = v;
 }
 
-// ---------------------------------------------------------------- r = 256 FP32 MFMA kernel
-// 256 threads = 4 waves, all of one class s at one level; each wave owns 32
-// columns and all 256 rows (8 row tiles of v_mfma_f32_32x32x2f32).  For each
-// of the class's 189 offsets v, K_v streams through LDS in 8 chunks of 32
-// k-values (32 KB, layout [row tile][lane][16]: lane l holds row l%32 of the
-// tile and k = 16*(l/32) + 0..15 of the chunk), double-buffered and loaded
-// by LDS-DMA one chunk ahead; the lane's B values are the 16 consecutive
-// coefficients k = 16*(l/32) + 0..15 of its source column.
-constexpr int kR256Chunks = 8;  // 256 / 32
-
-__global__ void __launch_bounds__(256) k_m2l_fp32_r256(GridArgs g)
+// ---------------------------------------------------------------- full-precision kernel
+// L_s[:, p] += K_v M_{s'}[:, p + d] in the build's own precision on
+// v_mfma_f32_16x16x4_f32 / v_mfma_f64_16x16x4_f64 (fp32 / fp64 operands and
+// sums), any rank 1..512, padded with zeros to kt tiles of 16.
+//
+// Operators: [k][row tile][k chunk of 16][lane] (k_real_layout): lane l
+// holds row 16 tile + real_row(l % 16) and columns 16 chunk + 4 (l / 16) ..
+// + 3, the operands of four products, in 16-byte pieces; the B fragment is
+// the same four coefficients of the lane's source column.
+//
+// A block is one class, RT tiles of rows and CT tiles of 16 columns (parents
+// x vectors) of one level; its waves take the offsets in ws slices, whose
+// sums are added through LDS in slice order.  Offsets
+// whose shifted tile lies outside the level in some axis for all CT tiles
+// read only ghost zeros: wave 0 lists the others once (with 16 vectors a
+// tile is one parent and no ghost is multiplied).  The fragments of the next
+// k chunk are loaded while the current one is multiplied.
+// Class s takes the blocks b % 8 = s, which run on one XCD: its L2 then holds
+// that class's operators only.
+//
+// Bound by the matrix unit at many columns (the fragments' loads come from L2
+// at 8 to 24 bytes a clock and CU), by the operators' bytes beyond L2 at high
+// rank and few columns, by latency at the smallest sizes.  M2L alone, scatter
+// included, against the kernels before it (fp32 or fp64 FMAs, a thread a row
+// or a lane a column; 32-column MFMA tiles without offset slices):
+//   n = 4, one vector: N = 65536 315 -> 32 us, 1M 553 -> 131 us (93 TFLOP/s
+//   of list products), fp64 100003 380 -> 54 us, 1M 1023 -> 242 us;
+//   n = 4, 16 vectors, 1M, fp32: 2640 -> 1600 us; n = 6, 80000, one vector:
+//   10120 -> 204 us (fp64 14250 -> 400); n = 8, 131072: one vector
+//   24.5 -> 0.96 ms, 16 vectors 19.25 -> 9.95 ms (135 TFLOP/s).
+#ifdef SINGLE
+typedef float realx4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ realx4 mfma_real(real a, real b, realx4 c)
 {
-  __shared__ f32x4 sK[2][8][64][4];  // [buffer][row tile][lane][16 floats]
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  // XCD-aware order: each XCD takes a contiguous run of (column group, class)
-  const int nb = g.blk0[g.maxlev + 1];
-  const int lb = (blockIdx.x & 7) * ((nb + 7) >> 3) + (blockIdx.x >> 3);
-  if (lb >= nb) return;
-  int l, s, grp;
-  decode_block(g, lb, l, s, grp);
-  const int P = 1 << (l - 1);
-  const int PP = P + 2;
-  const int ncols = P * P * P * g.nrhs;
-  const int half = lane >> 5;
-  // columns past the end compute a copy of column 0 and are not stored
-  const int col = (grp * 4 + wave) * 32 + (lane & 31);
-  const bool valid = col < ncols;
-  const int cc = valid ? col : 0;
-  const int pl = cc / g.nrhs;
-  const int rh = cc - pl * g.nrhs;
-  const int pz = pl % P, py = (pl / P) % P, px = pl / (P * P);
-  const int base = ((px + 1) * PP + py + 1) * PP + pz + 1;
-  const int slot0 = g.lvl_slot0[l];
-  const int cls = PP * PP * PP;
-  const float *Mf = (const float *)g.Mg0;
-  const int4 *tab = g.tab + s * kOffsets;
-  // chunk (v, kc) of the operator stream: 32 KB at Ka + (k * 8 + kc) * 32 KB
-  const f32x4 *Kq = (const f32x4 *)g.Ka;
-  typedef __attribute__((address_space(3))) void lds_void;
-  auto load_chunk = [&](int k, int kc, int buf) {
-    const f32x4 *src = Kq + ((size_t)k * kR256Chunks + kc) * 2048 + threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-      __builtin_amdgcn_global_load_lds((const void *)(src + i * 256),
-                                       (lds_void *)((f32x4 *)&sK[buf][0][0][0] + i * 256 + wave * 64), 16, 0, 0);
-  };
-  auto src_col = [&](int4 e) {
-    const int dx = ((e.z >> 4) & 3) - 1, dy = ((e.z >> 2) & 3) - 1, dz = (e.z & 3) - 1;
-    const int off = slot0 + e.y * cls + (dx * PP + dy) * PP + dz;
-    return ((size_t)(off + base) * g.nrhs + rh) * 256 + half * 16;
-  };
-  auto load_b = [&](size_t o, int kc, f32x4 *bq) {
-    const f32x4 *bp = (const f32x4 *)(Mf + o + kc * 32);
-#pragma unroll
-    for (int q = 0; q < 4; q++) bq[q] = bp[q];
-  };
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// row of the tile that A's lane i holds (accumulator v of lane group h is row 4 h + v)
+__host__ __device__ __forceinline__ int real_row(int i) { return i; }
+#else
+typedef double realx4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ realx4 mfma_real(real a, real b, realx4 c)
+{
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+// the fp64 product leaves its row 4 v + h in accumulator v of lane group h:
+// A's rows are permuted so that it too is row 4 h + v of the tile
+__host__ __device__ __forceinline__ int real_row(int i) { return 4 * (i & 3) + (i >> 2); }
+#endif
+typedef real realx __attribute__((ext_vector_type(16 / sizeof(real))));  // a 16-byte piece
+// L of any caller is stored four values at a time whatever its alignment
+typedef real realx4u __attribute__((ext_vector_type(4), aligned(sizeof(real))));
 
-  f32x16 acc[8];
-#pragma unroll
-  for (int t = 0; t < 8; t++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[t][e] = 0.0f;
+constexpr int kVW = 16 / (int)sizeof(real);  // coefficients of a 16-byte piece
+constexpr int kPW = 4 / kVW;                  // pieces of the four coefficients of a fragment
 
-  int4 e = tab[0];
-  size_t o = src_col(e);
-  f32x4 bq[4];
-  load_chunk(e.x, 0, 0);
-  load_b(o, 0, bq);
-  __builtin_amdgcn_s_waitcnt(kWaitVm0);
-  __syncthreads();
-  const int nsteps = kOffsets * kR256Chunks;
-  for (int st = 0; st < nsteps; st++) {
-    const int b = st & 1;
-    const int kc = st & (kR256Chunks - 1);
-    // next chunk: same offset, next k-chunk, or the next offset
-    const int sn = st + 1 < nsteps ? st + 1 : st;
-    const int kcn = sn & (kR256Chunks - 1);
-    const int4 en = tab[sn / kR256Chunks];
-    const size_t on = kcn == 0 ? src_col(en) : o;
-    // row tiles 0-3, then the fragments of tiles 4-7, then the loads of the
-    // next chunk (LDS reads must precede the DMA into the other buffer)
-    f32x4 a[4][4];
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) a[t][q] = sK[b][t][lane][q];
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int w = 0; w < 4; w++)
-          acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t][q][w], bq[q][w], acc[t], 0, 0, 0);
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) a[t][q] = sK[b][4 + t][lane][q];
-    __builtin_amdgcn_sched_barrier(0);
-    f32x4 bn[4];
-    load_chunk(en.x, kcn, b ^ 1);
-    load_b(on, kcn, bn);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int w = 0; w < 4; w++)
-          acc[4 + t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t][q][w], bq[q][w], acc[4 + t], 0, 0, 0);
-#pragma unroll
-    for (int q = 0; q < 4; q++) bq[q] = bn[q];
-    o = on;
-    (void)kc;
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    __syncthreads();
-  }
-  if (!valid) return;
-  const int fx = 2 * px + ((s >> 2) & 1), fy = 2 * py + ((s >> 1) & 1), fz = 2 * pz + (s & 1);
-  const int A = g.levsta[l] + morton3(fx, fy, fz, l);
-  float *Lp = (float *)g.L + ((size_t)rh * g.ncell + A) * 256 + 4 * half;
-#pragma unroll
-  for (int t = 0; t < 8; t++)
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      f32x4 v = {acc[t][4 * q], acc[t][4 * q + 1], acc[t][4 * q + 2], acc[t][4 * q + 3]};
-      *reinterpret_cast<f32x4 *>(Lp + 32 * t + 8 * q) = v;
-    }
+// out [k][tile][chunk][piece][lane][kVW] from the column-major operators (K_k(i, j) at k r^2 + j r + i)
+__global__ void __launch_bounds__(256) k_real_layout(int r, int kt, const real *__restrict__ K, real *__restrict__ out)
+{
+  const long long n = (long long)kNumOps * kt * kt * 256;
+  const long long o = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (o >= n) return;
+  const int e = (int)(o % kVW), lane = (int)(o / kVW % 64), h = (int)(o / (64 * kVW) % kPW);
+  const long long tc = o >> 8;
+  const int c = (int)(tc % kt), t = (int)((tc / kt) % kt), k = (int)(tc / kt / kt);
+  const int row = 16 * t + real_row(lane & 15), col = 16 * c + 4 * (lane >> 4) + kVW * h + e;
+  out[o] = row < r && col < r ? K[((size_t)k * r + col) * r + row] : (real)0;
 }
 
-// ---------------------------------------------------------------- plain kernel
-// One thread per (column, row); 256 / R columns per block, all of one class.
-template <int R>
-__global__ void __launch_bounds__(256) k_m2l_grid_plain(GridArgs g)
+// M [rhs][ncell][r] -> grids [plane][slot][rhs][kVW], plane p holding the
+// coefficients kVW p .. kVW p + kVW - 1 (zeros from r on): the 16 columns of
+// a fragment are then one 256-byte piece of a plane wherever the shift puts
+// them (as [slot][rhs][r] every lane's 16 bytes were a separate access of
+// the cache: the M2L of 131072 particles, n = 8, 16 vectors took 18.5 ms)
+__global__ void __launch_bounds__(256) k_real_scatter(GridArgs g, const real *__restrict__ M)
 {
-  constexpr int CPB = 256 / R;
-  const int lb = xcd_block(g, blockIdx.x);
-  if (lb < 0) return;
-  int l, s, grp;
-  decode_block(g, lb, l, s, grp);
-  const int P = 1 << (l - 1);
-  const int PP = P + 2;
-  const int ncols = P * P * P * g.nrhs;
-  const int i = threadIdx.x % R;
-  const int col = grp * CPB + threadIdx.x / R;
-  if (col >= ncols) return;  // no barrier in this kernel
-  const int pl = col / g.nrhs, rh = col - (col / g.nrhs) * g.nrhs;
-  const int pz = pl % P, py = (pl / P) % P, px = pl / (P * P);
-  const int base = ((px + 1) * PP + py + 1) * PP + pz + 1;
-  const int4 *tab = g.tab + s * kOffsets;
-  const real4 *K4 = (const real4 *)g.Ka;
-  const real *Mg = (const real *)g.Mg0;
-  const int slot0 = g.lvl_slot0[l];
-  real acc0 = 0, acc1 = 0;
-  for (int v = 0; v < kOffsets; v++) {
-    const int4 e = tab[v];
-    const int dx = ((e.z >> 4) & 3) - 1, dy = ((e.z >> 2) & 3) - 1, dz = (e.z & 3) - 1;
-    const size_t slot = (size_t)slot0 + e.y * PP * PP * PP + (dx * PP + dy) * PP + dz + base;
-    const real4 *Mp = (const real4 *)(Mg + (slot * g.nrhs + rh) * R);
-    const real4 *Kp = K4 + (size_t)e.x * (R / 4) * R + i;
-#pragma unroll 8
-    for (int jb = 0; jb < R / 4; jb += 2) {
-      const real4 ka = Kp[(size_t)jb * R], kb = Kp[(size_t)(jb + 1) * R];
-      const real4 ma = Mp[jb], mb = Mp[jb + 1];
-      acc0 += ka.x * ma.x;
-      acc1 += kb.x * mb.x;
-      acc0 += ka.y * ma.y;
-      acc1 += kb.y * mb.y;
-      acc0 += ka.z * ma.z;
-      acc1 += kb.z * mb.z;
-      acc0 += ka.w * ma.w;
-      acc1 += kb.w * mb.w;
-    }
-  }
-  const int fx = 2 * px + ((s >> 2) & 1), fy = 2 * py + ((s >> 1) & 1), fz = 2 * pz + (s & 1);
-  const int A = g.levsta[l] + morton3(fx, fy, fz, l);
-  g.L[((size_t)rh * g.ncell + A) * R + i] = acc0 + acc1;
+  const int np = 16 * g.kt / kVW;
+  const long long total = (long long)(g.levsta[g.maxlev + 1] - g.levsta[g.minlev]) * g.nrhs * np;
+  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (t >= total) return;
+  const int rhs = (int)(t % g.nrhs);
+  const long long cp = t / g.nrhs;
+  const int p = (int)(cp % np);
+  const int A = g.levsta[g.minlev] + (int)(cp / np);
+  int l = g.minlev;
+  while (A >= g.levsta[l + 1]) l++;
+  int x, y, z;
+  demorton3(A - g.levsta[l], l, x, y, z);
+  const size_t slot = grid_slot(g, l, ((x & 1) << 2) | ((y & 1) << 1) | (z & 1), x >> 1, y >> 1, z >> 1);
+  const real *src = M + ((size_t)rhs * g.ncell + A) * g.r + kVW * p;
+  realx v;
+#pragma unroll
+  for (int e = 0; e < kVW; e++) v[e] = kVW * p + e < g.r ? src[e] : (real)0;
+  *reinterpret_cast<realx *>((real *)g.Mg0 + p * g.plane + (slot * g.nrhs + rhs) * kVW) = v;
 }
 
-// r = 32, real precision: a block is 64 columns (lanes) of one class at one
-// level and wave w computes rows 8w..8w+7 of all of them.  K_v (column-major,
-// the reference's layout) is the same for every lane of a wave, so its
-// entries arrive by scalar loads into SGPRs: each FMA reads one SGPR (K) and
-// one VGPR (a coefficient of the lane's source column), no LDS or vector
-// load is spent on K, and the only vector loads are the lane's 32-coefficient
-// source column per offset, issued one offset ahead.
-__global__ void __launch_bounds__(256) k_m2l_grid_plain32(GridArgs g)
+// BUF: fragments by buffer loads (the uniform part of an address in the
+// resource, a 32-bit lane offset; planes of a k chunk within 4 GB), else by
+// 64-bit lane addresses, which cost the address path about twice as much
+// (131072 particles, n = 8, 16 vectors, CT = RT = 4: 13.2 against 15.7 ms).
+template <int RT, int CT, int KC, int MAXW, bool BUF>
+__global__ void __launch_bounds__(64 * MAXW) k_m2l_real(GridArgs g)
 {
-  const int lb = xcd_block(g, blockIdx.x);
-  if (lb < 0) return;
-  int l, s, grp;
-  decode_block(g, lb, l, s, grp);
+  extern __shared__ __align__(32) unsigned char smem_raw[];
+  realx4 *red = reinterpret_cast<realx4 *>(smem_raw);  // [slice][tile][64]
+  __shared__ int2 lst[192];  // offsets to multiply: operator | tiles << 16, slot shift
+  __shared__ int nlst;
+  const int lane = threadIdx.x & 63;
+  const int ws = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);  // offset slice
+  const int s = blockIdx.x & 7, gr = blockIdx.x >> 3;
+  const int gb = gr / g.nrg;               // column group
+  const int rt0 = (gr - gb * g.nrg) * RT;  // first row tile
+  int l = g.minlev;
+  while (l < g.maxlev && gb >= g.blk0[l + 1]) l++;
   const int P = 1 << (l - 1);
   const int PP = P + 2;
   const int ncols = P * P * P * g.nrhs;
-  const int lane = threadIdx.x & 63;
-  const int rg = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);  // row group
-  const int col = grp * 64 + lane;
-  const bool valid = col < ncols;
-  const int cc = valid ? col : 0;  // columns past the end compute column 0 and are not stored
-  const int pl = cc / g.nrhs, rh = cc - (cc / g.nrhs) * g.nrhs;
-  const int pz = pl % P, py = (pl / P) % P, px = pl / (P * P);
-  const int base = ((px + 1) * PP + py + 1) * PP + pz + 1;
-  const int4 *__restrict__ tab = g.tab + s * kOffsets;
-  const real *__restrict__ Kc = (const real *)g.Ka + rg * 8;
-  const real *__restrict__ Mg = (const real *)g.Mg0;
-  const size_t slot0 = (size_t)g.lvl_slot0[l] + base;
-  const int cls = PP * PP * PP;
-  auto src = [&](int v) {
-    const int4 e = tab[v];
-    const int dx = ((e.z >> 4) & 3) - 1, dy = ((e.z >> 2) & 3) - 1, dz = (e.z & 3) - 1;
-    const size_t slot = slot0 + e.y * cls + (dx * PP + dy) * PP + dz;
-    return reinterpret_cast<const real4 *>(Mg + (slot * g.nrhs + rh) * 32);
+  const int col0 = (gb - g.blk0[l]) * (16 * CT);
+  if (ws == 0) {
+    WaveBox box[CT];
+#pragma unroll
+    for (int t = 0; t < CT; t++) box[t] = wave_box(col0 + 16 * t, ncols, g.nrhs, P, 16);
+    int n = 0;
+    for (int q = 0; q < 3; q++) {
+      const int v = 64 * q + lane;
+      const int4 e = g.tab[s * kOffsets + min(v, kOffsets - 1)];
+      int m = 0;
+#pragma unroll
+      for (int t = 0; t < CT; t++) m |= ghost_step(box[t], e.z << 3, P) ? 0 : 1 << t;
+      if (v >= kOffsets) m = 0;
+      const unsigned long long act = __ballot(m != 0);
+      const int dx = ((e.z >> 4) & 3) - 1, dy = ((e.z >> 2) & 3) - 1, dz = (e.z & 3) - 1;
+      if (m)
+        lst[n + __popcll(act & ((1ull << lane) - 1))] =
+            make_int2(e.x | (m << 16), e.y * PP * PP * PP + ((dx + 1) * PP + dy + 1) * PP + dz + 1);
+      n += __popcll(act);
+    }
+    if (lane == 0) nlst = n;
+  }
+  const int kt = g.kt;
+  const int nrt = min(RT, kt - rt0);  // row tiles
+  // sources and operators: a uniform address plus a lane offset
+  size_t bo[CT];
+#pragma unroll
+  for (int t = 0; t < CT; t++) {
+    const int col = min(col0 + 16 * t + (lane & 15), ncols - 1);  // columns past the end are not stored
+    const int pl = col / g.nrhs, rh = col - pl * g.nrhs;
+    const int pz = pl % P, py = (pl / P) % P, px = pl / (P * P);
+    const int slot = (px * PP + py) * PP + pz;  // shifts add PP (PP + 1) + 1 at most, 0 at least
+    bo[t] = ((size_t)(lane >> 4) * kPW * g.plane + ((size_t)slot * g.nrhs + rh) * kVW) * sizeof(real);
+  }
+  const char *bbase = (const char *)((const real *)g.Mg0 + (size_t)g.lvl_slot0[l] * g.nrhs * kVW);
+  const size_t plane = g.plane * sizeof(real);
+  const int ktile = kt * 256 * (int)sizeof(real);
+  const char *abase = (const char *)g.Ka + (size_t)rt0 * ktile;
+  struct Frag {
+    realx a[RT][KC][kPW], b[CT][KC][kPW];
   };
-  real acc[8];
+  auto load = [&](Frag &f, int2 w, int c) {
+    const char *a = abase + (size_t)(w.x & 0xffff) * kt * ktile + (size_t)c * (256 * sizeof(real));
+    const char *b = bbase + (size_t)w.y * (g.nrhs * 16) + (size_t)c * (16 / kVW) * plane;
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)a, 0, -1, 0x00020000);
 #pragma unroll
-  for (int i = 0; i < 8; i++) acc[i] = 0;
-  auto load = [&](int v, real4 *m) {
-    const real4 *p = src(v);
+    for (int q = 0; q < KC; q++) {
+      const char *bq = b + (size_t)q * (16 / kVW) * plane;
+      const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)bq, 0, -1, 0x00020000);
 #pragma unroll
-    for (int q = 0; q < 8; q++) m[q] = p[q];
-  };
-  auto mac = [&](int v, const real4 *m) {
-    const real *__restrict__ Kk = Kc + (size_t)tab[v].x * 1024;
+      for (int h = 0; h < kPW; h++) {
 #pragma unroll
-    for (int jq = 0; jq < 8; jq++) {
-      const real mj[4] = {m[jq].x, m[jq].y, m[jq].z, m[jq].w};
+        for (int i = 0; i < RT; i++) {
+          const int at = min(i, nrt - 1) * ktile, al = q * (256 * (int)sizeof(real)) + h * 1024 + lane * 16;
+          if (BUF)
+            f.a[i][q][h] = __builtin_bit_cast(realx, __builtin_amdgcn_raw_buffer_load_b128(ra, al, at, 0));
+          else
+            f.a[i][q][h] = *reinterpret_cast<const realx *>(a + at + al);
+        }
 #pragma unroll
-      for (int t = 0; t < 4; t++) {
-        const real *__restrict__ kc = Kk + (4 * jq + t) * 32;  // column j: rows 8 rg .. 8 rg + 7
-#pragma unroll
-        for (int i = 0; i < 8; i++) acc[i] += kc[i] * mj[t];
+        for (int t = 0; t < CT; t++)
+          if (BUF)
+            f.b[t][q][h] =
+                __builtin_bit_cast(realx, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)bo[t], (int)(h * plane), 0));
+          else
+            f.b[t][q][h] = *reinterpret_cast<const realx *>(bq + h * plane + bo[t]);
       }
     }
   };
-  // two register sets in turn: the next offset's column is in flight while
-  // the current one is multiplied (no copy between the sets, so no wait for
-  // the loads at the end of an iteration)
-  real4 ma[8], mb[8];
-  load(0, ma);
-  static_assert(kOffsets % 2 == 1, "the loop below ends on an odd offset count");
-  for (int v = 0; v + 1 < kOffsets; v += 2) {
-    load(v + 1, mb);
-    __builtin_amdgcn_sched_barrier(0);  // loads issued before the products
-    mac(v, ma);
-    load(v + 2, ma);
+  realx4 acc[RT][CT];
+#pragma unroll
+  for (int i = 0; i < RT; i++)
+#pragma unroll
+    for (int t = 0; t < CT; t++) acc[i][t] = realx4{0, 0, 0, 0};
+  // the fragments of the current iteration have arrived once only the next
+  // one's loads are outstanding (waited for here, whatever products follow)
+  constexpr int kLoads = (RT + CT) * KC * kPW;
+  static_assert(kLoads < 64, "vmcnt immediate");
+  auto mac = [&](const Frag &f, int2 w) {
     __builtin_amdgcn_sched_barrier(0);
-    mac(v + 1, mb);
-  }
-  mac(kOffsets - 1, ma);
-  if (!valid) return;
-  const int fx = 2 * px + ((s >> 2) & 1), fy = 2 * py + ((s >> 1) & 1), fz = 2 * pz + (s & 1);
-  const int A = g.levsta[l] + morton3(fx, fy, fz, l);
-  real *Lp = g.L + ((size_t)rh * g.ncell + A) * 32 + rg * 8;
+    __builtin_amdgcn_s_waitcnt(kWaitVm0 | (kLoads & 15) | ((kLoads >> 4) << 14));
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int i = 0; i < 8; i++) Lp[i] = acc[i];
-}
-
-// Any rank (r other than 32 and 256): as k_m2l_grid_plain with K in the
-// reference's column-major layout (K_k(i, j) at k r^2 + j r + i) and scalar
-// loads; 256 / r columns per block (r <= 256) or one column with
-// ceil(r / 256) rows per thread.
-__global__ void __launch_bounds__(256) k_m2l_grid_plain_any(GridArgs g)
-{
-  constexpr int RPT = (kMaxRank + 255) / 256;
-  const int r = g.r;
-  const int rt = r < 256 ? r : 256, cpb = 256 / rt;
-  const int lb = xcd_block(g, blockIdx.x);
-  if (lb < 0) return;
-  int l, s, grp;
-  decode_block(g, lb, l, s, grp);
-  const int P = 1 << (l - 1);
-  const int PP = P + 2;
-  const int ncols = P * P * P * g.nrhs;
-  const int cl = (int)threadIdx.x / rt, i0 = (int)threadIdx.x - cl * rt;
-  const int col = grp * cpb + cl;
-  if (cl >= cpb || col >= ncols) return;  // no barrier in this kernel
-  const int pl = col / g.nrhs, rh = col - (col / g.nrhs) * g.nrhs;
-  const int pz = pl % P, py = (pl / P) % P, px = pl / (P * P);
-  const int base = ((px + 1) * PP + py + 1) * PP + pz + 1;
-  const int4 *tab = g.tab + s * kOffsets;
-  const real *Kc = (const real *)g.Ka;
-  const real *Mg = (const real *)g.Mg0;
-  const int slot0 = g.lvl_slot0[l];
-  real acc[RPT];
+    for (int t = 0; t < CT; t++) {
+      if (CT > 1 && !((w.x >> (16 + t)) & 1)) continue;
 #pragma unroll
-  for (int u = 0; u < RPT; u++) acc[u] = 0;
-  for (int v = 0; v < kOffsets; v++) {
-    const int4 e = tab[v];
-    const int dx = ((e.z >> 4) & 3) - 1, dy = ((e.z >> 2) & 3) - 1, dz = (e.z & 3) - 1;
-    const size_t slot = (size_t)slot0 + e.y * PP * PP * PP + (dx * PP + dy) * PP + dz + base;
-    const real *Mp = Mg + (slot * g.nrhs + rh) * r;
-    const real *Kk = Kc + (size_t)e.x * r * r + i0;
-    for (int j = 0; j < r; j++) {
-      const real m = Mp[j];
+      for (int i = 0; i < RT; i++) {
+        if (RT > 1 && i >= nrt) break;
 #pragma unroll
-      for (int u = 0; u < RPT; u++)
-        if (i0 + u * rt < r) acc[u] += Kk[(size_t)j * r + u * rt] * m;
+        for (int q = 0; q < KC; q++)
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            acc[i][t] = mfma_real(f.a[i][q][e / kVW][e % kVW], f.b[t][q][e / kVW][e % kVW], acc[i][t]);
+      }
+    }
+  };
+  __syncthreads();
+  const int n = __builtin_amdgcn_readfirstlane(nlst);
+  if (ws < n) {
+    // iterations (offset, k chunk); the next one's fragments are in flight
+    // while the current one's are multiplied (past the last offset of the
+    // slice, that offset's again)
+    const int jlast = ws + (n - 1 - ws) / g.ws * g.ws;
+    int j = ws, c = 0;
+    auto entry = [&](int i) {
+      const int2 e = lst[i];
+      return make_int2(__builtin_amdgcn_readfirstlane(e.x), __builtin_amdgcn_readfirstlane(e.y));
+    };
+    int2 w = entry(j);
+    int2 wn = w;
+    Frag f0, f1;
+    load(f0, w, c);
+    auto advance = [&]() {
+      c += KC;
+      if (c >= kt) {
+        c = 0;
+        j = min(j + g.ws, jlast);
+      }
+      wn = entry(j);
+    };
+    const int nit = (jlast - ws) / g.ws * (kt / KC) + kt / KC;
+    for (int it = nit >> 1; it > 0; it--) {
+      advance();
+      load(f1, wn, c);
+      mac(f0, w);
+      w = wn;
+      advance();
+      load(f0, wn, c);
+      mac(f1, w);
+      w = wn;
+    }
+    if (nit & 1) {
+      load(f1, wn, c);  // (the count of outstanding loads that mac waits for)
+      mac(f0, w);
     }
   }
-  const int fx = 2 * px + ((s >> 2) & 1), fy = 2 * py + ((s >> 1) & 1), fz = 2 * pz + (s & 1);
-  const int A = g.levsta[l] + morton3(fx, fy, fz, l);
+  auto store = [&](int rt, int t, realx4 v) {
+    const int col = col0 + 16 * t + (lane & 15);
+    const int row = 16 * rt + 4 * (lane >> 4);
+    if (col >= ncols || row >= g.r) return;
+    const int pl = col / g.nrhs, rh = col - pl * g.nrhs;
+    const int pz = pl % P, py = (pl / P) % P, px = pl / (P * P);
+    const int fx = 2 * px + ((s >> 2) & 1), fy = 2 * py + ((s >> 1) & 1), fz = 2 * pz + (s & 1);
+    const int A = g.levsta[l] + morton3(fx, fy, fz, l);
+    real *Lp = g.L + ((size_t)rh * g.ncell + A) * g.r + row;
+    if (row + 4 <= g.r) {
+      *reinterpret_cast<realx4u *>(Lp) = v;
+    } else {
 #pragma unroll
-  for (int u = 0; u < RPT; u++)
-    if (i0 + u * rt < r) g.L[((size_t)rh * g.ncell + A) * r + i0 + u * rt] = acc[u];
+      for (int e = 0; e < 3; e++)
+        if (row + e < g.r) Lp[e] = v[e];
+    }
+  };
+  if (g.ws == 1) {
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+      for (int t = 0; t < CT; t++) store(rt0 + i, t, acc[i][t]);  // rows past r are not stored
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < RT; i++)
+#pragma unroll
+    for (int t = 0; t < CT; t++) red[(ws * RT * CT + i * CT + t) * 64 + lane] = acc[i][t];
+  __syncthreads();
+  for (int f = ws; f < RT * CT; f += g.ws) {
+    realx4 v = red[f * 64 + lane];
+    for (int q = 1; q < g.ws; q++) v += red[(q * RT * CT + f) * 64 + lane];
+    store(rt0 + f / CT, f % CT, v);
+  }
 }
 
 // ---------------------------------------------------------------- host side
@@ -1286,8 +1244,61 @@ static int ss_classes(int variant)
 
 static int ss_tiles(int variant) { return variant == 6 || variant == 7 || variant == 8 ? 2 : 1; }
 
+// waves of a block of the full-precision kernel at most (their registers)
+constexpr int real_max_waves(int rt, int ct) { return rt * ct <= 4 ? 16 : 8; }
+// Tiles and slices of a block of the full-precision kernel, from the number
+// of 16 x 16 tiles of L.  Larger blocks load fewer fragments per product,
+// smaller ones fill the chip and even out its last round; beyond r = 32 the
+// operators no longer fit L2, so the columns widen first.  Where the lines
+// lie (us, fp32 unless said; columns x rank tiles):
+//   r = 32:  37 x 2 tiles a class (1 vector, depth 4): 1 x 2 32, 1 x 1 33,
+//            2 x 2 36; 73 x 2 (16 vectors, depth 3): 2 x 2 34, 1 x 2 35;
+//            585 x 2: 2 x 2 203, 2 x 4 209; 4681 x 2: 2 x 4 1599, 2 x 2 1639;
+//            fp64 37 x 2: 1 x 2 54, 2 x 1 60; 293 x 2: 2 x 1 242, 2 x 2 > 280
+//   r = 108: 37 x 7: 1 x 4 204, 2 x 2 235, 2 x 4 260; 147 x 7: 2 x 4 664,
+//            4 x 4 695; r = 256, 584 x 16: 4 x 4 9948, 2 x 4 11973;
+//            fp64 147 x 7: 4 x 2 1291, 2 x 2 1657
+// Slices: 8 (64K one vector 32 us, 2 slices 61), 4 once the blocks alone give
+// several rounds (1M, 4 vectors: 4 slices 426, 8 442), 16 at the smallest.
+static void real_shape(GridM2L *g)
+{
+  GridArgs &a = g->args;
+  // the planes of a k chunk within the 32-bit offsets of the buffer loads
+  a.buf = !g->flat && a.plane * sizeof(real) * (16 / kVW) < ((size_t)1 << 32);
+  long long t16 = 0;  // tiles of 16 columns of one class
+  for (int l = a.minlev; l <= a.maxlev; l++) t16 += ((1LL << (3 * (l - 1))) * a.nrhs + 15) / 16;
+  const long long u = 8 * t16 * a.kt;
+  auto take = [&](int rt, int ct) {
+    a.rt = rt;
+    a.ct = ct;
+  };
+  constexpr bool f64 = sizeof(real) == 8;
+  if (!a.buf) take(1, 1);
+  else if (g->variant == 2) take(2, 2);  // 32 columns of r = 32
+  else if (g->variant == 3) take(2, 4);  // 64
+  else if (a.kt <= 2) {
+    if (f64 && a.kt == 2 && u >= 2 * 1024) take(2, 1);
+    else if (!f64 && a.kt == 2 && u >= 8 * 4096) take(2, 4);
+    else if (!f64 && a.kt == 2 && u >= 4 * 256) take(2, 2);
+    else take(1, u >= 2 * 256 ? 2 : 1);
+  } else {
+    if (!f64 && u >= 16 * 2048) take(4, 4);
+    else if (u >= 8 * 512) take(f64 ? 4 : 2, f64 ? 2 : 4);
+    else take(1, u >= 4 * 384 ? 4 : u >= 2 * 256 ? 2 : 1);
+  }
+  a.nrg = (a.kt + a.rt - 1) / a.rt;
+  int groups = 0;
+  for (int l = a.minlev; l <= a.maxlev; l++) {
+    a.blk0[l] = groups;
+    groups += (int)(((1LL << (3 * (l - 1))) * a.nrhs + 16 * a.ct - 1) / (16 * a.ct));
+  }
+  a.blk0[a.maxlev + 1] = groups;
+  g->nblocks = 8 * groups * a.nrg;
+  a.ws = std::min(g->nblocks >= 2048 ? 4 : g->nblocks >= 128 ? 8 : 16, real_max_waves(a.rt, a.ct));
+}
+
 int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const real *K, hipStream_t s,
-                    int minlev, int variant, int variant_upper, int upper_split)
+                    int minlev, int variant, int variant_upper, int upper_split, const real *K_dev)
 {
   *out = nullptr;
   // variant 0 on a deepest level of 64 K columns (parents x vectors) or more,
@@ -1362,6 +1373,11 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
     const size_t gb = slots * (size_t)nrhs * r * 2;  // split-BF16 grids: 2 bytes per value
     a.gbytes = gb < ((size_t)1 << 31) ? (int)gb : 0;
   }
+  const bool real_form = form == BBFMM_M2L_PLAIN || form == BBFMM_M2L_FP32MFMA;
+  a.kt = (r + 15) / 16;
+  // plane stride an odd multiple of 256 bytes: the planes of a fragment start
+  // on different L2 channels (at a multiple of 4 KB they all share one)
+  a.plane = ((slots * nrhs * kVW * sizeof(real) + 4095) / 4096 * 4096 + 256) / sizeof(real);
   int tpw = 1, cpb;
   // variant 0 (automatic): source-stationary blocking (4 classes per wave)
   // once the deepest level has 8192 columns (parents x vectors) or more (at
@@ -1377,13 +1393,13 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
     a.ss_tpw = ss_tiles(variant);
     a.ss_pair = variant == 8;
   }
-  if (form == BBFMM_M2L_PLAIN) {
-    cpb = r == 32 ? 64 : 256 / (r < 256 ? r : 256);  // k_m2l_grid_plain32: 64 columns per block
+  if (real_form) {
+    cpb = 1 << 30;  // blocks: real_shape
   } else if (a.ss) {
     cpb = 4 * 32 * a.ss_tpw;  // 4 waves x 32 or 64 columns, one class group per block
   } else {
     // two tiles per wave once there are enough columns to fill the chip
-    tpw = variant == 3 ? 2 : variant == 2 ? 1 : (r == 32 && deep >= 8 * 1024 ? 2 : 1);  // r = 256: one tile
+    tpw = variant == 3 ? 2 : variant == 2 ? 1 : (deep >= 8 * 1024 ? 2 : 1);
     cpb = 4 * tpw * 32;
   }
   a.wave_cols = tpw * 32;
@@ -1411,6 +1427,7 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
   }
   a.blk0[maxlev + 1] = nb;
   g->nblocks = nb;
+  if (real_form) real_shape(g);
 
   std::vector<int4> tab;
   offset_table(tab);
@@ -1463,29 +1480,28 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
     fail(e, "copy");
   // operators in the form's layout
   if (rc == BBFMM_OK) {
-    if (form == BBFMM_M2L_PLAIN && r != 256) {
-      // r = 32 and any rank: the caller's column-major operators as they are
-      if ((e = hipMalloc(&g->d_K, sizeof(real) * (size_t)kNumOps * r * r)) != hipSuccess) fail(e, "hipMalloc");
-      else if ((e = hipMemcpyAsync(g->d_K, K, sizeof(real) * (size_t)kNumOps * r * r, hipMemcpyHostToDevice, s)) !=
-               hipSuccess)
-        fail(e, "copy");
-      if (rc == BBFMM_OK && (e = hipStreamSynchronize(s)) != hipSuccess) fail(e, "sync");
-      if (rc == BBFMM_OK && (e = hipMalloc(&g->d_Mg0, sizeof(real) * slots * nrhs * r)) != hipSuccess) fail(e, "hipMalloc");
-      if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_Mg0, 0, sizeof(real) * slots * nrhs * r, s)) != hipSuccess) fail(e, "memset");
-    } else if (form == BBFMM_M2L_PLAIN) {
-      std::vector<real4> K4((size_t)kNumOps * r * r / 4);
-      for (int k = 0; k < kNumOps; k++)
-        for (int jb = 0; jb < r / 4; jb++)
-          for (int i = 0; i < r; i++) {
-            const real *Kk = K + (size_t)k * r * r;
-            K4[((size_t)k * (r / 4) + jb) * r + i] = real4{Kk[(size_t)(4 * jb) * r + i], Kk[(size_t)(4 * jb + 1) * r + i],
-                                                          Kk[(size_t)(4 * jb + 2) * r + i], Kk[(size_t)(4 * jb + 3) * r + i]};
-          }
-      if ((e = hipMalloc(&g->d_K, sizeof(real4) * K4.size())) != hipSuccess) fail(e, "hipMalloc");
-      else if ((e = hipMemcpyAsync(g->d_K, K4.data(), sizeof(real4) * K4.size(), hipMemcpyHostToDevice, s)) != hipSuccess)
-        fail(e, "copy");
-      if (rc == BBFMM_OK && (e = hipMalloc(&g->d_Mg0, sizeof(real) * slots * nrhs * r)) != hipSuccess) fail(e, "hipMalloc");
-      if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_Mg0, 0, sizeof(real) * slots * nrhs * r, s)) != hipSuccess) fail(e, "memset");
+    if (real_form) {
+      // the column-major operators go up as they are (unless the caller has
+      // them on the device) and are laid out there
+      const size_t nk = (size_t)kNumOps * a.kt * a.kt * 256, nc = (size_t)kNumOps * r * r;
+      const size_t ng = sizeof(real) * a.plane * (16 * a.kt / kVW);
+      real *up = nullptr;
+      if ((e = hipMalloc(&g->d_K, sizeof(real) * nk)) != hipSuccess) fail(e, "hipMalloc");
+      if (rc == BBFMM_OK && !K_dev) {
+        if ((e = hipMalloc((void **)&up, sizeof(real) * nc)) != hipSuccess) fail(e, "hipMalloc");
+        else if ((e = hipMemcpyAsync(up, K, sizeof(real) * nc, hipMemcpyHostToDevice, s)) != hipSuccess) fail(e, "copy");
+      }
+      if (rc == BBFMM_OK) {
+        hipLaunchKernelGGL(k_real_layout, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, s, r, a.kt,
+                           K_dev ? K_dev : up, (real *)g->d_K);
+        if ((e = hipGetLastError()) != hipSuccess) fail(e, "operator layout");
+      }
+      if (rc == BBFMM_OK && (e = hipMalloc(&g->d_Mg0, ng)) != hipSuccess) fail(e, "hipMalloc");
+      if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_Mg0, 0, ng, s)) != hipSuccess) fail(e, "memset");
+      if (up) {
+        (void)hipStreamSynchronize(s);
+        (void)hipFree(up);
+      }
     }
 #ifdef SINGLE
     else if (form == BBFMM_M2L_BF16X2) {
@@ -1550,42 +1566,6 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
       }
       if (rc == BBFMM_OK && (e = hipMalloc(&g->d_lvl_max, sizeof(unsigned) * (kMaxLev + 1))) != hipSuccess)
         fail(e, "hipMalloc");
-    } else if (r == 256) {
-      // FP32, r = 256: [k][k-chunk][row tile][lane][16]: lane l holds row
-      // 32*tile + l%32 and columns 32*chunk + 16*(l/32) + 0..15
-      std::vector<float> Kf((size_t)kNumOps * 256 * 256);
-      for (int k = 0; k < kNumOps; k++)
-        for (int kc = 0; kc < 8; kc++)
-          for (int t = 0; t < 8; t++)
-            for (int lane = 0; lane < 64; lane++)
-              for (int ks = 0; ks < 16; ks++) {
-                const int row = 32 * t + (lane & 31), col = 32 * kc + 16 * (lane >> 5) + ks;
-                Kf[((((size_t)k * 8 + kc) * 8 + t) * 64 + lane) * 16 + ks] =
-                    K[(size_t)k * 256 * 256 + (size_t)col * 256 + row];
-              }
-      if ((e = hipMalloc(&g->d_K, sizeof(float) * Kf.size())) != hipSuccess) fail(e, "hipMalloc");
-      else if ((e = hipMemcpyAsync(g->d_K, Kf.data(), sizeof(float) * Kf.size(), hipMemcpyHostToDevice, s)) != hipSuccess)
-        fail(e, "copy");
-      // the host copy must outlive the asynchronous copy
-      if (rc == BBFMM_OK && (e = hipStreamSynchronize(s)) != hipSuccess) fail(e, "sync");
-      const size_t nb2 = sizeof(float) * slots * nrhs * r;
-      if (rc == BBFMM_OK && (e = hipMalloc(&g->d_Mg0, nb2)) != hipSuccess) fail(e, "hipMalloc");
-      if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_Mg0, 0, nb2, s)) != hipSuccess) fail(e, "memset");
-    } else {
-      // FP32: [k][lane][16]: lane l holds row l%32, k = 16*(l/32) + ks
-      std::vector<float> Kf((size_t)kNumOps * 64 * 16);
-      for (int k = 0; k < kNumOps; k++)
-        for (int lane = 0; lane < 64; lane++)
-          for (int ks = 0; ks < 16; ks++) {
-            const int row = lane & 31, col = 16 * (lane >> 5) + ks;
-            Kf[((size_t)k * 64 + lane) * 16 + ks] = K[(size_t)k * 32 * 32 + (size_t)col * 32 + row];
-          }
-      if ((e = hipMalloc(&g->d_K, sizeof(float) * Kf.size())) != hipSuccess) fail(e, "hipMalloc");
-      else if ((e = hipMemcpyAsync(g->d_K, Kf.data(), sizeof(float) * Kf.size(), hipMemcpyHostToDevice, s)) != hipSuccess)
-        fail(e, "copy");
-      const size_t nb2 = sizeof(float) * slots * nrhs * r;
-      if (rc == BBFMM_OK && (e = hipMalloc(&g->d_Mg0, nb2)) != hipSuccess) fail(e, "hipMalloc");
-      if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_Mg0, 0, nb2, s)) != hipSuccess) fail(e, "memset");
     }
 #endif
   }
@@ -1638,7 +1618,9 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
 
 void grid_m2l_set_flat(GridM2L *g, int flat)
 {
-  if (g) g->flat = flat != 0;
+  if (!g || g->flat == (flat != 0)) return;
+  g->flat = flat != 0;
+  if (g->form == BBFMM_M2L_PLAIN || g->form == BBFMM_M2L_FP32MFMA) real_shape(g);
 }
 
 void grid_m2l_destroy(GridM2L *g)
@@ -1653,6 +1635,39 @@ void grid_m2l_destroy(GridM2L *g)
   if (g->d_lvl_max) (void)hipFree(g->d_lvl_max);
   if (g->d_Lx) (void)hipFree(g->d_Lx);
   delete g;
+}
+
+template <int RT, int CT, int KC, bool BUF = true>
+static int launch_real_t(const GridArgs &a, int nblocks, hipStream_t s)
+{
+  constexpr int MAXW = real_max_waves(RT, CT);
+  const int lds = a.ws > 1 ? (int)(a.ws * RT * CT * 64 * sizeof(realx4)) : 0;
+  const auto kernel = k_m2l_real<RT, CT, KC, MAXW, BUF>;
+  hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(64 * a.ws), lds, s, a);
+  BB_HIP(hipGetLastError());
+  return BBFMM_OK;
+}
+
+// one k chunk per iteration, or two where they come in pairs and the block's
+// tiles leave the registers for them
+static int launch_real(const GridArgs &a, int nb, hipStream_t s)
+{
+  const bool two = a.kt % 2 == 0;
+  if (!a.buf) return launch_real_t<1, 1, 1, false>(a, nb, s);
+  switch (a.rt * 10 + a.ct) {
+  case 11: return two ? launch_real_t<1, 1, 2>(a, nb, s) : launch_real_t<1, 1, 1>(a, nb, s);
+  case 12: return two ? launch_real_t<1, 2, 2>(a, nb, s) : launch_real_t<1, 2, 1>(a, nb, s);
+  case 14: return two ? launch_real_t<1, 4, 2>(a, nb, s) : launch_real_t<1, 4, 1>(a, nb, s);
+#ifdef SINGLE
+  case 22: return launch_real_t<2, 2, 2>(a, nb, s);  // r = 32 only
+  case 24: return two ? launch_real_t<2, 4, 2>(a, nb, s) : launch_real_t<2, 4, 1>(a, nb, s);
+  case 44: return launch_real_t<4, 4, 1>(a, nb, s);
+#else
+  case 21: return launch_real_t<2, 1, 2>(a, nb, s);  // r = 17 .. 32 only
+  case 42: return launch_real_t<4, 2, 1>(a, nb, s);
+#endif
+  default: return set_error(BBFMM_E_ARG, "internal: block of %d x %d tiles", a.rt, a.ct);
+  }
 }
 
 #ifdef SINGLE
@@ -1706,21 +1721,11 @@ int grid_m2l_run(GridM2L *g, const real *M, real *L, int ncell, hipStream_t s, h
   const int sb = (int)((cells * (a.r / 8) + 255) / 256);
   switch (g->form) {
   case BBFMM_M2L_PLAIN:
-    if (a.r % 8 == 0)
-      hipLaunchKernelGGL(k_grid_scatter<BBFMM_M2L_PLAIN>, dim3(sb), dim3(256), 0, s, a, M);
-    else
-      hipLaunchKernelGGL((k_grid_scatter<BBFMM_M2L_PLAIN, 1>), dim3((int)((cells * a.r + 255) / 256)), dim3(256), 0,
-                         s, a, M);
+  case BBFMM_M2L_FP32MFMA:
+    hipLaunchKernelGGL(k_real_scatter, dim3((unsigned)((cells * (16 * a.kt / kVW) + 255) / 256)), dim3(256), 0, s, a, M);
     BB_HIP(hipGetLastError());
     if (mid) BB_HIP(hipEventRecord(mid, s));
-    if (a.r == 32)
-      hipLaunchKernelGGL(k_m2l_grid_plain32, dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
-    else if (a.r != 256)
-      hipLaunchKernelGGL(k_m2l_grid_plain_any, dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
-    else
-      hipLaunchKernelGGL(k_m2l_grid_plain<256>, dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
-    BB_HIP(hipGetLastError());
-    return BBFMM_OK;
+    return launch_real(a, g->nblocks, s);
 #ifdef SINGLE
   case BBFMM_M2L_BF16X2:
     if (deep_in_grid) {  // the levels above the deepest only
@@ -1771,18 +1776,6 @@ int grid_m2l_run(GridM2L *g, const real *M, real *L, int ncell, hipStream_t s, h
       hipLaunchKernelGGL((k_m2l_mfma<BBFMM_M2L_FP16X3, 2>), dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
     else
       hipLaunchKernelGGL((k_m2l_mfma<BBFMM_M2L_FP16X3, 1>), dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
-    BB_HIP(hipGetLastError());
-    return BBFMM_OK;
-  case BBFMM_M2L_FP32MFMA:
-    hipLaunchKernelGGL(k_grid_scatter<BBFMM_M2L_FP32MFMA>, dim3(sb), dim3(256), 0, s, a, M);
-    BB_HIP(hipGetLastError());
-    if (mid) BB_HIP(hipEventRecord(mid, s));
-    if (a.r == 256)  // rounded up to whole rounds of the 8 XCDs; the extra blocks exit
-      hipLaunchKernelGGL(k_m2l_fp32_r256, dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
-    else if (a.wave_cols == 64)
-      hipLaunchKernelGGL((k_m2l_mfma<BBFMM_M2L_FP32MFMA, 2>), dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
-    else
-      hipLaunchKernelGGL((k_m2l_mfma<BBFMM_M2L_FP32MFMA, 1>), dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
     BB_HIP(hipGetLastError());
     return BBFMM_OK;
 #endif

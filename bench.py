@@ -338,7 +338,7 @@ def run_c3(args):
     r = 256
     inter = plan.m2l_interactions
     flop_m2l = r * (2 * r - 1) * inter * nrhs
-    roof = {"kernel": "k_m2l_fp32_r256", "bound": "mfma", "unit": "TFLOP/s",
+    roof = {"kernel": "k_m2l_real", "bound": "mfma", "unit": "TFLOP/s",
             "achieved": flop_m2l / (st["m2l"] * 1e-3) / 1e12, "peak": PEAK_FP32_TFLOPS,
             "launch_ms": st["m2l"], "algorithmic_flop_per_launch": flop_m2l, "traffic": None}
     roof["frac"] = roof["achieved"] / roof["peak"]
