@@ -3,13 +3,11 @@
 // (the semantics of the reference GPU kernel direct.cu:69-209 and the CPU
 // anotherNearField.c:137-206; the r != 0 test is applied in the self leaf).
 //
-// One 64-lane wavefront per leaf; the neighbour particles are staged in LDS
-// 64 at a time and every lane (target) sweeps them (or a 1/2, 1/4 share of
-// them on leaves of at most 32, 16 particles).  NR right-hand sides are
-// processed together so that the geometry (dx, dy, dz, 1/r) is computed once
-// per pair and shared by NR charge vectors.
+// Up to 8 right-hand sides are processed together so that the geometry (dx,
+// dy, dz, 1/r) is computed once per pair and shared by their charges; 16 take
+// the kernels on the padded layout.
 // 1/r: fp32 uses the hardware v_rsq_f32 (AMD's own reciprocal square root,
-// about 1 ulp); fp64 uses the device math library's rsqrt.
+// about 1 ulp); fp64 one iteration from v_rsq_f64 (rsqrt_r).
 #include "common.h"
 #include "kernels.h"
 
@@ -20,108 +18,14 @@ __device__ __forceinline__ real rsqrt_r(real x)
 #ifdef SINGLE
   return __builtin_amdgcn_rsqf(x);
 #else
-  return rsqrt(x);
+  // the hardware's estimate (5e-8) and one third-order step: as exact as the
+  // library's rsqrt (1.4e-16 at most over 1e-12 .. 100) without its special
+  // cases (x is positive and finite here, or the result is not used), 47
+  // against 60 cycles a wavefront
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-x * y, y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
 #endif
-}
-
-// A leaf of at most 16 (32) targets takes 16 (32) lanes per target and
-// splits every source chunk 4 (2) ways over the lane groups (source k to
-// group k mod S), the groups' sums added across lanes at the end, so that
-// the wavefront's 64 lanes stay busy on leaves of a few dozen particles.
-template <int NR>
-__global__ void __launch_bounds__(64) k_p2p(P2PArgs a, int rhs0)
-{
-  constexpr int CH = 64;
-  __shared__ real4 sp[CH];
-  __shared__ real sq[NR][CH];
-  __shared__ int nsta[27], ncnt[27], nself[27];
-  const int leaf = blockIdx.x;
-  const int t = threadIdx.x;
-  const int sta = a.leafsta[leaf], cnt = a.leafcnt[leaf];
-  const int nn = a.nnbr[leaf];
-  if (t < nn) {
-    const int B = a.nbr[(size_t)leaf * 27 + t];
-    nsta[t] = a.leafsta[B];
-    ncnt[t] = a.leafcnt[B];
-    nself[t] = (B == leaf);
-  }
-  __syncthreads();
-  const size_t N = a.N;
-  const int S = cnt <= 16 ? 4 : cnt <= 32 ? 2 : 1;  // source groups (uniform in the block)
-  const int T = CH / S;                              // targets per pass
-  const int tl = t % T, h = t / T;
-  for (int tb = 0; tb < cnt; tb += T) {
-    const int i = tb + tl;
-    const bool act = i < cnt;
-    real4 xf;
-    if (act) {
-      xf = a.pos[sta + i];
-    } else {
-      xf.x = xf.y = xf.z = xf.w = 0;
-    }
-    real acc[NR], acc2[NR];
-#pragma unroll
-    for (int r = 0; r < NR; r++) acc[r] = acc2[r] = 0;
-    for (int b = 0; b < nn; b++) {
-      const int jsta = nsta[b], nj = ncnt[b];
-      const bool self = nself[b] != 0;
-      for (int jb = 0; jb < nj; jb += CH) {
-        const int nk = min(CH, nj - jb);
-        if (t < nk) {
-          sp[t] = a.pos[jsta + jb + t];
-#pragma unroll
-          for (int r = 0; r < NR; r++) sq[r][t] = a.q[(size_t)(rhs0 + r) * N + jsta + jb + t];
-        }
-        __syncthreads();
-        if (!self) {
-          int k = h;
-          for (; k + S < nk; k += 2 * S) {
-            const real4 s0 = sp[k], s1 = sp[k + S];
-            const real dx0 = s0.x - xf.x, dy0 = s0.y - xf.y, dz0 = s0.z - xf.z;
-            const real dx1 = s1.x - xf.x, dy1 = s1.y - xf.y, dz1 = s1.z - xf.z;
-            const real w0 = rsqrt_r(dx0 * dx0 + dy0 * dy0 + dz0 * dz0);
-            const real w1 = rsqrt_r(dx1 * dx1 + dy1 * dy1 + dz1 * dz1);
-#pragma unroll
-            for (int r = 0; r < NR; r++) {
-              acc[r] += w0 * sq[r][k];
-              acc2[r] += w1 * sq[r][k + S];
-            }
-          }
-          if (k < nk) {
-            const real4 s0 = sp[k];
-            const real dx0 = s0.x - xf.x, dy0 = s0.y - xf.y, dz0 = s0.z - xf.z;
-            const real w0 = rsqrt_r(dx0 * dx0 + dy0 * dy0 + dz0 * dz0);
-#pragma unroll
-            for (int r = 0; r < NR; r++) acc[r] += w0 * sq[r][k];
-          }
-        } else {
-          for (int k = h; k < nk; k += S) {
-            const real4 s0 = sp[k];
-            const real dx0 = s0.x - xf.x, dy0 = s0.y - xf.y, dz0 = s0.z - xf.z;
-            const real rr = dx0 * dx0 + dy0 * dy0 + dz0 * dz0;
-            const real w0 = rr != (real)0 ? rsqrt_r(rr) : (real)0;
-#pragma unroll
-            for (int r = 0; r < NR; r++) acc[r] += w0 * sq[r][k];
-          }
-        }
-        __syncthreads();
-      }
-    }
-    real tot[NR];
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-      tot[r] = acc[r] + acc2[r];
-      if (S == 4) tot[r] += __shfl_xor(tot[r], 16);
-      if (S >= 2) tot[r] += __shfl_xor(tot[r], 32);
-    }
-    if (act && h == 0) {
-#pragma unroll
-      for (int r = 0; r < NR; r++) {
-        const size_t o = (size_t)(rhs0 + r) * N + sta + i;
-        a.phi[o] += (a.potential ? (real)1 : a.q[o]) * tot[r];
-      }
-    }
-  }
 }
 
 // Sparse forests, where leaves hold a few particles: a lane per target
@@ -218,6 +122,206 @@ __device__ __forceinline__ int xcd_leaf(int b, int nleaf)
 {
   if (nleaf & 7) return b;
   return (b & 7) * (nleaf >> 3) + (b >> 3);
+}
+
+// ---------------------------------------------------------------- 1 to 8 vectors
+// A wavefront's lanes are 16 targets x 4 source groups: group h takes the
+// staged sources h, h + 4, ... for up to NTMAX tiles of 16 targets of the
+// leaf, so that leaves of a few dozen particles keep the lanes busy (a lane a
+// target left half of them idle at 33 to 48 particles) and every source read
+// from LDS serves NT targets.  The groups' sums are added across lanes at the
+// end.  The W waves of a block take the neighbour leaves in turn, their sums
+// added through LDS; the target tiles of a leaf go to gridDim.y blocks, so
+// that few large leaves fill the chip too.  Each wave stages up to kP2PLeaves
+// leaves (64 sources of each) at a time in its own part of LDS, their loads
+// in flight together, padded to a multiple of 8 with far sources of zero
+// charge (no tail masks).  The r != 0 test is applied in the self leaf, which
+// wave 0 stages by itself.
+// Bound by the vector ALUs (7 + NR fp32 operations and a reciprocal square
+// root a pair; fp64: the library rsqrt).  N = 1M, depth 5, one vector: 467 -> 244
+// us (45 cycles of a SIMD per 64 pairs of whole tiles; the operations alone
+// measure 37); 4096, depth 2 (64 leaves of 64): 192 -> 11.7 us; 65536, depth
+// 4: 33 -> 21.5 us; fp64 100003, depth 4: 117 -> 60 us; 4 vectors of 150001
+// on a sphere, depth 5: 249 -> 85 us.
+constexpr int kP2PLeaves = 4;  // leaves staged together
+constexpr int kP2PStage = 64 * kP2PLeaves;
+
+typedef real realx4 __attribute__((ext_vector_type(4)));
+
+// position and, for one vector, charge of the staged sources; more charges beside them
+template <int NR>
+struct P2PStage {
+  realx4 s[kP2PStage];
+  real q[NR > 1 ? kP2PStage : 1][NR] __attribute__((aligned(16)));
+};
+
+// acc += the sums over the n8 (a multiple of 8) staged sources, two of a lane's at a time
+template <int NR, int NT, bool SELF>
+__device__ __forceinline__ void p2p_sweep(const P2PStage<NR> &st, int n8, int h, const realx4 *x, real (&acc)[NT][NR])
+{
+  for (int k = 0; k < n8; k += 8) {
+    realx4 z[2];
+    real q[2][NR];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      z[u] = st.s[k + 4 * u + h];
+#pragma unroll
+      for (int r = 0; r < NR; r++) q[u][r] = NR > 1 ? st.q[k + 4 * u + h][r] : z[u].w;
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        const real dx = z[u].x - x[t].x, dy = z[u].y - x[t].y, dz = z[u].z - x[t].z;
+        const real rr = dx * dx + dy * dy + dz * dz;
+        const real g = SELF && rr == (real)0 ? (real)0 : rsqrt_r(rr);
+#pragma unroll
+        for (int r = 0; r < NR; r++) acc[t][r] += g * q[u][r];
+      }
+  }
+}
+
+template <int NR, int NT>
+__device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, int leaf, int tb, int sta, int cnt,
+                                          int nsta, int ncnt, int nn, P2PStage<NR> &st, real *red)
+{
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), W = blockDim.x >> 6;
+  const int ti = lane & 15, h = lane >> 4;
+  const size_t N = a.N;
+  const realx4 *pos = reinterpret_cast<const realx4 *>(a.pos);
+  realx4 x[NT];
+  real acc[NT][NR];
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    x[t] = pos[sta + min(tb + 16 * t + ti, cnt - 1)];  // targets past the leaf's end are not stored
+#pragma unroll
+    for (int r = 0; r < NR; r++) acc[t][r] = 0;
+  }
+  // source `at` of the staged ones (lanes below n) from particle j + lane
+  auto load = [&](int j, int n, realx4 &p, real (&q)[NR]) {
+    const int i = j + min(lane, n - 1);
+    p = pos[i];
+#pragma unroll
+    for (int r = 0; r < NR; r++) q[r] = r < nv ? a.q[(size_t)(rhs0 + r) * N + i] : (real)0;
+  };
+  auto put = [&](int at, int n, const realx4 &p, const real (&q)[NR]) {
+    if (lane < n) {
+      realx4 v = p;
+      v.w = q[0];
+      st.s[at + lane] = v;
+      if (NR > 1)
+#pragma unroll
+        for (int r = 0; r < NR; r++) st.q[at + lane][r] = q[r];
+    }
+  };
+  auto pad = [&](int n) {  // to a multiple of 8
+    const int n8 = (n + 7) & ~7;
+    if (lane < n8 - n) {
+      st.s[n + lane] = realx4{(real)1e6, (real)1e6, (real)1e6, 0};
+      if (NR > 1)
+#pragma unroll
+        for (int r = 0; r < NR; r++) st.q[n + lane][r] = 0;
+    }
+    return n8;
+  };
+  if (wave == 0) {  // the leaf itself
+    for (int j = 0; j < cnt; j += 64) {
+      const int n = min(64, cnt - j);
+      realx4 p;
+      real q[NR];
+      load(sta + j, n, p, q);
+      put(0, n, p, q);
+      p2p_sweep<NR, NT, true>(st, pad(n), h, x, acc);
+    }
+  }
+  // the other leaves: items (leaf b, 64 sources from j) of this wave
+  int b = wave, j = 0;
+  while (b < nn) {
+    realx4 p[kP2PLeaves];
+    real q[kP2PLeaves][NR];
+    int n[kP2PLeaves];
+#pragma unroll
+    for (int g = 0; g < kP2PLeaves; g++) {
+      // (an empty leaf, the leaf itself: a step without sources)
+      n[g] = 0;
+      if (b < nn) {
+        const int c = __builtin_amdgcn_readlane(ncnt, b);
+        n[g] = min(64, c - j);
+        if (n[g] > 0) load(__builtin_amdgcn_readlane(nsta, b) + j, n[g], p[g], q[g]);
+        j += 64;
+        if (j >= c) {
+          j = 0;
+          b += W;
+        }
+      }
+    }
+    int at = 0;
+#pragma unroll
+    for (int g = 0; g < kP2PLeaves; g++)
+      if (n[g] > 0) {
+        put(at, n[g], p[g], q[g]);
+        at += n[g];
+      }
+    if (at > 0) p2p_sweep<NR, NT, false>(st, pad(at), h, x, acc);
+  }
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+      acc[t][r] += __shfl_xor(acc[t][r], 16);
+      acc[t][r] += __shfl_xor(acc[t][r], 32);
+    }
+  if (W > 1) {
+    __syncthreads();  // the previous pass's sums have been read
+    if (h == 0)
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int r = 0; r < NR; r++) red[((wave * NT + t) * NR + r) * 16 + ti] = acc[t][r];
+    __syncthreads();
+    if (wave > 0) return;
+    for (int w = 1; w < W; w++)
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int r = 0; r < NR; r++) acc[t][r] += red[((w * NT + t) * NR + r) * 16 + ti];
+  }
+#pragma unroll
+  for (int t = 0; t < NT; t++) {
+    const int i = tb + 16 * t + ti;
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+      const size_t o = (size_t)(rhs0 + r) * N + sta + i;
+      if (i < cnt && r < nv && (r & 3) == h) a.phi[o] += (a.potential ? (real)1 : a.q[o]) * acc[t][r];
+    }
+  }
+}
+
+// vectors rhs0 .. rhs0 + nv - 1 (nv <= NR)
+template <int NR, int NTMAX, int MAXW>
+__global__ void __launch_bounds__(64 * MAXW) k_p2p(P2PArgs a, int rhs0, int nv)
+{
+  __shared__ P2PStage<NR> stage[MAXW];
+  __shared__ real red[MAXW > 1 ? MAXW * NTMAX * NR * 16 : 1];
+  const int leaf = xcd_leaf(blockIdx.x, a.nleaf);
+  const int lane = threadIdx.x & 63;
+  const int sta = a.leafsta[leaf], cnt = a.leafcnt[leaf], nn = a.nnbr[leaf];
+  int nsta = 0, ncnt = 0;  // lane b: neighbour leaf b (the leaf itself without sources)
+  if (lane < nn) {
+    const int B = a.nbr[(size_t)leaf * 27 + lane];
+    nsta = a.leafsta[B];
+    ncnt = B == leaf ? 0 : a.leafcnt[B];
+  }
+  P2PStage<NR> &st = stage[threadIdx.x >> 6];
+  // passes of NTMAX tiles, dealt to the gridDim.y blocks
+  for (int tb = blockIdx.y * 16 * NTMAX; tb < cnt; tb += gridDim.y * 16 * NTMAX) {
+    const int nt = min(NTMAX, (cnt - tb + 15) >> 4);
+    if (NTMAX >= 4 && nt == 4) p2p_tiles<NR, (NTMAX >= 4 ? 4 : 1)>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
+    else if (NTMAX >= 3 && nt == 3) p2p_tiles<NR, (NTMAX >= 3 ? 3 : 1)>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
+    else if (NTMAX >= 2 && nt == 2) p2p_tiles<NR, (NTMAX >= 2 ? 2 : 1)>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
+    else p2p_tiles<NR, 1>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
+  }
 }
 
 #ifdef SINGLE
@@ -677,6 +781,58 @@ __global__ void k_pad_charges16(int N, const int *__restrict__ pad_of, const flo
 }
 #endif
 
+template <int NR, int NTMAX, int W>
+static void p2p_few_t(const P2PArgs &a, int rhs, int nv, hipStream_t s)
+{
+  hipLaunchKernelGGL((k_p2p<NR, NTMAX, W>), dim3(a.nleaf, 4), dim3(64 * W), 0, s, a, rhs, nv);
+}
+
+// Tiles of a pass and waves of a block.  Many leaves fill the chip with a
+// wave each, and more tiles a pass read fewer staged sources per pair; few
+// leaves need their sources split over waves, as far as the waves' LDS leaves
+// room for enough of them.  The target tiles of a leaf are dealt to 4 blocks
+// (those without tiles end at once): N = 50000, 512 leaves 42.9 against 52.5
+// us on one block, surface 150001 85 against 130.  P2P in us, tiles x waves:
+//   fp32, 1 vector:  1M, 32768 leaves 4x1 244, 4x4 262; 262144, 4096 leaves
+//                    4x4 118, 4x1 123; 65536, 4096 leaves 2x4 21.5, 4x1 24.8;
+//                    50000, 512 leaves 2x8 42.9, 2x4 47.1; 4096, 64 leaves
+//                    2x8 11.7, 2x4 14.5, 4x8 15.1
+//   fp32, 4 vectors: 262144 4x4 170.5, 4x1 171.9; 65536 2x1 33.6, 2x4 39.7;
+//                    50000 2x4 63.4, 2x8 65.8; 4096 2x8 15.2, 2x4 19.1
+//   fp32, 7 vectors: 1M 4x1 524, 2x1 633; 16384, 512 leaves 2x4 24.1
+//   fp64:            100003, 4096 leaves, 1 vector 2x4 67.7, 2x1 71.7, 4
+//                    vectors 2x1 109.7, 2x4 128; 8000, 64 leaves, 1 vector
+//                    2x4 62.6, 2x1 177; 40000, 512 leaves, 7 vectors 2x1 177,
+//                    2x4 222
+template <int NR>
+static void p2p_few_n(const P2PArgs &a, int rhs, int nv, hipStream_t s)
+{
+#ifdef SINGLE
+  if (a.nleaf <= 1024) {
+    if (NR == 1 || (NR < 8 && a.nleaf <= 128)) p2p_few_t<NR, 2, NR < 8 ? 8 : 4>(a, rhs, nv, s);
+    else p2p_few_t<NR, 2, 4>(a, rhs, nv, s);
+  } else if (a.N > 24LL * a.nleaf) {
+    if (NR == 1 && a.nleaf <= 6144) p2p_few_t<NR, 4, NR == 1 ? 4 : 1>(a, rhs, nv, s);
+    else p2p_few_t<NR, 4, 1>(a, rhs, nv, s);
+  } else {
+    if (NR == 1 && a.nleaf <= 6144) p2p_few_t<NR, 2, 4>(a, rhs, nv, s);
+    else p2p_few_t<NR, 2, 1>(a, rhs, nv, s);
+  }
+#else
+  if (a.nleaf <= (NR == 1 ? 6144 : NR < 8 ? 1024 : 128)) p2p_few_t<NR, 2, 4>(a, rhs, nv, s);
+  else p2p_few_t<NR, 2, 1>(a, rhs, nv, s);
+#endif
+}
+
+// nv (1 to 8) vectors from rhs
+static void p2p_few(const P2PArgs &a, int rhs, int nv, hipStream_t s)
+{
+  if (nv > 4) p2p_few_n<8>(a, rhs, nv, s);
+  else if (nv > 2) p2p_few_n<4>(a, rhs, nv, s);
+  else if (nv == 2) p2p_few_n<2>(a, rhs, nv, s);
+  else p2p_few_n<1>(a, rhs, nv, s);
+}
+
 int launch_p2p(const P2PArgs &a, hipStream_t s)
 {
   if (a.nleaf <= 0 || a.N <= 0) return BBFMM_OK;
@@ -726,14 +882,12 @@ int launch_p2p(const P2PArgs &a, hipStream_t s)
           hipLaunchKernelGGL(k_p2p_seg16<false>, dim3(a.nleaf), dim3(64), 0, s, a, rhs);
       } else
 #endif
-        hipLaunchKernelGGL(k_p2p<16>, dim3(a.nleaf), dim3(64), 0, s, a, rhs);
+        for (int v = 0; v < 16; v += 8) p2p_few(a, rhs + v, 8, s);
       rhs += 16;
-    } else if (left >= 4) {
-      hipLaunchKernelGGL(k_p2p<4>, dim3(a.nleaf), dim3(64), 0, s, a, rhs);
-      rhs += 4;
     } else {
-      hipLaunchKernelGGL(k_p2p<1>, dim3(a.nleaf), dim3(64), 0, s, a, rhs);
-      rhs += 1;
+      const int nv = left < 8 ? left : 8;
+      p2p_few(a, rhs, nv, s);
+      rhs += nv;
     }
     BB_HIP(hipGetLastError());
   }
