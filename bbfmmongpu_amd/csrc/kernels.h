@@ -7,6 +7,15 @@
 
 namespace bb {
 
+// Blocks are dispatched round-robin over the 8 XCDs (each with its own L2):
+// give XCD x the x-th contiguous eighth of the leaves (Morton order), so that
+// neighbouring leaves, which read the same sources, share an L2.
+__device__ __forceinline__ int xcd_leaf(int b, int nleaf)
+{
+  if (nleaf & 7) return b;
+  return (b & 7) * (nleaf >> 3) + (b >> 3);
+}
+
 // Everything the pass kernels read, by value (device pointers).
 struct PassArgs {
   int N, n, r, ncell, maxlev, nleaf;
@@ -225,8 +234,10 @@ struct GradArgs {
   const real *F;                     // [2m][ncell][n^3] local values after L2L
   const real *qg;                    // [2m][N] leaf order
   real *dx;                          // [3][N] leaf order (scratch)
+  real *phi;                         // [2m][N] leaf order: far-field potentials; rows m.. get the near field added
 };
 // dx_out [N][3] (original order) = position gradient; iperm: original -> leaf order
+// The near field of the potentials of the vectors m .. 2m - 1 is added to phi on the way.
 int launch_gradient(const GradArgs &a, const int *iperm, real *dx_out, hipStream_t s);
 
 // ---- FP64 operator precompute ----

@@ -115,15 +115,6 @@ __global__ void k_pack_pq(int N, const real4 *__restrict__ pos, const real *__re
   pq[i] = v;
 }
 
-// Blocks are dispatched round-robin over the 8 XCDs (each with its own L2):
-// give XCD x the x-th contiguous eighth of the leaves (Morton order), so that
-// neighbouring leaves, which read the same sources, share an L2.
-__device__ __forceinline__ int xcd_leaf(int b, int nleaf)
-{
-  if (nleaf & 7) return b;
-  return (b & 7) * (nleaf >> 3) + (b >> 3);
-}
-
 // ---------------------------------------------------------------- 1 to 8 vectors
 // A wavefront's lanes are 16 targets x 4 source groups: group h takes the
 // staged sources h, h + 4, ... for up to NTMAX tiles of 16 targets of the
@@ -360,7 +351,7 @@ template <int NT>
 __device__ __forceinline__ void p2p16_store_t(const P2PArgs &a, int rhs0, int sta, int cnt, int psta, int tb,
                                               const f32x4 *acc)
 {
-  const int l = threadIdx.x;
+  const int l = threadIdx.x & 63;
   const int ti = l & 15, kq = l >> 4;
   if (a.phin) {
 #pragma unroll
@@ -443,11 +434,12 @@ __device__ __forceinline__ void p2p16_store(const P2PArgs &a, int rhs0, int sta,
 // BUF: the source positions and charge rows are read with buffer loads whose
 // group offset is a scalar register (the padded arrays then stay below 2 GB),
 // so no vector instructions go into the per-group addresses.
-template <int NT, bool BUF>
+template <int NT, bool BUF, int W>
 __device__ __forceinline__ void p2p16_pass(const P2PArgs &a, int rhs0, int2 sg, int nseg, int T, int sta,
-                                           int cnt, int psta, int pself, int tb)
+                                           int cnt, int psta, int pself, int tb, f32x4 *red)
 {
-  const int l = threadIdx.x;
+  const int l = threadIdx.x & 63;
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
   const int ti = l & 15, kq = l >> 4;
   const float4 *P = reinterpret_cast<const float4 *>(a.ppos);
   const float *Qt = a.qt;
@@ -482,7 +474,7 @@ __device__ __forceinline__ void p2p16_pass(const P2PArgs &a, int rhs0, int2 sg, 
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(bq, g[t], acc[t], 0, 0, 0);
   };
-  if (pself > 0) {
+  if (pself > 0 && wave == 0) {
     float4 zA = src_pos(psta);
     float qA = src_q(psta);
     for (int k = 0; k < pself; k += 8) {
@@ -497,10 +489,24 @@ __device__ __forceinline__ void p2p16_pass(const P2PArgs &a, int rhs0, int2 sg, 
       self_step(zB, qB);
     }
   }
-  if (T > 0) {
+  // this wave's groups of the other leaves (W > 1: the first wave, which has
+  // the self leaf too, takes the fewer)
+  const int T0 = W > 1 ? max(0, (int)((T + (pself >> 2)) * wave / W) - (pself >> 2)) : 0;
+  const int Tn = (W > 1 ? max(0, (int)((T + (pself >> 2)) * (wave + 1) / W) - (pself >> 2)) : T) - T0;
+  if (Tn > 0) {
     int b = 1;
     int pos = __builtin_amdgcn_readlane(sg.x, 1);
     int end = pos + __builtin_amdgcn_readlane(sg.y, 1);
+    if (W > 1) {
+      int skip = 4 * T0;
+      while (skip >= end - pos) {
+        skip -= end - pos;
+        b++;
+        pos = __builtin_amdgcn_readlane(sg.x, b);
+        end = pos + __builtin_amdgcn_readlane(sg.y, b);
+      }
+      pos += skip;
+    }
     // next group; stays on the last group at the end (loaded, never summed)
     auto advance = [&]() {
       if (pos + 4 < end) {
@@ -523,19 +529,30 @@ __device__ __forceinline__ void p2p16_pass(const P2PArgs &a, int rhs0, int2 sg, 
     load(y0, q0);
     load(y1, q1);
     load(y2, q2);
-    for (int t = 0; t < T; t += 4) {
+    for (int t = 0; t < Tn; t += 4) {
       load(y3, q3);
       p2p16_step<NT>(y0, q0, x, acc);
-      if (t + 1 >= T) break;
+      if (t + 1 >= Tn) break;
       load(y0, q0);
       p2p16_step<NT>(y1, q1, x, acc);
-      if (t + 2 >= T) break;
+      if (t + 2 >= Tn) break;
       load(y1, q1);
       p2p16_step<NT>(y2, q2, x, acc);
-      if (t + 3 >= T) break;
+      if (t + 3 >= Tn) break;
       load(y2, q2);
       p2p16_step<NT>(y3, q3, x, acc);
     }
+  }
+  if (W > 1) {
+    __syncthreads();  // the previous pass's sums have been read
+    if (wave > 0)
+#pragma unroll
+      for (int t = 0; t < NT; t++) red[((wave - 1) * NT + t) * 64 + l] = acc[t];
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      for (int w = 0; w < W - 1; w++) acc[t] += red[(w * NT + t) * 64 + l];
   }
   p2p16_store_t<NT>(a, rhs0, sta, cnt, psta, tb, acc);
 }
@@ -547,35 +564,51 @@ __device__ __forceinline__ void p2p16_pass(const P2PArgs &a, int rhs0, int2 sg, 
 // target, stored as one 16-byte piece of its row).  The self leaf is
 // summed first with the r != 0 exclusion; the other neighbours form one
 // flattened sequence of 4-source groups, loaded three groups ahead into a
-// ring of four register sets.  Up to four target tiles share a pass.
-template <bool BUF>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(7))) k_p2p_seg16(P2PArgs a, int rhs0)
+// ring of four register sets.  Up to ntp target tiles share a pass; the
+// passes are dealt to gridDim.y blocks, and the W waves of a block take equal
+// parts of the groups, their sums added through LDS.
+template <bool BUF, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W > 4 ? 5 : W > 1 ? 6 : 7)))
+    k_p2p_seg16(P2PArgs a, int rhs0, int ntp)
 {
+  __shared__ f32x4 red[W > 1 ? (W - 1) * 4 * 64 : 1];
   const int leaf = xcd_leaf(blockIdx.x, a.nleaf);
-  const int l = threadIdx.x;
+  const int l = threadIdx.x & 63;
   const int sta = a.leafsta[leaf], cnt = a.leafcnt[leaf];
-  if (cnt == 0) return;
+  // as few passes of equal tiles as ntp allows
+  const int tiles = (cnt + 15) >> 4, np = W > 1 ? (tiles + ntp - 1) / ntp : 1;
+  if (cnt == 0 || (int)blockIdx.y >= np) return;
   const int nseg = a.nseg[leaf];
   const int2 sg = l < nseg ? a.seg[(size_t)leaf * 27 + l] : make_int2(0, 0);
   const int psta = __builtin_amdgcn_readfirstlane(sg.x);
   const int pself = __builtin_amdgcn_readfirstlane(sg.y);
   int T = 0;
   for (int b = 1; b < nseg; b++) T += __builtin_amdgcn_readlane(sg.y, b) >> 2;
-  for (int tb = 0; tb < cnt;) {
-    const int tiles = (cnt - tb + 15) >> 4;
-    if (tiles >= 4) {
-      p2p16_pass<4, BUF>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb);
-      tb += 64;
-    } else if (tiles == 3) {
-      p2p16_pass<3, BUF>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb);
-      tb += 48;
-    } else if (tiles == 2) {
-      p2p16_pass<2, BUF>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb);
-      tb += 32;
-    } else {
-      p2p16_pass<1, BUF>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb);
-      tb += 16;
+  if (W == 1) {  // all passes here, up to 4 tiles each
+    for (int tb = 0; tb < cnt;) {
+      const int nt = (cnt - tb + 15) >> 4;
+      if (nt >= 4) {
+        p2p16_pass<4, BUF, W>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb, red);
+        tb += 64;
+      } else if (nt == 3) {
+        p2p16_pass<3, BUF, W>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb, red);
+        tb += 48;
+      } else if (nt == 2) {
+        p2p16_pass<2, BUF, W>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb, red);
+        tb += 32;
+      } else {
+        p2p16_pass<1, BUF, W>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb, red);
+        tb += 16;
+      }
     }
+    return;
+  }
+  for (int p = blockIdx.y; p < np; p += gridDim.y) {
+    const int t0 = tiles * p / np, nt = tiles * (p + 1) / np - t0, tb = 16 * t0;
+    if (nt >= 4) p2p16_pass<4, BUF, W>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb, red);
+    else if (nt == 3) p2p16_pass<3, BUF, W>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb, red);
+    else if (nt == 2) p2p16_pass<2, BUF, W>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb, red);
+    else p2p16_pass<1, BUF, W>(a, rhs0, sg, nseg, T, sta, cnt, psta, pself, tb, red);
   }
 }
 
@@ -833,6 +866,33 @@ static void p2p_few(const P2PArgs &a, int rhs, int nv, hipStream_t s)
   else p2p_few_n<1>(a, rhs, nv, s);
 }
 
+#ifdef SINGLE
+template <bool BUF, int W>
+static void p2p_seg16_t(const P2PArgs &a, int rhs, int ntp, hipStream_t s)
+{
+  hipLaunchKernelGGL((k_p2p_seg16<BUF, W>), dim3(a.nleaf, W > 1 ? 4 : 1), dim3(64 * W), 0, s, a, rhs, ntp);
+}
+
+// Tiles of a pass and waves of a block of the 16-vector near field, as for
+// few vectors.  Many leaves fill the chip with a wave each and are spared the
+// blocks without tiles.  Less than 8
+// particles a leaf on average means that most are empty (a surface) and the
+// others are large.  P2P in us, tiles x waves (4 blocks a leaf), and one wave
+// a leaf of up to 4 tiles before:
+//   4096, 64 leaves 2x8 16.3, 2x4 21.1 (118); 50021, 512 leaves 2x4 78.7, 4x4
+//   86.0 (265); 262144, 4096 leaves 4x4 233, 4x2 235 (350); 131072 4x4 78.2
+//   (106); 65536 4x4 36.1, 4x2 35.8 (44.6); 1M, 32768 leaves 4x1 490 (4 blocks
+//   502), 4x2 504; 150001 on a sphere, 32768 leaves 4x4 85.1, 4x2 97.8 (201)
+template <bool BUF>
+static void p2p_seg16(const P2PArgs &a, int rhs, hipStream_t s)
+{
+  if (a.nleaf <= 128) p2p_seg16_t<BUF, 8>(a, rhs, 2, s);
+  else if (a.nleaf <= 1024) p2p_seg16_t<BUF, 4>(a, rhs, 2, s);
+  else if (a.nleaf <= 8192 || a.N < 8LL * a.nleaf) p2p_seg16_t<BUF, 4>(a, rhs, 4, s);
+  else p2p_seg16_t<BUF, 1>(a, rhs, 4, s);
+}
+#endif
+
 int launch_p2p(const P2PArgs &a, hipStream_t s)
 {
   if (a.nleaf <= 0 || a.N <= 0) return BBFMM_OK;
@@ -877,9 +937,9 @@ int launch_p2p(const P2PArgs &a, hipStream_t s)
           else
             hipLaunchKernelGGL(k_p2p_seg16x<4>, dim3(a.nleaf), dim3(64), 0, s, a, rhs);
         } else if (!a.flat && a.npad > 0 && a.npad < (1 << 25))  // charge rows below 2 GB: scalar-offset buffer loads
-          hipLaunchKernelGGL(k_p2p_seg16<true>, dim3(a.nleaf), dim3(64), 0, s, a, rhs);
+          p2p_seg16<true>(a, rhs, s);
         else
-          hipLaunchKernelGGL(k_p2p_seg16<false>, dim3(a.nleaf), dim3(64), 0, s, a, rhs);
+          p2p_seg16<false>(a, rhs, s);
       } else
 #endif
         for (int v = 0; v < 16; v += 8) p2p_few(a, rhs + v, 8, s);

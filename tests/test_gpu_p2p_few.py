@@ -1,4 +1,4 @@
-"""The near field of 1 to 8 vectors (k_p2p) at the sizes where its tiles,
+"""The near field of 1 to 8 vectors (k_p2p) and of 16 (k_p2p_seg16) at the sizes where its tiles,
 staging and splits change: leaves of 0, 1, 15 .. 17, 63 .. 65 and hundreds of
 particles, coincident particles, every tile and wave count that the size rule
 picks, vector counts that leave part of a group.  Zero operators leave the
@@ -25,7 +25,7 @@ def _near(pos, q, depth, targets):
     return out
 
 
-def _check(prec, pos, depth, nrhs, cuda, ntargets, output="potential"):
+def _check(prec, pos, depth, nrhs, cuda, ntargets, output="potential", **opts):
     import torch
     import bbfmmongpu_amd as B
     dt = B.dtype(prec)
@@ -40,7 +40,7 @@ def _check(prec, pos, depth, nrhs, cuda, ntargets, output="potential"):
         lmod += 1
     plan = B.Plan(pos, 4, np.zeros(64 * 32, dt), np.zeros(316 * 1024, dt), nrhs=nrhs, lmod=lmod, prec=prec)
     assert plan.maxlev == depth
-    plan.set(scheme=B.SCHEME_IJ, form=B.FORM_PLAIN, output=output)
+    plan.set(scheme=B.SCHEME_IJ, output=output, **opts)
     phi = plan.solve(torch.from_numpy(q).to(cuda)).cpu().numpy().reshape(nrhs, N)
     plan.close()
     t = rng.choice(N, size=min(ntargets, N), replace=False)
@@ -52,11 +52,9 @@ def _check(prec, pos, depth, nrhs, cuda, ntargets, output="potential"):
     assert num.max() < TOL[prec]
 
 
-@pytest.mark.parametrize("prec", ["s", "d"])
-@pytest.mark.parametrize("nrhs", [1, 2, 3, 4, 5, 8, 9])
-def test_uneven_leaves(prec, nrhs, cuda):
-    """Depth 2: leaves of the counts where tiles and staged pieces end, most others empty or single."""
-    rng = np.random.default_rng(nrhs)
+def _uneven(seed):
+    """Depth 2: leaves of the counts where tiles and staged pieces end, the others empty."""
+    rng = np.random.default_rng(seed)
     counts = {0: 1, 1: 15, 2: 16, 3: 17, 5: 31, 6: 33, 8: 63, 9: 64, 10: 65, 13: 130, 20: 260, 42: 49, 63: 7}
     pos = []
     for leaf, c in counts.items():
@@ -64,7 +62,13 @@ def test_uneven_leaves(prec, nrhs, cuda):
         pos.append(corner + rng.random((c, 3)) / 4)
     pos = np.concatenate(pos)
     pos[20] = pos[19]  # coincident particles do not act on each other
-    _check(prec, pos, 2, nrhs, cuda, 200, output="q_phi" if nrhs == 2 else "potential")
+    return pos
+
+
+@pytest.mark.parametrize("prec", ["s", "d"])
+@pytest.mark.parametrize("nrhs", [1, 2, 3, 4, 5, 8, 9])
+def test_uneven_leaves(prec, nrhs, cuda):
+    _check(prec, _uneven(nrhs), 2, nrhs, cuda, 200, output="q_phi" if nrhs == 2 else "potential")
 
 
 @pytest.mark.parametrize("prec,N,depth,nrhs", [
@@ -76,3 +80,14 @@ def test_uneven_leaves(prec, nrhs, cuda):
 def test_size_rules(prec, N, depth, nrhs, cuda):
     pos = np.random.default_rng(N).random((N, 3)) - 0.5
     _check(prec, pos, depth, nrhs, cuda, 100)
+
+
+@pytest.mark.parametrize("flat", [False, True])
+@pytest.mark.parametrize("N,depth,nrhs", [
+    (0, 2, 16), (0, 2, 12), (20_000, 3, 16), (30_001, 4, 16),  # 64 leaves: 8 waves; 512, 4096: 4 waves
+    (60_000, 5, 16), (300_000, 5, 13), (20_000, 3, 33),  # 32768: 4 waves below 8 a leaf, else 1; two blocks of 16 and 1
+])
+def test_sixteen(N, depth, nrhs, flat, cuda):
+    import bbfmmongpu_amd as B
+    pos = np.random.default_rng(N).random((N, 3)) - 0.5 if N else _uneven(nrhs)
+    _check("s", pos, depth, nrhs, cuda, 100, form=B.FORM_BF16X2, flat_loads=flat)
