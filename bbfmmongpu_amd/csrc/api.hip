@@ -845,7 +845,9 @@ static bool near_beside(const bbfmm_amd_plan *p, bool rows)
   return rows && p->near_stream && p->side && p->d_phin;
 }
 
-static int solve_sorted(bbfmm_amd_plan *p, bool tm, bool rows)
+// near: with P2P (the gradient adds the near field itself, for the vectors
+// whose potentials it returns)
+static int solve_sorted(bbfmm_amd_plan *p, bool tm, bool rows, bool near = true)
 {
   hipStream_t s = p->stream;
   PassArgs a = pass_args(p, rows);
@@ -853,13 +855,13 @@ static int solve_sorted(bbfmm_amd_plan *p, bool tm, bool rows)
   const int nv = rows ? p->width : p->nrhs;  // vectors this solve computes
   pp.nrhs = nv;
 #ifdef SINGLE
-  if (pp.use_mfma && nv >= 16) {
+  if (near && pp.use_mfma && nv >= 16) {
     if (!p->d_qt) return set_error(BBFMM_E_ARG, "internal: solve not prepared");
     pp.qt = p->d_qt;
     if (rows) pp.phit = p->d_phit;
   }
 #endif
-  const bool beside = near_beside(p, rows);  // particle rows: fp32 build only
+  const bool beside = near && near_beside(p, rows);  // particle rows: fp32 build only
   // fork after the M2L: P2P (compute-bound) then shares the GPU with the
   // latency-bound downward pass
   auto fork_near = [&]() -> int {
@@ -927,7 +929,7 @@ static int solve_sorted(bbfmm_amd_plan *p, bool tm, bool rows)
   if (tm) BB_HIP(hipEventRecord(stage_event(p, ST_P2P), s));
   if (beside)
     BB_HIP(hipStreamWaitEvent(s, p->ev_join, 0));  // join
-  else
+  else if (near)
     BB_TRY(launch_p2p(pp, s));
   return BBFMM_OK;
 }
@@ -1372,11 +1374,9 @@ extern "C" int bbfmm_amd_gradient(bbfmm_amd_plan *p, const real *q_dev, const re
   BB_TRY(prepare_solve(p));
   const int saved_potential = p->potential;
   p->potential = 1;
-  const int rc = solve_sorted(p, false, false);  // not a timed solve
+  const int rc = solve_sorted(p, false, false, false);  // not a timed solve; the far field
   p->potential = saved_potential;
   BB_TRY(rc);
-  // dLoss/dq = A g: the potentials of the g vectors
-  BB_TRY(launch_scatter(p->d_iperm, p->d_phi + (size_t)m * N, dq_dev, N, m, s));
   GradArgs ga;
   ga.N = N;
   ga.n = p->n;
@@ -1398,7 +1398,10 @@ extern "C" int bbfmm_amd_gradient(bbfmm_amd_plan *p, const real *q_dev, const re
   ga.F = p->d_F;
   ga.qg = p->d_q;
   ga.dx = p->d_grad;
+  ga.phi = p->d_phi;
   BB_TRY(launch_gradient(ga, p->d_iperm, dx_dev, s));
+  // dLoss/dq = A g: the potentials of the g vectors
+  BB_TRY(launch_scatter(p->d_iperm, p->d_phi + (size_t)m * N, dq_dev, N, m, s));
   p->solved = true;
   return BBFMM_OK;
 }
