@@ -82,7 +82,8 @@ struct GridArgs {
   // tiles, column tiles and waves (offset slices); row groups of a column
   // group; 1: buffer loads
   int kt, rt, ct, ws, nrg, buf;
-  size_t plane;  // reals of one coefficient plane of the grids
+  size_t plane;  // values of one coefficient plane of the grids
+  int few;       // 1: split-BF16 on few columns (k_m2l_bf16_few; ct, ws, plane as above)
 };
 
 constexpr int kSteps = 208;  // 8 source classes x 26 non-zero parent shifts
@@ -1165,6 +1166,184 @@ __global__ void __launch_bounds__(64 * MAXW) k_m2l_real(GridArgs g)
   }
 }
 
+#ifdef SINGLE
+// ---------------------------------------------------------------- split-BF16, few columns
+// The split-BF16 products on few columns, blocked as the full-precision
+// kernel: a block is one class, all 32 rows and CT tiles of 16 columns of one
+// level, its waves take the offsets in slices; v_mfma_f32_16x16x32_bf16 takes
+// the whole rank at once.  Two offsets' fragments are loaded while the two
+// before are multiplied (past a slice's end: the zero operator).  Operators
+// [k][row tile][hi, lo][lane][8] (k_few_layout): lane l holds row 16 tile +
+// l % 16, columns 8 (l / 16) .. + 7.  Grids, hi and lo: [plane][slot][rhs][8],
+// plane p the coefficients 8 p .. 8 p + 7 (k_few_scatter).
+// Bound by latency and by the loads (6 KB per 6 products of 16 cycles at CT =
+// 1).  M2L of 50021 particles, depth 3, 16 vectors: 86 us with 32-column
+// tiles a wave and all offsets in turn, so 23; 4096, depth 2: 74 and 10.5.
+__global__ void __launch_bounds__(256) k_few_layout(const float *__restrict__ K, __bf16 *__restrict__ out)
+{
+  const int o = blockIdx.x * 256 + threadIdx.x;  // [k][tile][lane][8]
+  if (o >= (kNumOps + 1) * 1024) return;
+  const int e = o & 7, lane = (o >> 3) & 63, t = (o >> 9) & 1, k = o >> 10;
+  const int row = 16 * t + (lane & 15), col = 8 * (lane >> 4) + e;
+  const float v = k < kNumOps ? K[(size_t)k * 1024 + col * 32 + row] : 0.0f;
+  const __bf16 h = (__bf16)v;
+  const size_t at = ((size_t)(2 * k + t) * 2 * 64 + lane) * 8 + e;
+  out[at] = h;
+  out[at + 64 * 8] = (__bf16)(v - (float)h);
+}
+
+// M [rhs][ncell][32] -> the hi and lo planes, a thread 8 coefficients of a cell and vector
+__global__ void __launch_bounds__(256) k_few_scatter(GridArgs g, const float *__restrict__ M)
+{
+  const int total = (g.levsta[g.maxlev + 1] - g.levsta[g.minlev]) * g.nrhs * 4;
+  const int t = blockIdx.x * 256 + threadIdx.x;
+  if (t >= total) return;
+  const int rhs = t % g.nrhs, p = t / g.nrhs & 3, A = g.levsta[g.minlev] + t / g.nrhs / 4;
+  int l = g.minlev;
+  while (A >= g.levsta[l + 1]) l++;
+  int x, y, z;
+  demorton3(A - g.levsta[l], l, x, y, z);
+  const size_t slot = grid_slot(g, l, ((x & 1) << 2) | ((y & 1) << 1) | (z & 1), x >> 1, y >> 1, z >> 1);
+  const float *src = M + ((size_t)rhs * g.ncell + A) * 32 + 8 * p;
+  bf16x8 hi, lo;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const __bf16 h = (__bf16)src[e];
+    hi[e] = h;
+    lo[e] = (__bf16)(src[e] - (float)h);
+  }
+  const size_t dst = p * g.plane + (slot * g.nrhs + rhs) * 8;
+  *reinterpret_cast<bf16x8 *>((__bf16 *)g.Mg0 + dst) = hi;
+  *reinterpret_cast<bf16x8 *>((__bf16 *)g.Mg1 + dst) = lo;
+}
+
+template <int CT>
+__global__ void __launch_bounds__(512) k_m2l_bf16_few(GridArgs g)
+{
+  constexpr int G = CT == 1 ? 2 : 1;  // offsets per iteration
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  f32x4 *red = reinterpret_cast<f32x4 *>(smem_raw);  // [slice][tile][64]
+  __shared__ int2 lst[192];  // offsets to multiply: operator, slot shift
+  __shared__ int nlst;
+  const int lane = threadIdx.x & 63;
+  const int ws = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int s = blockIdx.x & 7, gb = blockIdx.x >> 3;
+  int l = g.minlev;
+  while (l < g.maxlev && gb >= g.blk0[l + 1]) l++;
+  const int P = 1 << (l - 1);
+  const int PP = P + 2;
+  const int ncols = P * P * P * g.nrhs;
+  const int col0 = (gb - g.blk0[l]) * (16 * CT);
+  if (ws == 0) {
+    const WaveBox box = wave_box(col0, ncols, g.nrhs, P, 16 * CT);
+    int n = 0;
+    for (int q = 0; q < 3; q++) {
+      const int v = 64 * q + lane;
+      const int4 e = g.tab[s * kOffsets + min(v, kOffsets - 1)];
+      const bool on = v < kOffsets && !ghost_step(box, e.z << 3, P);
+      const unsigned long long act = __ballot(on);
+      const int dx = (e.z >> 4) & 3, dy = (e.z >> 2) & 3, dz = e.z & 3;  // shift + 1
+      if (on)
+        lst[n + __popcll(act & ((1ull << lane) - 1))] =
+            make_int2(e.x, (e.y * PP * PP * PP + (dx * PP + dy) * PP + dz) * g.nrhs);
+      n += __popcll(act);
+    }
+    if (lane == 0) nlst = n;
+  }
+  unsigned bo[CT];
+#pragma unroll
+  for (int t = 0; t < CT; t++) {
+    const int col = min(col0 + 16 * t + (lane & 15), ncols - 1);  // columns past the end are not stored
+    const int pl = col / g.nrhs, rh = col - pl * g.nrhs;
+    const int pz = pl % P, py = (pl / P) % P, px = pl / (P * P);
+    const int slot = g.lvl_slot0[l] + (px * PP + py) * PP + pz;  // shifts count from (-1, -1, -1)
+    bo[t] = (unsigned)(((lane >> 4) * g.plane + ((size_t)slot * g.nrhs + rh) * 8) * 2);
+  }
+  // few columns: operators and grids are far below 2 GB
+  const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void *)g.Ka, 0, g.kbytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rH = __builtin_amdgcn_make_buffer_rsrc((void *)g.Mg0, 0, g.gbytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rL = __builtin_amdgcn_make_buffer_rsrc((void *)g.Mg1, 0, g.gbytes, 0x00020000);
+  struct Frag {
+    bf16x8 a[G][2][2], h[G][CT], l[G][CT];
+  };
+  constexpr int kLoads = G * (4 + 2 * CT);
+  auto load = [&](Frag &f, int j, int n) {
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+      const int jj = j + u * g.ws;
+      const int2 e = lst[min(jj, n - 1)];
+      const int k = __builtin_amdgcn_readfirstlane(jj < n ? e.x : kZeroOp);
+      const int so = __builtin_amdgcn_readfirstlane(e.y) * 16;
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+          f.a[u][t][q] = __builtin_bit_cast(
+              bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rK, lane * 16 + (2 * t + q) * 1024, k * 4096, 0));
+#pragma unroll
+      for (int t = 0; t < CT; t++) {
+        f.h[u][t] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rH, (int)bo[t], so, 0));
+        f.l[u][t] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rL, (int)bo[t], so, 0));
+      }
+    }
+  };
+  f32x4 acc[2][CT];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int t = 0; t < CT; t++) acc[i][t] = f32x4{0, 0, 0, 0};
+  auto mac = [&](const Frag &f) {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(kWaitVm0 | (kLoads & 15) | ((kLoads >> 4) << 14));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < G; u++)
+#pragma unroll
+      for (int q = 0; q < 3; q++)  // hi hi, hi lo, lo hi
+#pragma unroll
+        for (int t = 0; t < CT; t++)
+#pragma unroll
+          for (int i = 0; i < 2; i++)
+            acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[u][i][q == 2], q == 1 ? f.l[u][t] : f.h[u][t],
+                                                                acc[i][t], 0, 0, 0);
+  };
+  __syncthreads();
+  const int n = __builtin_amdgcn_readfirstlane(nlst);
+  if (ws < n) {
+    Frag f0, f1;
+    int j = ws;
+    const int step = G * g.ws, nit = (n - ws + step - 1) / step;
+    load(f0, j, n);
+    for (int it = nit >> 1; it > 0; it--) {
+      load(f1, j += step, n);
+      mac(f0);
+      load(f0, j += step, n);
+      mac(f1);
+    }
+    if (nit & 1) {
+      load(f1, j, n);  // (the count of outstanding loads that mac waits for)
+      mac(f0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int t = 0; t < CT; t++) red[(ws * 2 * CT + i * CT + t) * 64 + lane] = acc[i][t];
+  __syncthreads();
+  for (int f = ws; f < 2 * CT; f += g.ws) {
+    f32x4 v = red[f * 64 + lane];
+    for (int q = 1; q < g.ws; q++) v += red[(q * 2 * CT + f) * 64 + lane];
+    const int col = col0 + 16 * (f % CT) + (lane & 15);
+    if (col >= ncols) continue;
+    const int pl = col / g.nrhs, rh = col - pl * g.nrhs;
+    const int pz = pl % P, py = (pl / P) % P, px = pl / (P * P);
+    const int fx = 2 * px + ((s >> 2) & 1), fy = 2 * py + ((s >> 1) & 1), fz = 2 * pz + (s & 1);
+    const int A = g.levsta[l] + morton3(fx, fy, fz, l);
+    *reinterpret_cast<realx4u *>(g.L + ((size_t)rh * g.ncell + A) * 32 + 16 * (f / CT) + 4 * (lane >> 4)) = v;
+  }
+}
+#endif
+
 // ---------------------------------------------------------------- host side
 static void offset_table(std::vector<int4> &tab)
 {
@@ -1297,6 +1476,33 @@ static void real_shape(GridM2L *g)
   a.ws = std::min(g->nblocks >= 2048 ? 4 : g->nblocks >= 128 ? 8 : 16, real_max_waves(a.rt, a.ct));
 }
 
+// Split-BF16 on fewer columns of the deepest level than this runs
+// k_m2l_bf16_few, on more the source-stationary kernel, whose step parts then
+// fill the chip (us, 4096 columns 80 against 141; 8192 of depth 5 119 against
+// 104, of depth 4 106 against 103).
+constexpr long long kFewColumns = 8192;
+
+// Two tiles of 16 columns a block once they leave 128 blocks and more (us:
+// 37 tiles a class 22.9 against 27.5, 72 22.7 against 26.6, 23 20.1 against
+// 17.1, 8 13.1 against 10.5), with 8 offset slices, else 4.
+static void few_shape(GridM2L *g)
+{
+  GridArgs &a = g->args;
+  a.plane = ((g->nslots * a.nrhs * 16 + 4095) / 4096 * 4096 + 256) / 2;
+  a.gbytes = (int)(a.plane * 4 * 2);
+  long long t16 = 0;
+  for (int l = a.minlev; l <= a.maxlev; l++) t16 += ((1LL << (3 * (l - 1))) * a.nrhs + 15) / 16;
+  a.ct = t16 >= 32 ? 2 : 1;
+  a.ws = a.ct == 2 ? 8 : 4;
+  int groups = 0;
+  for (int l = a.minlev; l <= a.maxlev; l++) {
+    a.blk0[l] = groups;
+    groups += (int)(((1LL << (3 * (l - 1))) * a.nrhs + 16 * a.ct - 1) / (16 * a.ct));
+  }
+  a.blk0[a.maxlev + 1] = groups;
+  g->nblocks = 8 * groups;
+}
+
 int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const real *K, hipStream_t s,
                     int minlev, int variant, int variant_upper, int upper_split, const real *K_dev)
 {
@@ -1379,22 +1585,23 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
   // on different L2 channels (at a multiple of 4 KB they all share one)
   a.plane = ((slots * nrhs * kVW * sizeof(real) + 4095) / 4096 * 4096 + 256) / sizeof(real);
   int tpw = 1, cpb;
-  // variant 0 (automatic): source-stationary blocking (4 classes per wave)
-  // once the deepest level has 8192 columns (parents x vectors) or more (at
-  // depth 4 with 16 vectors: 0.177 ms against 0.228 ms for two class-stationary
-  // tiles per wave);
+  // variant 0 (automatic): split-BF16 takes the source-stationary blocking (4
+  // classes per wave) once the deepest level has kFewColumns columns (parents
+  // x vectors) or more, k_m2l_bf16_few below;
   // 1 / 4 / 5: source-stationary with 8 / 4 / 2 field classes per wave and
   // one 32-column tile, 6 / 7: 2 / 4 classes and two tiles per wave;
   // 2 / 3: class-stationary, one / two 32-column tiles per wave
   const long long deep = (long long)(1 << (3 * (maxlev - 1))) * nrhs;
   a.ss = 0;
   if (form == BBFMM_M2L_BF16X2) {
+    a.few = variant == 0 && deep < kFewColumns;
     a.ss = variant == 0 && deep >= 8 * 1024 ? 4 : ss_classes(variant);
+    if (a.few) a.ss = 0;
     a.ss_tpw = ss_tiles(variant);
     a.ss_pair = variant == 8;
   }
-  if (real_form) {
-    cpb = 1 << 30;  // blocks: real_shape
+  if (real_form || a.few) {
+    cpb = 1 << 30;  // blocks: real_shape, few_shape
   } else if (a.ss) {
     cpb = 4 * 32 * a.ss_tpw;  // 4 waves x 32 or 64 columns, one class group per block
   } else {
@@ -1428,6 +1635,7 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
   a.blk0[maxlev + 1] = nb;
   g->nblocks = nb;
   if (real_form) real_shape(g);
+  if (a.few) few_shape(g);
 
   std::vector<int4> tab;
   offset_table(tab);
@@ -1504,7 +1712,29 @@ int grid_m2l_create(GridM2L **out, int r, int maxlev, int nrhs, int form, const 
       }
     }
 #ifdef SINGLE
-    else if (form == BBFMM_M2L_BF16X2) {
+    else if (a.few) {
+      a.kbytes = (kNumOps + 1) * 4096;
+      float *up = nullptr;
+      if ((e = hipMalloc(&g->d_K, a.kbytes)) != hipSuccess) fail(e, "hipMalloc");
+      if (rc == BBFMM_OK && !K_dev) {
+        if ((e = hipMalloc((void **)&up, sizeof(float) * kNumOps * 1024)) != hipSuccess) fail(e, "hipMalloc");
+        else if ((e = hipMemcpyAsync(up, K, sizeof(float) * kNumOps * 1024, hipMemcpyHostToDevice, s)) != hipSuccess)
+          fail(e, "copy");
+      }
+      if (rc == BBFMM_OK) {
+        hipLaunchKernelGGL(k_few_layout, dim3((kNumOps + 1) * 4), dim3(256), 0, s, K_dev ? K_dev : up, (__bf16 *)g->d_K);
+        if ((e = hipGetLastError()) != hipSuccess) fail(e, "operator layout");
+      }
+      void **grids[2] = {&g->d_Mg0, &g->d_Mg1};
+      for (void **gp : grids) {
+        if (rc == BBFMM_OK && (e = hipMalloc(gp, a.gbytes)) != hipSuccess) fail(e, "hipMalloc");
+        if (rc == BBFMM_OK && (e = hipMemsetAsync(*gp, 0, a.gbytes, s)) != hipSuccess) fail(e, "memset");
+      }
+      if (up) {
+        (void)hipStreamSynchronize(s);
+        (void)hipFree(up);
+      }
+    } else if (form == BBFMM_M2L_BF16X2) {
       // [k][kstep][hi/lo][lane][8]: lane l holds row l%32, k = 16*kstep + 8*(l/32) + e
       // one extra all-zero operator (kZeroOp) after the 316
       std::vector<__bf16> Kb((size_t)(kNumOps + 1) * 2 * 2 * 64 * 8, (__bf16)0.0f);
@@ -1698,7 +1928,7 @@ static void launch_ss(const GridM2L *g, const GridArgs &a, int nblocks, hipStrea
 int grid_m2l_leaf_grids(const GridM2L *g, void **hi, void **lo, int *slot0)
 {
 #ifdef SINGLE
-  if (g && g->form == BBFMM_M2L_BF16X2 && g->nrhs == 16 && g->args.minlev <= g->args.maxlev) {
+  if (g && g->form == BBFMM_M2L_BF16X2 && !g->args.few && g->nrhs == 16 && g->args.minlev <= g->args.maxlev) {
     *hi = g->d_Mg0;
     *lo = g->d_Mg1;
     *slot0 = g->args.lvl_slot0[g->args.maxlev];
@@ -1728,6 +1958,16 @@ int grid_m2l_run(GridM2L *g, const real *M, real *L, int ncell, hipStream_t s, h
     return launch_real(a, g->nblocks, s);
 #ifdef SINGLE
   case BBFMM_M2L_BF16X2:
+    if (a.few) {
+      hipLaunchKernelGGL(k_few_scatter, dim3((unsigned)((cells * 4 + 255) / 256)), dim3(256), 0, s, a, M);
+      BB_HIP(hipGetLastError());
+      if (mid) BB_HIP(hipEventRecord(mid, s));
+      const size_t lds = (size_t)a.ws * 2 * a.ct * 64 * sizeof(f32x4);
+      if (a.ct == 1) hipLaunchKernelGGL(k_m2l_bf16_few<1>, dim3(g->nblocks), dim3(64 * a.ws), lds, s, a);
+      else hipLaunchKernelGGL(k_m2l_bf16_few<2>, dim3(g->nblocks), dim3(64 * a.ws), lds, s, a);
+      BB_HIP(hipGetLastError());
+      return BBFMM_OK;
+    }
     if (deep_in_grid) {  // the levels above the deepest only
       if (a.maxlev > a.minlev) {
         GridArgs u = a;

@@ -87,3 +87,22 @@ def test_values_stay_in_their_columns(cuda):
     ref = _m2l(B, "s", 4, r, depth, nrhs, K, M, cuda, 0, scheme=B.SCHEME_BA)
     assert np.array_equal(got[[0, 2]], clean[[0, 2]])
     assert np.array_equal(np.isfinite(got[1]), np.isfinite(ref[1]))
+
+
+@pytest.mark.parametrize("depth,nrhs", [(2, 1), (2, 16), (2, 130), (3, 1), (3, 3), (3, 16), (4, 1), (4, 5), (4, 15)])
+def test_split_bf16_few_columns(depth, nrhs, cuda):
+    """The split-BF16 kernel of few columns (k_m2l_bf16_few): one and two
+    column tiles a block, partial tiles, M and L at any alignment.  The bound
+    is that of the form, as everywhere (3e-5)."""
+    import bbfmmongpu_amd as B
+    r = 32
+    ncell = (8 ** (depth + 1) - 1) // 7
+    rng = np.random.default_rng(nrhs)
+    K = rng.standard_normal(316 * r * r, dtype=np.float32)
+    M = rng.standard_normal((nrhs, ncell, r), dtype=np.float32)
+    ref = _m2l(B, "d", 4, r, depth, nrhs, K, M, cuda, 0, scheme=B.SCHEME_BA)
+    got = _m2l(B, "s", 4, r, depth, nrhs, K, M, cuda, 1, scheme=B.SCHEME_IJ, form=B.FORM_BF16X2)
+    assert not got[:, :9].any()
+    err = (np.linalg.norm((got - ref)[:, 9:], axis=(1, 2)) / np.linalg.norm(ref[:, 9:], axis=(1, 2))).max()
+    print(f"depth={depth} nrhs={nrhs}: {err:.2e}", flush=True)
+    assert err < 3e-5
