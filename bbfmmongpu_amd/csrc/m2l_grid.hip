@@ -37,7 +37,9 @@
 #include "kernels.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace bb {
@@ -2029,83 +2031,53 @@ int grid_m2l_run(GridM2L *g, const real *M, real *L, int ncell, hipStream_t s, h
 // gathered columns.  The field cells of levels >= 2 are grouped by sibling
 // class s; for class s and its 189 offsets v (the dense-grid table order)
 // vsrc[F * 189 + j] names the source cell F + v, or the zero cell ncell when
-// that cell holds no points.  A block (4 waves x 32 columns, columns = (field
-// cell, vector) pairs of one class) multiplies K_v by the gathered source
-// columns for every v: the operator is shared by the whole block, as in the
-// dense-grid kernel.  M is copied per solve to [rhs][ncell + 1][r] (bf16 hi
-// and lo for the split form) with a zero last cell.
+// that cell holds no points.  M is copied per solve to one 128-byte line a
+// cell and vector, [rhs][ncell + 1] (bf16 hi and lo, or the 32 floats) with a
+// zero last cell; k_m2l_list_packed multiplies them.
+
+// A wave's units of k_m2l_list_packed, of 64 columns and of 32, and the first
+// entry of each.
+struct ListPart {
+  int unit[2], count[2];
+  long long entry[2];
+};
 
 struct ListArgs {
   int ncell, nrhs;
-  int cls_off[9];   // class c cells: cls_cells[cls_off[c] .. cls_off[c + 1])
-  int blk0[9];      // block count of class c: blk0[c + 1] - blk0[c]
-  // logical block -> 8 * (block within its class) + class: the classes are
-  // interleaved in proportion to their sizes, so that the blocks running at
-  // one time (and the contiguous range each XCD takes) cover one region of
-  // the forest for all 8 classes and share its source cells in L2
-  const int *blk_tab;
+  int cls_off[9];  // class c cells: cls_cells[cls_off[c] .. cls_off[c + 1])
   const int *cls_cells;
   const int *vsrc;  // [ncell * 189]
   const int4 *tab;  // [8][189] (operator, ...)
-  // per wave (4 per block): bit v of words 0..2 set when some column of the
-  // wave has a non-empty source at offset v
-  const unsigned long long *mask;  // [4 * blocks][4]
-  // one vector per cell (nrhs = 1): per wave, the source cells of its 32
-  // columns at each offset, so that one offset's indices are one 128-byte
-  // line (ncell for columns past the end); null otherwise (the columns of a
-  // wave then hold at most 16 cells, read from vsrc)
-  const int *vsw;  // [4 * blocks][189][32]
+  // blocks of at most cw cells x vb vectors, ws waves with their accumulators
+  // in ts LDS slots each; in launch order, the classes interleaved in proportion to their
+  // sizes, so that the blocks running at one time (and the contiguous range
+  // each XCD takes) cover one region of the forest for all 8 classes and
+  // share its source cells in L2
+  int nblk, vb, cw, ts, ws;
+  const int2 *blk;             // [nblk] first of cls_cells, cells
+  const ListPart *part;        // [nblk * ws]
+  const unsigned *unit;        // operator | entries << 16
+  const int *esrc;             // entries: source cell
+  const unsigned char *eslot;  // and target (cell within the block)
   const void *Ka;
-  const void *M0, *M1;
+  const void *M0;
   real *L;
   int kbytes;  // bytes of Ka
-  int mbytes;  // bytes of M0 (and M1) when below 2 GB (scalar-offset buffer loads), else 0
+  int mbytes;  // bytes of M0 when below 2 GB (32-bit buffer offsets), else 0
 };
 
 struct ListM2L {
-  int form = 0, nrhs = 1, ncell = 0, nblocks = 0;
+  int form = 0;
   int flat = 0;  // 1: pointer-form loads even on arrays below 2 GB
   ListArgs args{};
   int4 *d_tab = nullptr;
-  int *d_blk = nullptr;
-  unsigned long long *d_mask = nullptr;
-  int *d_vsw = nullptr;
-  void *d_K = nullptr, *d_M0 = nullptr, *d_M1 = nullptr;
+  int2 *d_blk = nullptr;
+  ListPart *d_part = nullptr;
+  unsigned *d_unit = nullptr;
+  int *d_esrc = nullptr;
+  unsigned char *d_eslot = nullptr;
+  void *d_K = nullptr, *d_M0 = nullptr;
 };
-
-// Columns of wave w of block b (in the list kernel's logical block order):
-// class s and the column range.  Shared by the kernel and its mask set-up.
-__device__ __forceinline__ int2 list_block(const ListArgs &g, int lb)
-{
-  const int code = g.blk_tab[lb];
-  return make_int2(code & 7, code >> 3);  // class, block within the class
-}
-
-// One wave per wave of the list kernel: the union over its valid columns of
-// the non-empty offsets (vsrc != ncell), as a 189-bit mask, and the wave's
-// column-contiguous copy of the source table.
-__global__ void __launch_bounds__(64) k_m2l_list_mask(ListArgs g, unsigned long long *mask, int *vsw)
-{
-  const int gw = blockIdx.x;  // 4 * logical block + wave
-  const int lb = gw >> 2, wave = gw & 3;
-  const int2 sb = list_block(g, lb);
-  const int s = sb.x, grp = sb.y;
-  const int ncols = (g.cls_off[s + 1] - g.cls_off[s]) * g.nrhs;
-  const int lane = threadIdx.x;
-  const int col = (grp * 4 + wave) * 32 + (lane & 31);
-  const bool valid = lane < 32 && col < ncols;
-  const int F = valid ? g.cls_cells[g.cls_off[s] + col / g.nrhs] : 0;
-  const int *vs = g.vsrc + (size_t)F * kOffsets;
-  unsigned long long m[3] = {0, 0, 0};
-  int *out = vsw ? vsw + (size_t)gw * kOffsets * 32 + lane : nullptr;
-  for (int v = 0; v < kOffsets; v++) {
-    const int S = valid ? vs[v] : g.ncell;
-    const bool any = __ballot(S != g.ncell) != 0;
-    if (any) m[v >> 6] |= 1ull << (v & 63);
-    if (out && lane < 32) out[v * 32] = S;
-  }
-  if (lane < 4) mask[(size_t)gw * 4 + lane] = lane < 3 ? m[lane] : 0ull;
-}
 
 template <int FORM>
 __global__ void __launch_bounds__(256) k_m2l_list_prep(ListArgs g, const real *__restrict__ M)
@@ -2117,7 +2089,7 @@ __global__ void __launch_bounds__(256) k_m2l_list_prep(ListArgs g, const real *_
   const long long cr = t >> 2;
   const int A = (int)(cr % g.ncell), rh = (int)(cr / g.ncell);
   const real *src = M + ((size_t)rh * g.ncell + A) * 32 + ch * 8;
-  const size_t dst = ((size_t)rh * (g.ncell + 1) + A) * 32 + ch * 8;
+  const size_t row = (size_t)rh * (g.ncell + 1) + A;  // one 128-byte line a cell and vector
   if (FORM == BBFMM_M2L_BF16X2) {
     bf16x8 hi, lo;
 #pragma unroll
@@ -2127,149 +2099,13 @@ __global__ void __launch_bounds__(256) k_m2l_list_prep(ListArgs g, const real *_
       hi[e] = h;
       lo[e] = (__bf16)(v - (float)h);
     }
-    *reinterpret_cast<bf16x8 *>((__bf16 *)g.M0 + dst) = hi;
-    *reinterpret_cast<bf16x8 *>((__bf16 *)g.M1 + dst) = lo;
+    __bf16 *d = (__bf16 *)g.M0 + row * 64 + ch * 8;  // hi, lo
+    *reinterpret_cast<bf16x8 *>(d) = hi;
+    *reinterpret_cast<bf16x8 *>(d + 32) = lo;
   } else {
-    float *d = (float *)g.M0 + dst;
+    float *d = (float *)g.M0 + row * 32 + ch * 8;
 #pragma unroll
     for (int e = 0; e < 8; e++) d[e] = (float)src[e];
-  }
-}
-
-template <int FORM>
-__global__ void __launch_bounds__(256) k_m2l_list_mfma(ListArgs g)
-{
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  // XCD-aware order: the launch is a multiple of 8 blocks and hardware block b
-  // runs on XCD b % 8, which takes a contiguous range of logical blocks lb
-  // (one region of the forest, all classes) so that neighbouring targets,
-  // which gather the same sources, share one L2.
-  const int nb = g.blk0[8];
-  const int b = blockIdx.x;
-  const int lb = (b & 7) * ((nb + 7) >> 3) + (b >> 3);
-  if (lb >= nb) return;
-  const int2 sb = list_block(g, lb);
-  const int s = sb.x, grp = sb.y;
-  const int ncols = (g.cls_off[s + 1] - g.cls_off[s]) * g.nrhs;
-  const int half = lane >> 5;
-  // columns past the end compute a copy of the class's first column and are not stored
-  const int col = (grp * 4 + wave) * 32 + (lane & 31);
-  const bool valid = col < ncols;
-  const int cc = valid ? col : 0;
-  const int F = g.cls_cells[g.cls_off[s] + cc / g.nrhs];
-  const int rh = cc % g.nrhs;
-  const int4 *tab = g.tab + s * kOffsets;
-  const size_t rbase = (size_t)rh * (g.ncell + 1);
-  const int gw = __builtin_amdgcn_readfirstlane(lb * 4 + wave);
-  // source of column (lane % 32) at offset v: the wave-major copy, or vsrc
-  const int *vsl = g.vsw ? g.vsw + (size_t)gw * kOffsets * 32 + (lane & 31) : g.vsrc + (size_t)F * kOffsets;
-  const int vst = g.vsw ? 32 : 1;
-  auto vs = [&](int v) { return vsl[v * vst]; };
-  f32x16 acc;
-#pragma unroll
-  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
-  // Only the offsets at which some column of the wave has a non-empty source
-  // are visited (the others would add K_v times the zero cell); they come in
-  // increasing order from the wave's 189-bit mask.  Software pipeline: the
-  // operator fragments and the gathered source column of the next offset are
-  // in flight while the MFMAs of the current one run, and the source index
-  // of the one after that a step earlier (two register stages, the loop
-  // unrolled by two so that no stage is copied).
-  struct Stage {
-    f32x4 a[4], b[4];  // BF16X2: a[0..3] = hi0, lo0, hi1, lo1 of K_v; b likewise of the source
-  };
-  auto load = [&](int v, int S, Stage &t) {
-    const int k = tab[v].x;
-    if (FORM == BBFMM_M2L_BF16X2) {
-      const f32x4 *Ka = (const f32x4 *)((const bf16x8 *)g.Ka + (size_t)k * 4 * 64 + lane);
-#pragma unroll
-      for (int q = 0; q < 4; q++) t.a[q] = Ka[q * 64];
-      const size_t o = (rbase + S) * 32 + half * 8;
-      t.b[0] = *(const f32x4 *)((const __bf16 *)g.M0 + o);
-      t.b[1] = *(const f32x4 *)((const __bf16 *)g.M1 + o);
-      t.b[2] = *(const f32x4 *)((const __bf16 *)g.M0 + o + 16);
-      t.b[3] = *(const f32x4 *)((const __bf16 *)g.M1 + o + 16);
-    } else {
-      const f32x4 *Ka = (const f32x4 *)g.Ka + ((size_t)k * 64 + lane) * 4;
-      const f32x4 *bp = (const f32x4 *)((const float *)g.M0 + (rbase + S) * 32 + half * 16);
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        t.a[q] = Ka[q];
-        t.b[q] = bp[q];
-      }
-    }
-  };
-  auto mma = [&](const Stage &t) {
-    if (FORM == BBFMM_M2L_BF16X2) {
-      typedef __attribute__((ext_vector_type(8))) __bf16 b8;
-      const b8 a0h = __builtin_bit_cast(b8, t.a[0]), a0l = __builtin_bit_cast(b8, t.a[1]);
-      const b8 a1h = __builtin_bit_cast(b8, t.a[2]), a1l = __builtin_bit_cast(b8, t.a[3]);
-      const b8 b0h = __builtin_bit_cast(b8, t.b[0]), b0l = __builtin_bit_cast(b8, t.b[1]);
-      const b8 b1h = __builtin_bit_cast(b8, t.b[2]), b1l = __builtin_bit_cast(b8, t.b[3]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0h, b0h, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0h, b0l, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0l, b0h, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1h, b1h, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1h, b1l, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1l, b1h, acc, 0, 0, 0);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-#pragma unroll
-        for (int w = 0; w < 4; w++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(t.a[q][w], t.b[q][w], acc, 0, 0, 0);
-    }
-  };
-  unsigned long long m0 = g.mask[(size_t)gw * 4], m1 = g.mask[(size_t)gw * 4 + 1], m2 = g.mask[(size_t)gw * 4 + 2];
-  // next visited offset, or -1 past the last (scalar selects, no branches)
-  auto pop = [&]() -> int {
-    const bool a0 = m0 != 0, a1 = m1 != 0, a2 = m2 != 0;
-    const int t0 = a0 ? __builtin_ctzll(m0) : 0, t1 = a1 ? __builtin_ctzll(m1) : 0,
-              t2 = a2 ? __builtin_ctzll(m2) : 0;
-    const int v = a0 ? t0 : a1 ? 64 + t1 : a2 ? 128 + t2 : -1;
-    m0 = a0 ? m0 & (m0 - 1) : m0;
-    m1 = !a0 && a1 ? m1 & (m1 - 1) : m1;
-    m2 = !a0 && !a1 ? m2 & (m2 - 1) : m2;
-    return v;
-  };
-  // Loads are unconditional (offset 0 stands in past the last) so that no
-  // branch separates a load from the MFMAs that wait for it; the source
-  // indices are read an iteration (two offsets) before their columns.
-  Stage X, Y;
-  int vy, vz, vw;
-  const int vx = pop();
-  vy = pop();
-  vz = pop();
-  vw = pop();
-  if (vx >= 0) {
-    load(vx, vs(vx), X);
-    load(max(vy, 0), vs(max(vy, 0)), Y);
-    int Sz = vs(max(vz, 0)), Sw = vs(max(vw, 0));
-    // X holds an offset, Y the next one (vy, when vy >= 0); vz and vw follow,
-    // with sources Sz and Sw
-    for (;;) {
-      const int vu = pop(), vt = pop();
-      const int Su = vs(max(vu, 0)), St = vs(max(vt, 0));
-      __builtin_amdgcn_sched_barrier(0);
-      mma(X);
-      load(max(vz, 0), Sz, X);
-      if (vy < 0) break;
-      mma(Y);
-      load(max(vw, 0), Sw, Y);
-      if (vz < 0) break;
-      vy = vw;
-      vz = vu;
-      vw = vt;
-      Sz = Su;
-      Sw = St;
-    }
-  }
-  if (!valid) return;
-  float *Lp = (float *)g.L + ((size_t)rh * g.ncell + F) * 32 + 4 * half;
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    f32x4 o = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-    *reinterpret_cast<f32x4 *>(Lp + 8 * q) = o;
   }
 }
 
@@ -2308,137 +2144,484 @@ int class_slot(int s, int vx, int vy, int vz)
   return slot[s * 343 + 49 * (vx + 3) + 7 * (vy + 3) + (vz + 3)];
 }
 
-// Split-BF16 list M2L with the operator shared by the block: the 4 waves of
-// a block visit the union of their offset masks in step, and each offset's
-// operator fragments (4 KB) are loaded once per block (one 1 KB fragment per
-// wave, through registers into LDS, double-buffered) instead of once per
-// wave; the vector-memory pipe, which the per-wave kernel saturates with
-// 8 KB per offset and wave, then moves 5 KB.  Per step: the next offset's
-// fragment and source column are loaded while the current offset's six
-// products run; one barrier per step.  Same columns, order of products and
-// results as k_m2l_list_mfma<BBFMM_M2L_BF16X2> (the extra offsets a wave
-// visits add K_v times its zero sources).
-template <bool BUF>
-__global__ void __launch_bounds__(256) k_m2l_list_lds(ListArgs g)
+typedef __attribute__((ext_vector_type(4))) int i32x4;
+
+// Entries of a unit of R columns of k_m2l_list_packed: whole cells of vb vectors.
+template <int R>
+__host__ __device__ constexpr int unit_cells(int vb)
 {
-  __shared__ bf16x8 sK[2][4][64];  // [buffer][fragment: k-step x hi/lo][lane]
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int nb = g.blk0[8];
-  const int b = blockIdx.x;
-  const int lb = (b & 7) * ((nb + 7) >> 3) + (b >> 3);
-  if (lb >= nb) return;  // whole block
-  const int2 sb = list_block(g, lb);
-  const int s = sb.x, grp = sb.y;
-  const int ncols = (g.cls_off[s + 1] - g.cls_off[s]) * g.nrhs;
-  const int half = lane >> 5;
-  const int col = (grp * 4 + wave) * 32 + (lane & 31);
-  const bool valid = col < ncols;
-  const int cc = valid ? col : 0;
-  const int F = g.cls_cells[g.cls_off[s] + cc / g.nrhs];
-  const int rh = cc % g.nrhs;
-  const int4 *tab = g.tab + s * kOffsets;
-  const size_t rbase = (size_t)rh * (g.ncell + 1);
-  const int gw = __builtin_amdgcn_readfirstlane(lb * 4 + wave);
-  // source of column (lane % 32) at offset v: the wave-major copy, or vsrc
-  const int *vsl = g.vsw ? g.vsw + (size_t)gw * kOffsets * 32 + (lane & 31) : g.vsrc + (size_t)F * kOffsets;
-  const int vst = g.vsw ? 32 : 1;
-  auto vs = [&](int v) { return vsl[v * vst]; };
-  // the block's union of the 4 waves' masks
-  const unsigned long long *mk = g.mask + (size_t)lb * 16;
-  unsigned long long m0 = mk[0] | mk[4] | mk[8] | mk[12];
-  unsigned long long m1 = mk[1] | mk[5] | mk[9] | mk[13];
-  unsigned long long m2 = mk[2] | mk[6] | mk[10] | mk[14];
-  auto pop = [&]() -> int {
-    const bool a0 = m0 != 0, a1 = m1 != 0, a2 = m2 != 0;
-    const int t0 = a0 ? __builtin_ctzll(m0) : 0, t1 = a1 ? __builtin_ctzll(m1) : 0,
-              t2 = a2 ? __builtin_ctzll(m2) : 0;
-    const int v = a0 ? t0 : a1 ? 64 + t1 : a2 ? 128 + t2 : -1;
-    m0 = a0 ? m0 & (m0 - 1) : m0;
-    m1 = !a0 && a1 ? m1 & (m1 - 1) : m1;
-    m2 = !a0 && !a1 ? m2 & (m2 - 1) : m2;
-    return v;
-  };
-  // this wave's fragment of offset v's operator, and a column's source.
-  // BUF: buffer loads, the operator's index a scalar offset over a fixed
-  // per-lane part, the source's offset one 32-bit lane value (grids below
-  // 2 GB), so that no 64-bit address arithmetic goes into a step
-  const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void *)g.Ka, 0, g.kbytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rM0 = __builtin_amdgcn_make_buffer_rsrc((void *)g.M0, 0, g.mbytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rM1 = __builtin_amdgcn_make_buffer_rsrc((void *)g.M1, 0, g.mbytes, 0x00020000);
-  auto load_k = [&](int v) {
-    const int k = tab[v].x;
-    if (BUF)
-      return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rK, (wave * 64 + lane) * 16, k * 4096, 0));
-    return *((const f32x4 *)((const bf16x8 *)g.Ka + ((size_t)k * 4 + wave) * 64 + lane));
-  };
-  auto load_b = [&](int S, f32x4 *t) {
-    if (BUF) {
-      const int o = (((int)rbase + S) * 32 + half * 8) * 2;
-      t[0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rM0, o, 0, 0));
-      t[1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rM1, o, 0, 0));
-      t[2] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rM0, o + 32, 0, 0));
-      t[3] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rM1, o + 32, 0, 0));
-      return;
-    }
-    const size_t o = (rbase + S) * 32 + half * 8;
-    t[0] = *(const f32x4 *)((const __bf16 *)g.M0 + o);
-    t[1] = *(const f32x4 *)((const __bf16 *)g.M1 + o);
-    t[2] = *(const f32x4 *)((const __bf16 *)g.M0 + o + 16);
-    t[3] = *(const f32x4 *)((const __bf16 *)g.M1 + o + 16);
-  };
-  typedef __attribute__((ext_vector_type(8))) __bf16 b8;
-  f32x16 acc;
+  return R / vb;
+}
+
+// What a block of k_m2l_list_packed multiplies: units of 64 columns and of 32
+// (kind 0, 1), and their entries.
+struct ListCount {
+  int unit[2], entry[2];
+};
+
+// The units and entries of each block of k_m2l_list_packed (FILL: written;
+// else counted).  An entry is a (target, source) pair of non-empty cells; a
+// unit holds entries of one offset, the last of an offset those that are left.
+// base: first unit and entry of the block (kind 0, then kind 1).  The cells'
+// rows of vsrc are read into LDS whole (1.65M cells: 0.5 ms to count, 1.7 ms
+// to write; with a wave a block and a lane a cell, 10.9 ms together).
+template <bool FILL>
+__global__ void __launch_bounds__(1024) k_m2l_list_pack(ListArgs g, const int *__restrict__ cls, ListCount *cnt,
+                                                       const longlong2 *__restrict__ base, unsigned *unit, int *esrc,
+                                                       unsigned char *eslot, ListPart *part)
+{
+  extern __shared__ int rows[];  // [cells][189]
+  __shared__ int cells[128];
+  __shared__ ListCount sum[256];  // inclusive over the offsets
+  const int w = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int2 d = g.blk[w];
+  const int4 *tab = g.tab + cls[w] * kOffsets;
+  const int e64 = unit_cells<64>(g.vb), e32 = unit_cells<32>(g.vb);
+  if (tid < d.y) cells[tid] = g.cls_cells[d.x + tid];
+  __syncthreads();
+  for (int i0 = tid; i0 < d.y * kOffsets; i0 += 8 * 1024) {
+    int S[8];
 #pragma unroll
-  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
-  int v = pop();
-  if (v >= 0) {  // uniform over the block
-    f32x4 bc[4];
-    {
-      const f32x4 kf = load_k(v);
-      load_b(vs(v), bc);
-      *reinterpret_cast<f32x4 *>(&sK[0][wave][lane]) = kf;
+    for (int k = 0; k < 8; k++) {
+      const int i = min(i0 + k * 1024, d.y * kOffsets - 1), j = i / kOffsets;
+      S[k] = g.vsrc[(size_t)cells[j] * kOffsets + (i - j * kOffsets)];
     }
-    int vn = pop();
-    int Sn = vs(max(vn, 0));
-    __syncthreads();
-    for (int buf = 0;; buf ^= 1) {
-      const b8 a0h = __builtin_bit_cast(b8, sK[buf][0][lane]), a0l = __builtin_bit_cast(b8, sK[buf][1][lane]);
-      const b8 a1h = __builtin_bit_cast(b8, sK[buf][2][lane]), a1l = __builtin_bit_cast(b8, sK[buf][3][lane]);
-      // next offset (offset 0 stands in past the last): operator fragment and
-      // source column, issued before this offset's products (kept there)
-      const f32x4 kn = load_k(max(vn, 0));
-      f32x4 bn[4];
-      load_b(Sn, bn);
-      const int vnn = pop();
-      const int Snn = vs(max(vnn, 0));
-      __builtin_amdgcn_sched_barrier(0);
-      const b8 b0h = __builtin_bit_cast(b8, bc[0]), b0l = __builtin_bit_cast(b8, bc[1]);
-      const b8 b1h = __builtin_bit_cast(b8, bc[2]), b1l = __builtin_bit_cast(b8, bc[3]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0h, b0h, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0h, b0l, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0l, b0h, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1h, b1h, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1h, b1l, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1l, b1h, acc, 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (vn < 0) break;  // uniform over the block
-      *reinterpret_cast<f32x4 *>(&sK[buf ^ 1][wave][lane]) = kn;
-      __syncthreads();
 #pragma unroll
-      for (int q = 0; q < 4; q++) bc[q] = bn[q];
-      vn = vnn;
-      Sn = Snn;
-    }
+    for (int k = 0; k < 8; k++)
+      if (i0 + k * 1024 < d.y * kOffsets) rows[i0 + k * 1024] = S[k];
   }
-  if (!valid) return;
-  float *Lp = (float *)g.L + ((size_t)rh * g.ncell + F) * 32 + 4 * half;
-#pragma unroll
-  for (int q = 0; q < 4; q++) {
-    f32x4 o = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-    *reinterpret_cast<f32x4 *>(Lp + 8 * q) = o;
+  __syncthreads();
+  // an offset of n entries: u0 units of 64 columns with the first m, then u1
+  // (at most one) of 32 with the rest
+  int n = 0;
+  if (tid < kOffsets)
+    for (int j = 0; j < d.y; j++) n += rows[j * kOffsets + tid] != g.ncell;
+  const int rem = n % e64;
+  const int u0 = n / e64 + (rem > e32 ? 1 : 0), u1 = rem > 0 && rem <= e32 ? 1 : 0;
+  const int m = u1 ? n - rem : n;
+  ListCount at{{u0, u1}, {m, n - m}};
+  for (int k = 1; k < 256; k <<= 1) {
+    if (tid < 256) sum[tid] = at;
+    __syncthreads();
+    if (tid >= k && tid < 256) {
+      const ListCount o = sum[tid - k];
+      for (int i = 0; i < 2; i++) {
+        at.unit[i] += o.unit[i];
+        at.entry[i] += o.entry[i];
+      }
+    }
+    __syncthreads();
+  }
+  if (!FILL) {
+    if (tid == kOffsets - 1) cnt[w] = at;
+    return;
+  }
+  if (tid < 256) sum[tid] = at;
+  __syncthreads();
+  const ListCount tot = cnt[w];
+  const longlong2 bs = base[w];
+  const long long eb = bs.y + tot.entry[0];  // entries of kind 1
+  if (tid < kOffsets) {
+    const unsigned op = (unsigned)tab[tid].x;
+    for (int i = 0; i < u0; i++)
+      unit[bs.x + at.unit[0] - u0 + i] = op | (unsigned)min(e64, m - i * e64) << 16;
+    if (u1) unit[bs.x + tot.unit[0] + at.unit[1] - 1] = op | (unsigned)rem << 16;
+  }
+  if (tid < g.ws) {
+    ListPart p;
+    for (int k = 0; k < 2; k++) {
+      const int first = (int)((long long)tot.unit[k] * tid / g.ws);
+      p.unit[k] = (int)bs.x + (k ? tot.unit[0] : 0) + first;
+      p.count[k] = (int)((long long)tot.unit[k] * (tid + 1) / g.ws) - first;
+      int v = 0;  // the offset that holds unit `first`
+      while (v < kOffsets - 1 && sum[v].unit[k] <= first) v++;
+      const int u = v ? sum[v - 1].unit[k] : 0, e = v ? sum[v - 1].entry[k] : 0;
+      p.entry[k] = (k ? eb : bs.y) + e + (first - u) * (k ? 1 : e64);
+    }
+    part[w * g.ws + tid] = p;
+  }
+  const unsigned long long below = (1ull << lane) - 1;
+  for (int v = tid >> 6; v < kOffsets; v += 16) {
+    ListCount o{};
+    if (v) o = sum[v - 1];
+    const int mv = sum[v].entry[0] - o.entry[0];
+    int first = 0;
+    for (int j0 = 0; j0 < d.y; j0 += 64) {
+      const int j = j0 + lane;
+      const int S = j < d.y ? rows[j * kOffsets + v] : g.ncell;
+      const unsigned long long mask = __ballot(S != g.ncell);
+      const int at_v = first + __popcll(mask & below);
+      if (S != g.ncell) {
+        const long long k = at_v < mv ? bs.y + o.entry[0] + at_v : eb + o.entry[1] + at_v - mv;
+        esrc[k] = S;
+        eslot[k] = (unsigned char)j;
+      }
+      first += __popcll(mask);
+    }
   }
 }
+
+__device__ __forceinline__ int quad_xor(int x, int p)
+{
+  return p == 1   ? __builtin_amdgcn_mov_dpp(x, 0xb1, 0xf, 0xf, false)
+         : p == 2 ? __builtin_amdgcn_mov_dpp(x, 0x4e, 0xf, 0xf, false)
+                  : __builtin_amdgcn_mov_dpp(x, 0x1b, 0xf, 0xf, false);
+}
+// exchange the odd rows of 16 lanes of x with the even rows of y; the upper
+// half of x with the lower half of y
+__device__ __forceinline__ void row_swap(unsigned &x, unsigned &y)
+{
+  const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  x = r[0];
+  y = r[1];
+}
+__device__ __forceinline__ void half_swap(unsigned &x, unsigned &y)
+{
+  const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+  x = r[0];
+  y = r[1];
+}
+
+// 64 lines of 64 bytes, v[j] of lane 4 Q + i holding piece i ^ j of line
+// 4 Q + j: to v[t] of lane 16 q + c holding piece q of line 16 t + c.
+__device__ __forceinline__ void lines_to_columns(i32x4 (&v)[4], bool b0, bool b1)
+{
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int x0 = v[0][e], x1 = v[1][e], x2 = v[2][e], x3 = v[3][e];
+    const int y0 = b0 ? x1 : x0, y1 = b0 ? x0 : x1, y2 = b0 ? x3 : x2, y3 = b0 ? x2 : x3;
+    // piece p of the lane's own line: lane i ^ p holds it in its register i
+    unsigned u[4];
+    u[0] = b1 ? y2 : y0;
+    u[1] = quad_xor(b1 ? y3 : y1, 1);
+    u[2] = quad_xor(b1 ? y0 : y2, 2);
+    u[3] = quad_xor(b1 ? y1 : y3, 3);
+    half_swap(u[0], u[2]);
+    half_swap(u[1], u[3]);
+    row_swap(u[0], u[1]);
+    row_swap(u[2], u[3]);
+#pragma unroll
+    for (int t = 0; t < 4; t++) v[t][e] = u[t];
+  }
+}
+
+// List M2L over the non-empty (target, source) pairs only.  In a sparse tree
+// a cell has a source at 67 of the 189 offsets (a batch of Plummer spheres and
+// surfaces, 1.65M cells), while 32 neighbouring cells have some source at 165
+// of them: columns that stay with their cells, accumulated in registers,
+// multiply 2.5 times as many as there are.  Here the accumulators of a
+// block's 127 columns lie in LDS, one set a wave, and per offset only the
+// cells with a source are packed into units of 64 or 32 columns, built once a
+// plan: the unit's accumulators are read, multiplied into and written back.
+// The block's units are split over its 4 waves (summed at the end in wave
+// order), so that the cells in flight on an XCD are few enough for their
+// sources to stay in its L2 (misses 32M lines -> 8.6M).
+//
+// Bound: the cache's return path (TD busy 84%, TA 73%; LDS about 70%).  A
+// load whose adjacent lanes take 16 bytes each of different lines costs an
+// access a lane, 64; so the 4 lanes of a quad take the 64 bytes of one line
+// (16 accesses), and the columns are put where the products want them in
+// registers (lines_to_columns; through ds_bpermute for 32 columns).
+// Measured, split BF16, against 32 columns a wave with block-shared
+// operators: 64 instances of 4096 to 131072 points 2970 -> 1840 us, 16 up to
+// 32768 371 -> 204, 16 up to 65536 with 2 vectors 1553 -> 718, 8 up to 16384
+// 120 -> 80.
+template <int FORM, bool BUF>
+__global__ void __launch_bounds__(256) k_m2l_list_packed(ListArgs g)
+{
+  extern __shared__ f32x4 accs[];  // [wave][row quad 8][slot ts]
+  typedef __attribute__((ext_vector_type(8))) __bf16 b8;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.x;
+  const int lb = (b & 7) * ((g.nblk + 7) >> 3) + (b >> 3);
+  if (lb >= g.nblk) return;  // whole block
+  const int ts = g.ts, vb = g.vb;
+  const int2 d = g.blk[lb];
+  const ListPart part = g.part[lb * g.ws + wave];
+  f32x4 *acc = accs + wave * 8 * ts;
+  for (int i = lane; i < 8 * ts; i += 64) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  __syncthreads();
+  const int rh0 = blockIdx.y * vb, nv = min(vb, g.nrhs - rh0);
+  const int dummy = ts - 1;  // columns past a unit's last
+  const int c = lane & 15, q = lane >> 4;
+  const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc((void *)g.Ka, 0, g.kbytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rM = __builtin_amdgcn_make_buffer_rsrc((void *)g.M0, 0, g.mbytes, 0x00020000);
+  // two tiles of 16 columns: accumulator columns sl, sources b0, b1
+  auto products = [&](const f32x4 *k, const i32x4 *b0, const i32x4 *b1, const int *sl) {
+    f32x4 C[2][2];
+    int a[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      a[i] = q * ts + sl[i];
+      C[i][0] = acc[a[i]];
+      C[i][1] = acc[a[i] + 4 * ts];
+    }
+    if (FORM == BBFMM_M2L_BF16X2) {
+#pragma unroll
+      for (int p = 0; p < 3; p++)  // hi x hi, hi x lo, lo x hi
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int m = 0; m < 2; m++)
+            C[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, k[2 * m + (p == 2)]),
+                                                              __builtin_bit_cast(b8, (p == 1 ? b1 : b0)[i]), C[i][m],
+                                                              0, 0, 0);
+    } else {
+#pragma unroll
+      for (int p = 0; p < 8; p++)  // step p: k = 4 q + p % 4 (+ 16)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int m = 0; m < 2; m++)
+            C[i][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[2 * m + (p >> 2)][p & 3],
+                                                           __builtin_bit_cast(f32x4, (p < 4 ? b0 : b1)[i])[p & 3],
+                                                           C[i][m], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      acc[a[i]] = C[i][0];
+      acc[a[i] + 4 * ts] = C[i][1];
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  // the units of R columns
+  auto phase = [&](auto rc) {
+    constexpr int R = decltype(rc)::value, kind = R == 64 ? 0 : 1;
+    constexpr int NB = R / 16, NE = R == 64 ? 1 : 2;
+    struct Entry {
+      int src[NE], slot[NE];
+    };
+    struct Buf {
+      f32x4 k[4];
+      i32x4 b0[NB], b1[NB];  // the two 64-byte halves of the lines
+      int slot[NE];
+    };
+    const int nu = part.count[kind];
+    if (nu <= 0) return;
+    const unsigned *unit = g.unit + part.unit[kind];
+    const int *esrc = g.esrc + part.entry[kind];
+    const unsigned char *eslot = g.eslot + part.entry[kind];
+    // R = 64: a lane reads the line and slot of column `lane`.  R = 32: the
+    // lines of columns lane / 4 (+ 16), which its quad loads, and the slots
+    // of columns lane % 16 (+ 16), which it multiplies.
+    int es[NE], rs[NE], ed[NE], rd[NE];  // entry and vector of the line, of the slot
+    bool ls[NE], ld[NE];
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+      const int cs = R == 64 ? lane : 16 * i + (lane >> 2), cd = R == 64 ? lane : 16 * i + c;
+      es[i] = cs / vb;
+      rs[i] = cs - es[i] * vb;
+      ed[i] = cd / vb;
+      rd[i] = cd - ed[i] * vb;
+      ls[i] = es[i] < unit_cells<R>(vb) && rs[i] < nv;
+      ld[i] = ed[i] < unit_cells<R>(vb) && rd[i] < nv;
+      rs[i] = (rh0 + rs[i]) * (g.ncell + 1);
+    }
+    auto word = [&](int i) { return i < nu ? unit[i] : 0u; };
+    auto entries = [&](int start) {
+      Entry e;
+#pragma unroll
+      for (int i = 0; i < NE; i++) {
+        e.src[i] = esrc[start + es[i]];
+        e.slot[i] = eslot[start + ed[i]];
+      }
+      return e;
+    };
+    auto load = [&](unsigned u, const Entry &e, Buf &t) {
+      const int n = (int)(u >> 16), k = (int)(u & 0xffff);
+      int row[NE];
+#pragma unroll
+      for (int i = 0; i < NE; i++) {
+        row[i] = ls[i] && es[i] < n ? rs[i] + e.src[i] : g.ncell;
+        t.slot[i] = ld[i] && ed[i] < n ? e.slot[i] * vb + rd[i] : dummy;
+      }
+      // load j: the 4 lanes of a quad share a line
+      int rj[4];
+      if (R == 64) {
+        rj[0] = __builtin_amdgcn_mov_dpp(row[0], 0x00, 0xf, 0xf, false);
+        rj[1] = __builtin_amdgcn_mov_dpp(row[0], 0x55, 0xf, 0xf, false);
+        rj[2] = __builtin_amdgcn_mov_dpp(row[0], 0xaa, 0xf, 0xf, false);
+        rj[3] = __builtin_amdgcn_mov_dpp(row[0], 0xff, 0xf, 0xf, false);
+      } else {
+        rj[0] = row[0];
+        rj[1] = row[NE - 1];
+      }
+#pragma unroll
+      for (int j = 0; j < NB; j++) {
+        const int piece = R == 64 ? (lane & 3) ^ j : lane & 3;
+        if (BUF) {
+          const int o = rj[j] * 128 + piece * 16;
+          t.b0[j] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rM, o, 0, 0));
+          t.b1[j] = __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rM, o + 64, 0, 0));
+        } else {
+          const char *o = (const char *)g.M0 + (size_t)rj[j] * 128 + piece * 16;
+          t.b0[j] = *(const i32x4 *)o;
+          t.b1[j] = *(const i32x4 *)(o + 64);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        t.k[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rK, lane * 16 + i * 1024, k * 4096, 0));
+    };
+    auto run = [&](Buf &t) {
+      if constexpr (R == 64) {
+        lines_to_columns(t.b0, lane & 1, lane & 2);
+        lines_to_columns(t.b1, lane & 1, lane & 2);
+        unsigned sl[4];
+        sl[0] = sl[2] = t.slot[0];
+        half_swap(sl[0], sl[2]);
+        sl[1] = sl[0];
+        sl[3] = sl[2];
+        row_swap(sl[0], sl[1]);
+        row_swap(sl[2], sl[3]);
+        products(t.k, t.b0, t.b1, (const int *)sl);
+        products(t.k, t.b0 + 2, t.b1 + 2, (const int *)sl + 2);
+      } else {
+        // line 16 j + Q, piece i in lane 4 Q + i: to lane 16 i + Q
+        const int from = 4 * (4 * c + q);
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const int x = t.b0[j][e], y = t.b1[j][e];
+            t.b0[j][e] = __builtin_amdgcn_ds_bpermute(from, x);
+            t.b1[j][e] = __builtin_amdgcn_ds_bpermute(from, y);
+          }
+        products(t.k, t.b0, t.b1, t.slot);
+      }
+    };
+    Buf X, Y;
+    unsigned u0 = word(0), u1 = word(1), u2 = word(2);
+    int start = 0;
+    Entry e0 = entries(0);
+    start += u0 >> 16;
+    Entry e1 = entries(start);
+    start += u1 >> 16;
+    load(u0, e0, X);
+    for (int i = 0;;) {
+      // entries of unit i + 2, operator and sources of i + 1, products of i
+      const Entry e2 = entries(start);
+      start += u2 >> 16;
+      load(u1, e1, Y);
+      const unsigned u3 = word(i + 3);
+      __builtin_amdgcn_sched_barrier(0);
+      run(X);
+      __builtin_amdgcn_sched_barrier(0);
+      if (++i >= nu) break;
+      e1 = entries(start);
+      start += u3 >> 16;
+      load(u2, e2, X);
+      const unsigned u4 = word(i + 3);
+      __builtin_amdgcn_sched_barrier(0);
+      run(Y);
+      __builtin_amdgcn_sched_barrier(0);
+      if (++i >= nu) break;
+      u0 = u2;
+      u1 = u3;
+      u2 = u4;
+    }
+  };
+  phase(std::integral_constant<int, 64>());
+  phase(std::integral_constant<int, 32>());
+  __syncthreads();
+  // columns of the block: 8 lanes a column
+  for (int i = threadIdx.x; i < d.y * vb * 8; i += blockDim.x) {
+    const int col = i >> 3, p = i & 7;
+    const int cell = col / vb, rh = rh0 + col - cell * vb;
+    f32x4 v = accs[p * ts + col];
+    for (int w = 1; w < g.ws; w++) v += accs[(8 * w + p) * ts + col];
+    if (rh < g.nrhs)
+      *(f32x4 *)((float *)g.L + ((size_t)rh * g.ncell + g.cls_cells[d.x + cell]) * 32 + 4 * p) = v;
+  }
+}
+
+#ifdef SINGLE
+// The blocks of k_m2l_list_packed, their units and entries.
+static int pack_lists(ListM2L *g, hipStream_t s)
+{
+  ListArgs &a = g->args;
+  const int nv = (a.nrhs + 15) / 16;
+  a.vb = (a.nrhs + nv - 1) / nv;
+  // 128 slots and 4 waves: 64 KB of LDS, 2 blocks a CU.  64 slots leave the
+  // units 40% emptier (batch of 1.65M cells 2391 us against 2050), 96 the same
+  // time; 1 wave a block 2215, and 222 against 92 where 8 small instances
+  // give too few blocks; 8 waves leave each too few units (2896)
+  a.ts = 128;
+  a.ws = 4;
+  a.cw = (a.ts - 1) / a.vb;
+  // the classes' blocks interleaved in proportion to their sizes
+  std::vector<std::pair<double, int2>> order;
+  for (int c = 0; c < 8; c++) {
+    const int n = a.cls_off[c + 1] - a.cls_off[c], nb = (n + a.cw - 1) / a.cw;
+    for (int k = 0; k < nb; k++) order.push_back({(k + 0.5) / nb, make_int2(c, a.cls_off[c] + k * a.cw)});
+  }
+  std::stable_sort(order.begin(), order.end(), [](const auto &x, const auto &y) { return x.first < y.first; });
+  const int nb = a.nblk = (int)order.size();
+  if (nb == 0) return BBFMM_OK;
+  std::vector<int2> blk(nb);
+  std::vector<int> cls(nb);
+  for (int w = 0; w < nb; w++) {
+    const int2 o = order[w].second;
+    cls[w] = o.x;
+    blk[w] = make_int2(o.y, std::min(a.cw, a.cls_off[o.x + 1] - o.y));
+  }
+  int *d_cls = nullptr;
+  ListCount *d_cnt = nullptr;
+  longlong2 *d_base = nullptr;
+  std::vector<ListCount> cnt(nb);
+  std::vector<longlong2> base(nb);
+  const size_t rows = sizeof(int) * kOffsets * std::min(a.cw, a.cls_off[8]);
+  const char *what = "hipMalloc";
+  auto set_up = [&]() -> hipError_t {
+    hipError_t e;
+    if ((e = hipMalloc(&d_cls, sizeof(int) * nb)) != hipSuccess) return e;
+    if ((e = hipMalloc(&d_cnt, sizeof(ListCount) * nb)) != hipSuccess) return e;
+    if ((e = hipMalloc(&d_base, sizeof(longlong2) * nb)) != hipSuccess) return e;
+    if ((e = hipMalloc(&g->d_blk, sizeof(int2) * nb)) != hipSuccess) return e;
+    if ((e = hipMalloc(&g->d_part, sizeof(ListPart) * nb * a.ws)) != hipSuccess) return e;
+    a.blk = g->d_blk;
+    a.part = g->d_part;
+    what = "list set-up";
+    if ((e = hipMemcpyAsync(d_cls, cls.data(), sizeof(int) * nb, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+    if ((e = hipMemcpyAsync(g->d_blk, blk.data(), sizeof(int2) * nb, hipMemcpyHostToDevice, s)) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_m2l_list_pack<false>, dim3(nb), dim3(1024), rows, s, a, d_cls, d_cnt, d_base, nullptr, nullptr,
+                       nullptr, nullptr);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if ((e = hipMemcpyAsync(cnt.data(), d_cnt, sizeof(ListCount) * nb, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+    if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
+    long long nu = 0, ne = 0;
+    for (int w = 0; w < nb; w++) {
+      base[w] = make_longlong2(nu, ne);
+      nu += cnt[w].unit[0] + cnt[w].unit[1];
+      ne += (long long)cnt[w].entry[0] + cnt[w].entry[1];
+    }
+    what = "list of more than 2^31 units";
+    if (nu > INT_MAX) return hipErrorInvalidValue;
+    what = "hipMalloc";
+    if ((e = hipMalloc(&g->d_unit, sizeof(unsigned) * (nu + 1))) != hipSuccess) return e;
+    // a unit's entries are read as if it were full, two units ahead
+    const size_t ahead = 256;
+    if ((e = hipMalloc(&g->d_esrc, sizeof(int) * (ne + ahead))) != hipSuccess) return e;
+    if ((e = hipMalloc(&g->d_eslot, (size_t)ne + ahead)) != hipSuccess) return e;
+    what = "list set-up";
+    if ((e = hipMemcpyAsync(d_base, base.data(), sizeof(longlong2) * nb, hipMemcpyHostToDevice, s)) != hipSuccess)
+      return e;
+    hipLaunchKernelGGL(k_m2l_list_pack<true>, dim3(nb), dim3(1024), rows, s, a, d_cls, d_cnt, d_base, g->d_unit, g->d_esrc,
+                       g->d_eslot, g->d_part);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    return hipStreamSynchronize(s);
+  };
+  const hipError_t rc = set_up();
+  if (d_cls) (void)hipFree(d_cls);
+  if (d_cnt) (void)hipFree(d_cnt);
+  if (d_base) (void)hipFree(d_base);
+  if (rc != hipSuccess) return set_error(BBFMM_E_HIP, "list M2L: %s: %s", what, hipGetErrorString(rc));
+  a.unit = g->d_unit;
+  a.esrc = g->d_esrc;
+  a.eslot = g->d_eslot;
+  return BBFMM_OK;
+}
+#endif
 
 int list_m2l_create(ListM2L **out, int r, int nrhs, int form, const real *K, int ncell, const int *cls_off,
                     const int *d_cls_cells, const int *d_vsrc, hipStream_t s)
@@ -2453,33 +2636,12 @@ int list_m2l_create(ListM2L **out, int r, int nrhs, int form, const real *K, int
     return set_error(BBFMM_E_ARG, "the list MFMA M2L runs the split-BF16 or FP32 MFMA form");
   ListM2L *g = new ListM2L();
   g->form = form;
-  g->nrhs = nrhs;
-  g->ncell = ncell;
   ListArgs &a = g->args;
   a.ncell = ncell;
   a.nrhs = nrhs;
-  int nb = 0;
   for (int c = 0; c <= 8; c++) a.cls_off[c] = cls_off[c];
-  for (int c = 0; c < 8; c++) {
-    a.blk0[c] = nb;
-    const long long cols = (long long)(cls_off[c + 1] - cls_off[c]) * nrhs;
-    nb += (int)((cols + 127) / 128);
-  }
-  a.blk0[8] = nb;
-  g->nblocks = nb;
   std::vector<int4> tab;
   offset_table(tab);
-  // proportional interleave of the classes' blocks (stable: ties by class)
-  std::vector<std::pair<double, int>> order;
-  order.reserve(nb);
-  for (int c = 0; c < 8; c++) {
-    const int n = a.blk0[c + 1] - a.blk0[c];
-    for (int k = 0; k < n; k++) order.push_back({(k + 0.5) / n, 8 * k + c});
-  }
-  std::stable_sort(order.begin(), order.end(),
-                   [](const std::pair<double, int> &x, const std::pair<double, int> &y) { return x.first < y.first; });
-  std::vector<int> blk(nb);
-  for (int i = 0; i < nb; i++) blk[i] = order[i].second;
   int rc = BBFMM_OK;
   auto fail = [&](hipError_t e, const char *what) {
     rc = set_error(BBFMM_E_HIP, "list M2L: %s: %s", what, hipGetErrorString(e));
@@ -2488,50 +2650,45 @@ int list_m2l_create(ListM2L **out, int r, int nrhs, int form, const real *K, int
   if ((e = hipMalloc(&g->d_tab, sizeof(int4) * tab.size())) != hipSuccess) fail(e, "hipMalloc");
   if (rc == BBFMM_OK && (e = hipMemcpy(g->d_tab, tab.data(), sizeof(int4) * tab.size(), hipMemcpyHostToDevice)) != hipSuccess)
     fail(e, "copy");
-  if (rc == BBFMM_OK && nb > 0) {
-    if ((e = hipMalloc(&g->d_blk, sizeof(int) * (size_t)nb)) != hipSuccess) fail(e, "hipMalloc");
-    else if ((e = hipMemcpy(g->d_blk, blk.data(), sizeof(int) * (size_t)nb, hipMemcpyHostToDevice)) != hipSuccess)
-      fail(e, "copy");
-  }
   if (rc == BBFMM_OK) {
     if (form == BBFMM_M2L_BF16X2) {
+      // 16x16x32 products: [operator][row half][hi, lo][lane][8]
       std::vector<__bf16> Kb((size_t)kNumOps * 2 * 2 * 64 * 8);
       for (int k = 0; k < kNumOps; k++)
-        for (int ks = 0; ks < 2; ks++)
+        for (int m = 0; m < 2; m++)
           for (int lane = 0; lane < 64; lane++)
             for (int q = 0; q < 8; q++) {
-              const int row = lane & 31, col = 16 * ks + 8 * (lane >> 5) + q;
+              const int row = 16 * m + (lane & 15), col = 8 * (lane >> 4) + q;
               const float v = K[(size_t)k * 32 * 32 + (size_t)col * 32 + row];
               const __bf16 h = (__bf16)v;
-              Kb[((((size_t)k * 2 + ks) * 2 + 0) * 64 + lane) * 8 + q] = h;
-              Kb[((((size_t)k * 2 + ks) * 2 + 1) * 64 + lane) * 8 + q] = (__bf16)(v - (float)h);
+              Kb[((((size_t)k * 2 + m) * 2 + 0) * 64 + lane) * 8 + q] = h;
+              Kb[((((size_t)k * 2 + m) * 2 + 1) * 64 + lane) * 8 + q] = (__bf16)(v - (float)h);
             }
       if ((e = hipMalloc(&g->d_K, sizeof(__bf16) * Kb.size())) != hipSuccess) fail(e, "hipMalloc");
       else if ((e = hipMemcpy(g->d_K, Kb.data(), sizeof(__bf16) * Kb.size(), hipMemcpyHostToDevice)) != hipSuccess)
         fail(e, "copy");
-      const size_t nb2 = sizeof(__bf16) * (size_t)nrhs * (ncell + 1) * 32;
-      a.kbytes = (int)(sizeof(__bf16) * Kb.size());
-      a.mbytes = nb2 < ((size_t)1 << 31) ? (int)nb2 : 0;
-      if (rc == BBFMM_OK && (e = hipMalloc(&g->d_M0, nb2)) != hipSuccess) fail(e, "hipMalloc");
-      if (rc == BBFMM_OK && (e = hipMalloc(&g->d_M1, nb2)) != hipSuccess) fail(e, "hipMalloc");
-      if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_M0, 0, nb2, s)) != hipSuccess) fail(e, "memset");
-      if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_M1, 0, nb2, s)) != hipSuccess) fail(e, "memset");
     } else {
+      // 16x16x4 products, k = 4 (lane / 16) + step % 4 (+ 16): [operator][row half][step / 4][lane][step % 4]
       std::vector<float> Kf((size_t)kNumOps * 64 * 16);
       for (int k = 0; k < kNumOps; k++)
-        for (int lane = 0; lane < 64; lane++)
-          for (int ks = 0; ks < 16; ks++) {
-            const int row = lane & 31, col = 16 * (lane >> 5) + ks;
-            Kf[((size_t)k * 64 + lane) * 16 + ks] = K[(size_t)k * 32 * 32 + (size_t)col * 32 + row];
-          }
+        for (int m = 0; m < 2; m++)
+          for (int lane = 0; lane < 64; lane++)
+            for (int p = 0; p < 8; p++) {
+              const int row = 16 * m + (lane & 15), col = 4 * (lane >> 4) + (p & 3) + 16 * (p >> 2);
+              Kf[((((size_t)k * 2 + m) * 2 + (p >> 2)) * 64 + lane) * 4 + (p & 3)] =
+                  K[(size_t)k * 32 * 32 + (size_t)col * 32 + row];
+            }
       if ((e = hipMalloc(&g->d_K, sizeof(float) * Kf.size())) != hipSuccess) fail(e, "hipMalloc");
       else if ((e = hipMemcpy(g->d_K, Kf.data(), sizeof(float) * Kf.size(), hipMemcpyHostToDevice)) != hipSuccess)
         fail(e, "copy");
-      const size_t nb2 = sizeof(float) * (size_t)nrhs * (ncell + 1) * 32;
-      if (rc == BBFMM_OK && (e = hipMalloc(&g->d_M0, nb2)) != hipSuccess) fail(e, "hipMalloc");
-      if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_M0, 0, nb2, s)) != hipSuccess) fail(e, "memset");
     }
   }
+  // the sources: one 128-byte line a cell and vector, the last a zero cell
+  const size_t mb = (size_t)128 * nrhs * (ncell + 1);
+  a.kbytes = kNumOps * 4096;
+  a.mbytes = mb < ((size_t)1 << 31) ? (int)mb : 0;
+  if (rc == BBFMM_OK && (e = hipMalloc(&g->d_M0, mb)) != hipSuccess) fail(e, "hipMalloc");
+  if (rc == BBFMM_OK && (e = hipMemsetAsync(g->d_M0, 0, mb, s)) != hipSuccess) fail(e, "memset");
   if (rc == BBFMM_OK && (e = hipStreamSynchronize(s)) != hipSuccess) fail(e, "sync");
   if (rc != BBFMM_OK) {
     list_m2l_destroy(g);
@@ -2540,25 +2697,12 @@ int list_m2l_create(ListM2L **out, int r, int nrhs, int form, const real *K, int
   a.cls_cells = d_cls_cells;
   a.vsrc = d_vsrc;
   a.tab = g->d_tab;
-  a.blk_tab = g->d_blk;
   a.Ka = g->d_K;
   a.M0 = g->d_M0;
-  a.M1 = g->d_M1;
-  if (nb > 0) {
-    if ((e = hipMalloc(&g->d_mask, sizeof(unsigned long long) * 16 * (size_t)nb)) != hipSuccess ||
-        (nrhs == 1 && (e = hipMalloc(&g->d_vsw, sizeof(int) * 4 * (size_t)nb * kOffsets * 32)) != hipSuccess)) {
-      fail(e, "hipMalloc");
-    } else {
-      hipLaunchKernelGGL(k_m2l_list_mask, dim3(4 * nb), dim3(64), 0, s, a, g->d_mask, g->d_vsw);
-      if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(s)) != hipSuccess) fail(e, "mask set-up");
-    }
-    if (rc != BBFMM_OK) {
-      list_m2l_destroy(g);
-      return rc;
-    }
+  if ((rc = pack_lists(g, s)) != BBFMM_OK) {
+    list_m2l_destroy(g);
+    return rc;
   }
-  a.mask = g->d_mask;
-  a.vsw = g->d_vsw;
   *out = g;
   return BBFMM_OK;
 #endif
@@ -2572,7 +2716,8 @@ void list_m2l_set_flat(ListM2L *g, int flat)
 void list_m2l_destroy(ListM2L *g)
 {
   if (!g) return;
-  for (void *p : {(void *)g->d_tab, (void *)g->d_blk, (void *)g->d_mask, (void *)g->d_vsw, g->d_K, g->d_M0, g->d_M1})
+  for (void *p : {(void *)g->d_tab, (void *)g->d_blk, (void *)g->d_part, (void *)g->d_unit, (void *)g->d_esrc,
+                  (void *)g->d_eslot, g->d_K, g->d_M0})
     if (p) (void)hipFree(p);
   delete g;
 }
@@ -2584,19 +2729,20 @@ int list_m2l_run(ListM2L *g, const real *M, real *L, hipStream_t s, hipEvent_t m
   const long long prep = (long long)a.nrhs * a.ncell * 4;
   const int pb = (int)((prep + 255) / 256);
 #ifdef SINGLE
-  if (g->form == BBFMM_M2L_BF16X2) {
-    hipLaunchKernelGGL(k_m2l_list_prep<BBFMM_M2L_BF16X2>, dim3(pb), dim3(256), 0, s, a, M);
-    BB_HIP(hipGetLastError());
-    if (mid) BB_HIP(hipEventRecord(mid, s));
-    if (g->nblocks && a.mbytes > 0 && !g->flat)  // grids below 2 GB: scalar-offset buffer loads
-      hipLaunchKernelGGL(k_m2l_list_lds<true>, dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
-    else if (g->nblocks)
-      hipLaunchKernelGGL(k_m2l_list_lds<false>, dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
-  } else {
-    hipLaunchKernelGGL(k_m2l_list_prep<BBFMM_M2L_FP32MFMA>, dim3(pb), dim3(256), 0, s, a, M);
-    BB_HIP(hipGetLastError());
-    if (mid) BB_HIP(hipEventRecord(mid, s));
-    if (g->nblocks) hipLaunchKernelGGL(k_m2l_list_mfma<BBFMM_M2L_FP32MFMA>, dim3((g->nblocks + 7) & ~7), dim3(256), 0, s, a);
+  const bool bf16 = g->form == BBFMM_M2L_BF16X2;
+  const bool buf = a.mbytes > 0 && !g->flat;  // grids below 2 GB: 32-bit buffer offsets
+  if (bf16) hipLaunchKernelGGL(k_m2l_list_prep<BBFMM_M2L_BF16X2>, dim3(pb), dim3(256), 0, s, a, M);
+  else hipLaunchKernelGGL(k_m2l_list_prep<BBFMM_M2L_FP32MFMA>, dim3(pb), dim3(256), 0, s, a, M);
+  BB_HIP(hipGetLastError());
+  if (mid) BB_HIP(hipEventRecord(mid, s));
+  if (a.nblk > 0) {
+    const dim3 grid((a.nblk + 7) & ~7, (a.nrhs + a.vb - 1) / a.vb);
+    const size_t lds = sizeof(f32x4) * 8 * a.ts * a.ws;
+    auto launch = [&](auto *k) { hipLaunchKernelGGL(k, grid, dim3(64 * a.ws), lds, s, a); };
+    if (bf16 && buf) launch(k_m2l_list_packed<BBFMM_M2L_BF16X2, true>);
+    else if (bf16) launch(k_m2l_list_packed<BBFMM_M2L_BF16X2, false>);
+    else if (buf) launch(k_m2l_list_packed<BBFMM_M2L_FP32MFMA, true>);
+    else launch(k_m2l_list_packed<BBFMM_M2L_FP32MFMA, false>);
   }
   BB_HIP(hipGetLastError());
   return BBFMM_OK;
