@@ -615,6 +615,7 @@ static PassArgs pass_args(const bbfmm_amd_plan *p, bool rows = false)
   a.M = p->d_M;
   a.L = p->d_L;
   a.F = p->d_F;
+  a.complete = p->complete;
   a.potential = p->potential;
   a.l2p_ref = p->l2p_ref;
 #ifdef SINGLE
@@ -631,7 +632,6 @@ static PassArgs pass_args(const bbfmm_amd_plan *p, bool rows = false)
     a.qt = p->d_qt;
     a.phit = p->d_phit;
     a.pad_of = p->d_pad_of;
-    a.farfield = p->d_farfield;
   }
   return a;
 }
@@ -846,14 +846,24 @@ static bool near_beside(const bbfmm_amd_plan *p, bool rows)
 }
 
 // near: with P2P (the gradient adds the near field itself, for the vectors
-// whose potentials it returns)
-static int solve_sorted(bbfmm_amd_plan *p, bool tm, bool rows, bool near = true)
+// whose potentials it returns); q_dev, phi_dev: the charges and potentials in
+// the user's order, gathered and scattered by P2M and P2P (null: d_q is filled,
+// and d_phi holds the sums)
+static int solve_sorted(bbfmm_amd_plan *p, bool tm, bool rows, bool near = true, const real *q_dev = nullptr,
+                        real *phi_dev = nullptr)
 {
   hipStream_t s = p->stream;
   PassArgs a = pass_args(p, rows);
   P2PArgs pp = p2p_args(p);
   const int nv = rows ? p->width : p->nrhs;  // vectors this solve computes
   pp.nrhs = nv;
+  a.farfield = p->d_farfield;
+  if (q_dev) {
+    a.qin = q_dev;
+    a.perm = pp.perm = p->d_perm;
+    a.qsort = p->d_q;
+    pp.out = phi_dev;
+  }
 #ifdef SINGLE
   if (near && pp.use_mfma && nv >= 16) {
     if (!p->d_qt) return set_error(BBFMM_E_ARG, "internal: solve not prepared");
@@ -922,8 +932,6 @@ static int solve_sorted(bbfmm_amd_plan *p, bool tm, bool rows, bool near = true)
     BB_TRY(launch_down_leaf(a, p->h_ploff.data(), s));
   else
     BB_TRY(launch_l2p(a, s, nv));
-  if (!rows)  // the particle-row L2P writes the far field itself
-    BB_HIP(hipMemcpyAsync(p->d_farfield, p->d_phi, sizeof(real) * p->N, hipMemcpyDeviceToDevice, s));
   // "p2p" stage: P2P itself, or with the near field beside the far field the
   // wait for it after the far field is done (its own time: ST_TOTAL + 1)
   if (tm) BB_HIP(hipEventRecord(stage_event(p, ST_P2P), s));
@@ -1004,18 +1012,25 @@ static int solve_eager(bbfmm_amd_plan *p, const real *q_dev, real *phi_dev, bool
   hipStream_t s = p->stream;
   const bool rows = rows16(p);
   if (tm) BB_HIP(hipEventRecord(stage_event(p, ST_GATHER), s));
+  // complete trees, fewer than 16 vectors: P2M gathers and P2P scatters, two
+  // launches and two passes over the vectors less (1M particles 19 us, of which
+  // P2M and P2P take back 13; 64K 7 of 7)
+  const bool direct = !rows && p->complete && p->nrhs < 16 && p->nleaf > 0;
   if (rows)
     BB_TRY(launch_gather_rows16(p->d_ipad, q_dev, p->nrhs, p->d_qt, p->N, s));
-  else
+  else if (!direct)
     BB_TRY(launch_gather(p->d_perm, q_dev, p->d_q, p->N, p->nrhs, s));
-  BB_TRY(solve_sorted(p, tm, rows));
+  if (direct)
+    BB_TRY(solve_sorted(p, tm, rows, true, q_dev, phi_dev));
+  else
+    BB_TRY(solve_sorted(p, tm, rows));
   if (tm) BB_HIP(hipEventRecord(stage_event(p, ST_SCATTER), s));
   if (rows) {
     const bool beside = near_beside(p, rows);
     BB_TRY(launch_scatter_rows16(p->d_ipad, p->d_phit, beside ? p->d_phin : nullptr, p->d_qt, p->potential, phi_dev,
                                  p->nrhs, p->N, s));
   }
-  else
+  else if (!direct)
     BB_TRY(launch_scatter(p->d_iperm, p->d_phi, phi_dev, p->N, p->nrhs, s));
   if (tm) BB_HIP(hipEventRecord(stage_event(p, ST_TOTAL), s));
   return BBFMM_OK;

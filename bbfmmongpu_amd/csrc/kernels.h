@@ -35,19 +35,24 @@ struct PassArgs {
   const real *Ucm;      // U column-major (n^3 x r)
   const real *Urm;      // U row-major
   const real *q;        // [rhs][N] leaf order
+  // not null: P2M reads the charges here, in the user's order (perm: leaf
+  // order -> user), and writes q (qsort)
+  const real *qin = nullptr;
+  const int *perm = nullptr;
+  real *qsort = nullptr;
   real *phi;            // [rhs][N] leaf order
   real *S, *M, *L, *F;
+  int complete = 0;     // 1: every cell of the levels above the leaves has 8 children
   int potential = 0;    // 1: L2P writes the potential, 0: q * potential (the reference's output)
   int l2p_ref = 0;      // n % 4 == 3: L2P restates the reference's z weights (anotherDownwardPassX.c:304)
   // particle-row form of 16 vectors (rows = 1): charges and potentials as
   // rows of 16 in the padded leaf order of the MFMA P2P; P2M reads qt, L2P
-  // writes the far-field potential into phit and vector 0's far field (with
-  // the output's q factor) into farfield
+  // writes the far-field potential into phit
   int rows = 0;
   const real *qt = nullptr;   // [Npad][16]
   real *phit = nullptr;       // [Npad][16]
   const int *pad_of = nullptr;  // [N] leaf-order index -> padded index
-  real *farfield = nullptr;   // [N] leaf order
+  real *farfield = nullptr;   // [N] leaf order: vector 0's far field (with the output's q factor); null: not kept
   // fused last downward level (launch_down_leaf): post-M2L skips cells from
   // cell_end on and L2L stops before parents of level l2l_end
   int cell_end = 0x7fffffff;
@@ -190,6 +195,10 @@ struct P2PArgs {
   const int *nnbr;         // [nleaf]
   const real *q;           // [rhs][N]
   real *phi;               // [rhs][N] (accumulated into)
+  // not null (fewer than 16 vectors, a leaf per wave or block): the sums go
+  // here, in the user's order (perm: leaf order -> user), and phi is only read
+  real *out = nullptr;
+  const int *perm = nullptr;
   int use_mfma = 0;        // fp32: 16 vectors at a time on MFMA
   int potential = 0;       // 1: add the potential, 0: q * potential (the reference's output)
   // padded particle copy (every leaf padded to a multiple of 4 with far-away,

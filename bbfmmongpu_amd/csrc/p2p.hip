@@ -284,7 +284,11 @@ __device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, in
 #pragma unroll
     for (int r = 0; r < NR; r++) {
       const size_t o = (size_t)(rhs0 + r) * N + sta + i;
-      if (i < cnt && r < nv && (r & 3) == h) a.phi[o] += (a.potential ? (real)1 : a.q[o]) * acc[t][r];
+      if (i < cnt && r < nv && (r & 3) == h) {
+        const real v = a.phi[o] + (a.potential ? (real)1 : a.q[o]) * acc[t][r];
+        if (a.out) a.out[(size_t)(rhs0 + r) * N + a.perm[sta + i]] = v;
+        else a.phi[o] = v;
+      }
     }
   }
 }

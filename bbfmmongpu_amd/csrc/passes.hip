@@ -192,7 +192,16 @@ __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
     } else {
       for (int o = threadIdx.x; o < NR * CH; o += BLOCK) {
         const int k = o / CH, j = o % CH;
-        if (j < nk) sq[j * QS + k] = a.q[(size_t)(rhs0 + k) * a.N + sta + base + j];
+        if (j >= nk) continue;
+        const size_t v = (size_t)(rhs0 + k) * a.N;
+        const int i = sta + base + j;
+        if (a.qin) {
+          const real q = a.qin[v + a.perm[i]];
+          sq[j * QS + k] = q;
+          a.qsort[v + i] = q;
+        } else {
+          sq[j * QS + k] = a.q[v + i];
+        }
       }
     }
     __syncthreads();
@@ -897,8 +906,56 @@ __global__ void __launch_bounds__(1024) k_l2l_v16(PassArgs a, int off)
   }
 }
 
-// M2M for one level (anotherUpwardPass.c:345-560): one block per parent,
-// separable interpolation of the eight children's node values (z, y, x).
+// M2M of one parent (anotherUpwardPass.c:345-560): separable interpolation of
+// the eight children's node values sc (z, y, x) by threads t of nt; every
+// thread of the block calls it (block barriers).  out(l, S_l) gets the nodes.
+template <int NN, class Out>
+__device__ __forceinline__ void m2m_cell(const real *sc, real *szz, real *syy, const real *cw, real prefac3, int t,
+                                         int nt, Out out)
+{
+  constexpr int N3 = NN * NN * NN, N2 = NN * NN;
+  for (int o = t; o < 4 * N3; o += nt) { // z
+    const int pair = o / N3, rem = o % N3, l1 = rem / NN, pz = rem % NN;
+    real v = 0;
+#pragma unroll
+    for (int zb = 0; zb < 2; zb++) {
+      const real *ch = &sc[(2 * pair + zb) * N3 + l1 * NN];
+      const real *w = &cw[zb * N2 + pz * NN];
+#pragma unroll
+      for (int k = 0; k < NN; k++) v += ch[k] * w[k];
+    }
+    szz[o] = v;
+  }
+  __syncthreads();
+  for (int o = t; o < 2 * N3; o += nt) { // y
+    const int xb = o / N3, rem = o % N3, cx = rem / N2, py = (rem / NN) % NN, pz = rem % NN;
+    real v = 0;
+#pragma unroll
+    for (int yb = 0; yb < 2; yb++) {
+      const real *s = &szz[(2 * xb + yb) * N3 + cx * N2 + pz];
+      const real *w = &cw[yb * N2 + py * NN];
+#pragma unroll
+      for (int k = 0; k < NN; k++) v += s[k * NN] * w[k];
+    }
+    syy[o] = v;
+  }
+  __syncthreads();
+  for (int l = t; l < N3; l += nt) { // x
+    const int px = l / N2, rem = l % N2;
+    real v = 0;
+#pragma unroll
+    for (int xb = 0; xb < 2; xb++) {
+      const real *s = &syy[xb * N3 + rem];
+      const real *w = &cw[xb * N2 + px * NN];
+#pragma unroll
+      for (int k = 0; k < NN; k++) v += s[k * N2] * w[k];
+    }
+    out(l, v * prefac3);
+  }
+  __syncthreads();
+}
+
+// M2M for one level: one block per parent.
 template <int NN, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) k_m2m(PassArgs a, int off)
 {
@@ -917,48 +974,53 @@ __global__ void __launch_bounds__(BLOCK) k_m2m(PassArgs a, int off)
   }
   for (int o = threadIdx.x; o < 2 * N2; o += BLOCK) cw[o] = a.Cw[o];
   __syncthreads();
-  for (int o = threadIdx.x; o < 4 * N3; o += BLOCK) { // z
-    const int pair = o / N3, rem = o % N3, l1 = rem / NN, pz = rem % NN;
-    real v = 0;
-#pragma unroll
-    for (int zb = 0; zb < 2; zb++) {
-      const real *ch = &sc[(2 * pair + zb) * N3 + l1 * NN];
-      const real *w = &cw[zb * N2 + pz * NN];
-#pragma unroll
-      for (int k = 0; k < NN; k++) v += ch[k] * w[k];
-    }
-    szz[o] = v;
-  }
-  __syncthreads();
-  for (int o = threadIdx.x; o < 2 * N3; o += BLOCK) { // y
-    const int xb = o / N3, rem = o % N3, cx = rem / N2, py = (rem / NN) % NN, pz = rem % NN;
-    real v = 0;
-#pragma unroll
-    for (int yb = 0; yb < 2; yb++) {
-      const real *s = &szz[(2 * xb + yb) * N3 + cx * N2 + pz];
-      const real *w = &cw[yb * N2 + py * NN];
-#pragma unroll
-      for (int k = 0; k < NN; k++) v += s[k * NN] * w[k];
-    }
-    syy[o] = v;
-  }
-  __syncthreads();
-  for (int l = threadIdx.x; l < N3; l += BLOCK) { // x
-    const int px = l / N2, rem = l % N2;
-    real v = 0;
-#pragma unroll
-    for (int xb = 0; xb < 2; xb++) {
-      const real *s = &syy[xb * N3 + rem];
-      const real *w = &cw[xb * N2 + px * NN];
-#pragma unroll
-      for (int k = 0; k < NN; k++) v += s[k * N2] * w[k];
-    }
-    v *= a.prefac3;
+  m2m_cell<NN>(sc, szz, syy, cw, a.prefac3, threadIdx.x, BLOCK, [&](int l, real v) {
     S[(size_t)A * N3 + l] = v;
     sw[l] = v * a.Kw[l];
-  }
-  __syncthreads();
+  });
   project_u<NN, BLOCK>(sw, a.Urm, a.r, a.M + (size_t)rhs * a.ncell * a.r + (size_t)A * a.r);
+}
+
+// M2M of the levels 3 and 2 of a complete tree in one launch (n <= 4): one
+// block per cell of level 2, a wave per child, whose nodes stay in LDS for the
+// parent.  Bound by the latency of its few blocks, as the two launches it
+// replaces were: 64K particles 12.9 -> 6.3 us, 1M 21.9 -> 16.5 with level 4's.
+template <int NN>
+__global__ void __launch_bounds__(512) k_m2m_top(PassArgs a, int off)
+{
+  constexpr int N3 = NN * NN * NN, N2 = NN * NN;
+  __shared__ real sc[8][8 * N3];
+  __shared__ real szz[8][4 * N3];
+  __shared__ real syy[8][2 * N3];
+  __shared__ real s3[8][N3], sw[8][N3];  // the children's S and Kw .* S
+  __shared__ real cw[2 * N2];
+  const int t = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int A = a.plist[off + blockIdx.x], rhs = blockIdx.y;
+  const int B = a.child[(size_t)8 * A + w];
+  real *S = a.S + (size_t)rhs * a.ncell * N3, *M = a.M + (size_t)rhs * a.ncell * a.r;
+  for (int o = t; o < 8 * N3; o += 64) sc[w][o] = S[(size_t)a.child[(size_t)8 * B + o / N3] * N3 + o % N3];
+  for (int o = threadIdx.x; o < 2 * N2; o += 512) cw[o] = a.Cw[o];
+  __syncthreads();
+  m2m_cell<NN>(sc[w], szz[w], syy[w], cw, a.prefac3, t, 64, [&](int l, real v) {
+    S[(size_t)B * N3 + l] = v;
+    s3[w][l] = v;
+    sw[w][l] = v * a.Kw[l];
+  });
+  auto project = [&](const real *s, int cell) {
+    for (int i = t; i < a.r; i += 64) {
+      real m = 0;
+#pragma unroll 8
+      for (int l = 0; l < N3; l++) m += a.Urm[(size_t)l * a.r + i] * s[l];
+      M[(size_t)cell * a.r + i] = m;
+    }
+  };
+  project(sw[w], B);
+  __syncthreads();
+  m2m_cell<NN>(s3[0], szz[0], syy[0], cw, a.prefac3, threadIdx.x, 512, [&](int l, real v) {
+    S[(size_t)A * N3 + l] = v;
+    sw[0][l] = v * a.Kw[l];
+  });
+  if (w == 0) project(sw[0], A);
 }
 
 // post-M2L (auxAnotherFMMInteraction.c:398-416, scale per level as
@@ -996,8 +1058,41 @@ __global__ void __launch_bounds__(BLOCK) k_postm2l(PassArgs a, int Afirst)
   }
 }
 
-// L2L for one level (anotherDownwardPassX.c:40-211): one block per parent,
-// children F += (2/n)^3 * interpolation of the parent's F (x, y, z).
+// L2L of one parent (anotherDownwardPassX.c:40-211): (2/n)^3 * interpolation
+// of the parent's nodes fa (x, y, z) by threads t of nt; every thread of the
+// block calls it (block barriers).  out(j, l, v): what child j's node l gains.
+template <int NN, class Out>
+__device__ __forceinline__ void l2l_cell(const real *fa, real *fx, real *fy, const real *cw, real prefac3, int t,
+                                         int nt, Out out)
+{
+  constexpr int N3 = NN * NN * NN, N2 = NN * NN;
+  for (int o = t; o < 2 * N3; o += nt) { // x
+    const int xb = o / N3, rem = o % N3, cx = rem / N2, yz = rem % N2;
+    real v = 0;
+#pragma unroll
+    for (int k = 0; k < NN; k++) v += fa[k * N2 + yz] * cw[xb * N2 + k * NN + cx];
+    fx[o] = v;
+  }
+  __syncthreads();
+  for (int o = t; o < 4 * N3; o += nt) { // y
+    const int jj = o / N3, rem = o % N3, cx = rem / N2, cy = (rem / NN) % NN, pz = rem % NN;
+    real v = 0;
+#pragma unroll
+    for (int k = 0; k < NN; k++)
+      v += fx[(jj >> 1) * N3 + cx * N2 + k * NN + pz] * cw[(jj & 1) * N2 + k * NN + cy];
+    fy[o] = v;
+  }
+  __syncthreads();
+  for (int o = t; o < 8 * N3; o += nt) { // z
+    const int j = o / N3, rem = o % N3, l1 = rem / NN, cz = rem % NN;
+    real v = 0;
+#pragma unroll
+    for (int k = 0; k < NN; k++) v += fy[(j >> 1) * N3 + l1 * NN + k] * cw[(j & 1) * N2 + k * NN + cz];
+    out(j, rem, prefac3 * v);
+  }
+}
+
+// L2L for one level: one block per parent.
 template <int NN, int BLOCK>
 __global__ void __launch_bounds__(BLOCK) k_l2l(PassArgs a, int off)
 {
@@ -1012,31 +1107,40 @@ __global__ void __launch_bounds__(BLOCK) k_l2l(PassArgs a, int off)
   for (int o = threadIdx.x; o < N3; o += BLOCK) fa[o] = F[(size_t)A * N3 + o];
   for (int o = threadIdx.x; o < 2 * N2; o += BLOCK) cw[o] = a.Cw[o];
   __syncthreads();
-  for (int o = threadIdx.x; o < 2 * N3; o += BLOCK) { // x
-    const int xb = o / N3, rem = o % N3, cx = rem / N2, yz = rem % N2;
-    real v = 0;
-#pragma unroll
-    for (int k = 0; k < NN; k++) v += fa[k * N2 + yz] * cw[xb * N2 + k * NN + cx];
-    fx[o] = v;
-  }
-  __syncthreads();
-  for (int o = threadIdx.x; o < 4 * N3; o += BLOCK) { // y
-    const int jj = o / N3, rem = o % N3, cx = rem / N2, cy = (rem / NN) % NN, pz = rem % NN;
-    real v = 0;
-#pragma unroll
-    for (int k = 0; k < NN; k++)
-      v += fx[(jj >> 1) * N3 + cx * N2 + k * NN + pz] * cw[(jj & 1) * N2 + k * NN + cy];
-    fy[o] = v;
-  }
-  __syncthreads();
-  for (int o = threadIdx.x; o < 8 * N3; o += BLOCK) { // z, add into the children
-    const int j = o / N3, rem = o % N3, l1 = rem / NN, cz = rem % NN;
-    real v = 0;
-#pragma unroll
-    for (int k = 0; k < NN; k++) v += fy[(j >> 1) * N3 + l1 * NN + k] * cw[(j & 1) * N2 + k * NN + cz];
+  l2l_cell<NN>(fa, fx, fy, cw, a.prefac3, threadIdx.x, BLOCK, [&](int j, int l, real v) {
     const int ch = a.child[(size_t)8 * A + j];
-    if (ch >= 0) F[(size_t)ch * N3 + rem] += a.prefac3 * v;
-  }
+    if (ch >= 0) F[(size_t)ch * N3 + l] += v;
+  });
+}
+
+// L2L of the levels 2 and 3 of a complete tree in one launch (n <= 4): one
+// block per cell of level 2, then a wave per child, whose nodes are in LDS.
+// 64K particles 12.1 -> 7.5 us, 1M 23.4 -> 18.2 with level 4's.
+template <int NN>
+__global__ void __launch_bounds__(512) k_l2l_top(PassArgs a, int off)
+{
+  constexpr int N3 = NN * NN * NN, N2 = NN * NN;
+  __shared__ real fa[N3], f3[8][N3];
+  __shared__ real fx[8][2 * N3];
+  __shared__ real fy[8][4 * N3];
+  __shared__ real cw[2 * N2];
+  const int t = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int A = a.plist[off + blockIdx.x], rhs = blockIdx.y;
+  const int *child = a.child + (size_t)8 * A;
+  real *F = a.F + (size_t)rhs * a.ncell * N3;
+  for (int o = threadIdx.x; o < N3; o += 512) fa[o] = F[(size_t)A * N3 + o];
+  for (int o = threadIdx.x; o < 2 * N2; o += 512) cw[o] = a.Cw[o];
+  __syncthreads();
+  l2l_cell<NN>(fa, fx[0], fy[0], cw, a.prefac3, threadIdx.x, 512, [&](int j, int l, real v) {
+    real *f = &F[(size_t)child[j] * N3 + l];
+    v += *f;
+    *f = v;
+    f3[j][l] = v;
+  });
+  __syncthreads();
+  const int *grand = a.child + (size_t)8 * child[w];
+  l2l_cell<NN>(f3[w], fx[w], fy[w], cw, a.prefac3, t, 64,
+               [&](int j, int l, real v) { F[(size_t)grand[j] * N3 + l] += v; });
 }
 
 // L2P (anotherDownwardPassX.c:226-424): one thread per particle,
@@ -1070,7 +1174,9 @@ __global__ void __launch_bounds__(256) k_l2p(PassArgs a)
       sum += sxv[l1] * syv[l2] * inner;
     }
   const size_t o = (size_t)rhs * a.N + i;
-  a.phi[o] = (a.potential ? (real)1 : a.q[o]) * a.prefac3 * sum;
+  const real v = (a.potential ? (real)1 : a.q[o]) * a.prefac3 * sum;
+  a.phi[o] = v;
+  if (rhs == 0 && a.farfield) a.farfield[i] = v;
 }
 
 // L2P for NR vectors: one block per leaf, the leaf's F values in LDS
@@ -1136,7 +1242,9 @@ __global__ void __launch_bounds__(64) k_l2p_leaf(PassArgs a)
 #pragma unroll
       for (int k = 0; k < RS; k++) {
         const size_t o = (size_t)(rhs0 + g * RS + k) * a.N + sta + j;
-        a.phi[o] = (a.potential ? (real)1 : a.q[o]) * a.prefac3 * sum[k];
+        const real v = (a.potential ? (real)1 : a.q[o]) * a.prefac3 * sum[k];
+        a.phi[o] = v;
+        if (rhs0 + g * RS + k == 0 && a.farfield) a.farfield[sta + j] = v;
       }
     }
   }
@@ -1493,14 +1601,35 @@ int launch_p2m(const PassArgs &a, hipStream_t s, int nrhs)
   return BBFMM_OK;
 }
 
+// orders of k_m2m_top and k_l2l_top (a wave per cell): n = 3, 4
+constexpr int kTopOrder = 4;
+#define BB_WITH_TOP_ORDER(n, ...)      \
+  do {                                 \
+    if ((n) == 4) {                    \
+      constexpr int NN = 4;            \
+      __VA_ARGS__;                     \
+    } else {                           \
+      constexpr int NN = 3;            \
+      __VA_ARGS__;                     \
+    }                                  \
+  } while (0)
+
 int launch_m2m(const PassArgs &a, const int *h_ploff, hipStream_t s, int nrhs)
 {
   if (a.n < kMinOrder || a.n > kMaxOrder)
     return set_error(BBFMM_E_ARG, "Chebyshev order n=%d not supported (n = %d..%d)", a.n, kMinOrder, kMaxOrder);
+  const bool v16 = a.n == 4 && a.r == 32 && nrhs == 16;
   for (int level = std::min(a.maxlev - 1, a.m2m_start); level >= kMinLev; level--) {
-    const int off = h_ploff[level], count = h_ploff[level + 1] - off;
+    int off = h_ploff[level], count = h_ploff[level + 1] - off;
     if (count <= 0) continue;
-    if (a.n == 4 && a.r == 32 && nrhs == 16)
+    if (level == kMinLev + 1 && a.complete && a.n <= kTopOrder && !v16) {
+      off = h_ploff[kMinLev];
+      count = h_ploff[kMinLev + 1] - off;
+      BB_WITH_TOP_ORDER(a.n, hipLaunchKernelGGL(k_m2m_top<NN>, dim3(count, nrhs), dim3(512), 0, s, a, off));
+      BB_HIP(hipGetLastError());
+      break;
+    }
+    if (v16)
       hipLaunchKernelGGL(k_m2m_v16, dim3(count), dim3(1024), 0, s, a, off);
 #ifdef SINGLE
     else if (a.mplist && a.T8m && a.n == 4 && a.r == 32)
@@ -1557,10 +1686,15 @@ int launch_l2l(const PassArgs &a, const int *h_ploff, hipStream_t s, int nrhs)
   // L2L only (parents at levels minlev..maxlev-1)
   if (a.n < kMinOrder || a.n > kMaxOrder)
     return set_error(BBFMM_E_ARG, "Chebyshev order n=%d not supported (n = %d..%d)", a.n, kMinOrder, kMaxOrder);
-  for (int level = kMinLev; level < std::min(a.maxlev, a.l2l_end); level++) {
+  const bool v16 = a.n == 4 && nrhs == 16;
+  const int end = std::min(a.maxlev, a.l2l_end);
+  for (int level = kMinLev; level < end; level++) {
     const int off = h_ploff[level], count = h_ploff[level + 1] - off;
     if (count <= 0) continue;
-    if (a.n == 4 && nrhs == 16)
+    if (level == kMinLev && level + 1 < end && a.complete && a.n <= kTopOrder && !v16) {
+      BB_WITH_TOP_ORDER(a.n, hipLaunchKernelGGL(k_l2l_top<NN>, dim3(count, nrhs), dim3(512), 0, s, a, off));
+      level++;
+    } else if (v16)
       hipLaunchKernelGGL(k_l2l_v16, dim3(count), dim3(1024), 0, s, a, off);
     else
       BB_WITH_ORDER(a.n, hipLaunchKernelGGL((k_l2l<NN, node_block(NN)>), dim3(count, nrhs), dim3(node_block(NN)),
