@@ -11,6 +11,8 @@
 #include "common.h"
 #include "kernels.h"
 
+#include <type_traits>
+
 namespace bb {
 
 __device__ __forceinline__ real rsqrt_r(real x)
@@ -116,8 +118,8 @@ __global__ void k_pack_pq(int N, const real4 *__restrict__ pos, const real *__re
 }
 
 // ---------------------------------------------------------------- 1 to 8 vectors
-// A wavefront's lanes are 16 targets x 4 source groups: group h takes the
-// staged sources h, h + 4, ... for up to NTMAX tiles of 16 targets of the
+// A wavefront's lanes are 16 targets x 4 source groups (fp64: 8 x 8): group h
+// takes the staged sources h, h + 4, ... for up to NTMAX tiles of targets of the
 // leaf, so that leaves of a few dozen particles keep the lanes busy (a lane a
 // target left half of them idle at 33 to 48 particles) and every source read
 // from LDS serves NT targets.  The groups' sums are added across lanes at the
@@ -125,17 +127,23 @@ __global__ void k_pack_pq(int N, const real4 *__restrict__ pos, const real *__re
 // added through LDS; the target tiles of a leaf go to gridDim.y blocks, so
 // that few large leaves fill the chip too.  Each wave stages up to kP2PLeaves
 // leaves (64 sources of each) at a time in its own part of LDS, their loads
-// in flight together, padded to a multiple of 8 with far sources of zero
+// in flight together, padded to a multiple of 8 (16) with far sources of zero
 // charge (no tail masks).  The r != 0 test is applied in the self leaf, which
 // wave 0 stages by itself.
 // Bound by the vector ALUs (7 + NR fp32 operations and a reciprocal square
 // root a pair; fp64: the library rsqrt).  N = 1M, depth 5, one vector: 467 -> 244
 // us (45 cycles of a SIMD per 64 pairs of whole tiles; the operations alone
 // measure 37); 4096, depth 2 (64 leaves of 64): 192 -> 11.7 us; 65536, depth
-// 4: 33 -> 21.5 us; fp64 100003, depth 4: 117 -> 60 us; 4 vectors of 150001
+// 4: 33 -> 21.5 us; fp64 100003, depth 4: 117 -> 57.6 us; 4 vectors of 150001
 // on a sphere, depth 5: 249 -> 85 us.
 constexpr int kP2PLeaves = 4;  // leaves staged together
 constexpr int kP2PStage = 64 * kP2PLeaves;
+// Targets of a tile.  fp64: 8 leave fewer lanes without a target, 100003
+// particles, depth 4, 66.9 -> 57.6 us, 500000, depth 5, 206 -> 191; fp32 gains
+// nothing (1M 246 and 246, 65536 20.6 and 22.4), its pairs being cheap against
+// the staged sources' padding to 16 and the longer sums across lanes.
+constexpr int kTile = sizeof(real) == 4 ? 16 : 8;
+constexpr int kGroups = 64 / kTile;    // source groups
 
 typedef real realx4 __attribute__((ext_vector_type(4)));
 
@@ -146,18 +154,18 @@ struct P2PStage {
   real q[NR > 1 ? kP2PStage : 1][NR] __attribute__((aligned(16)));
 };
 
-// acc += the sums over the n8 (a multiple of 8) staged sources, two of a lane's at a time
+// acc += the sums over the n2 (a multiple of 2 kGroups) staged sources, two of a lane's at a time
 template <int NR, int NT, bool SELF>
-__device__ __forceinline__ void p2p_sweep(const P2PStage<NR> &st, int n8, int h, const realx4 *x, real (&acc)[NT][NR])
+__device__ __forceinline__ void p2p_sweep(const P2PStage<NR> &st, int n2, int h, const realx4 *x, real (&acc)[NT][NR])
 {
-  for (int k = 0; k < n8; k += 8) {
+  for (int k = 0; k < n2; k += 2 * kGroups) {
     realx4 z[2];
     real q[2][NR];
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-      z[u] = st.s[k + 4 * u + h];
+      z[u] = st.s[k + kGroups * u + h];
 #pragma unroll
-      for (int r = 0; r < NR; r++) q[u][r] = NR > 1 ? st.q[k + 4 * u + h][r] : z[u].w;
+      for (int r = 0; r < NR; r++) q[u][r] = NR > 1 ? st.q[k + kGroups * u + h][r] : z[u].w;
     }
 #pragma unroll
     for (int u = 0; u < 2; u++)
@@ -178,14 +186,14 @@ __device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, in
 {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), W = blockDim.x >> 6;
-  const int ti = lane & 15, h = lane >> 4;
+  const int ti = lane % kTile, h = lane / kTile;
   const size_t N = a.N;
   const realx4 *pos = reinterpret_cast<const realx4 *>(a.pos);
   realx4 x[NT];
   real acc[NT][NR];
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    x[t] = pos[sta + min(tb + 16 * t + ti, cnt - 1)];  // targets past the leaf's end are not stored
+    x[t] = pos[sta + min(tb + kTile * t + ti, cnt - 1)];  // targets past the leaf's end are not stored
 #pragma unroll
     for (int r = 0; r < NR; r++) acc[t][r] = 0;
   }
@@ -206,15 +214,15 @@ __device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, in
         for (int r = 0; r < NR; r++) st.q[at + lane][r] = q[r];
     }
   };
-  auto pad = [&](int n) {  // to a multiple of 8
-    const int n8 = (n + 7) & ~7;
-    if (lane < n8 - n) {
+  auto pad = [&](int n) {  // to a multiple of 2 kGroups
+    const int n2 = (n + 2 * kGroups - 1) & ~(2 * kGroups - 1);
+    if (lane < n2 - n) {
       st.s[n + lane] = realx4{(real)1e6, (real)1e6, (real)1e6, 0};
       if (NR > 1)
 #pragma unroll
         for (int r = 0; r < NR; r++) st.q[n + lane][r] = 0;
     }
-    return n8;
+    return n2;
   };
   if (wave == 0) {  // the leaf itself
     for (int j = 0; j < cnt; j += 64) {
@@ -260,8 +268,7 @@ __device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, in
   for (int t = 0; t < NT; t++)
 #pragma unroll
     for (int r = 0; r < NR; r++) {
-      acc[t][r] += __shfl_xor(acc[t][r], 16);
-      acc[t][r] += __shfl_xor(acc[t][r], 32);
+      for (int k = kTile; k < 64; k <<= 1) acc[t][r] += __shfl_xor(acc[t][r], k);
     }
   if (W > 1) {
     __syncthreads();  // the previous pass's sums have been read
@@ -269,22 +276,22 @@ __device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, in
 #pragma unroll
       for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int r = 0; r < NR; r++) red[((wave * NT + t) * NR + r) * 16 + ti] = acc[t][r];
+        for (int r = 0; r < NR; r++) red[((wave * NT + t) * NR + r) * kTile + ti] = acc[t][r];
     __syncthreads();
     if (wave > 0) return;
     for (int w = 1; w < W; w++)
 #pragma unroll
       for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int r = 0; r < NR; r++) acc[t][r] += red[((w * NT + t) * NR + r) * 16 + ti];
+        for (int r = 0; r < NR; r++) acc[t][r] += red[((w * NT + t) * NR + r) * kTile + ti];
   }
 #pragma unroll
   for (int t = 0; t < NT; t++) {
-    const int i = tb + 16 * t + ti;
+    const int i = tb + kTile * t + ti;
 #pragma unroll
     for (int r = 0; r < NR; r++) {
       const size_t o = (size_t)(rhs0 + r) * N + sta + i;
-      if (i < cnt && r < nv && (r & 3) == h) {
+      if (i < cnt && r < nv && (r & (kGroups - 1)) == h) {
         const real v = a.phi[o] + (a.potential ? (real)1 : a.q[o]) * acc[t][r];
         if (a.out) a.out[(size_t)(rhs0 + r) * N + a.perm[sta + i]] = v;
         else a.phi[o] = v;
@@ -298,7 +305,7 @@ template <int NR, int NTMAX, int MAXW>
 __global__ void __launch_bounds__(64 * MAXW) k_p2p(P2PArgs a, int rhs0, int nv)
 {
   __shared__ P2PStage<NR> stage[MAXW];
-  __shared__ real red[MAXW > 1 ? MAXW * NTMAX * NR * 16 : 1];
+  __shared__ real red[MAXW > 1 ? MAXW * NTMAX * NR * kTile : 1];
   const int leaf = xcd_leaf(blockIdx.x, a.nleaf);
   const int lane = threadIdx.x & 63;
   const int sta = a.leafsta[leaf], cnt = a.leafcnt[leaf], nn = a.nnbr[leaf];
@@ -310,12 +317,21 @@ __global__ void __launch_bounds__(64 * MAXW) k_p2p(P2PArgs a, int rhs0, int nv)
   }
   P2PStage<NR> &st = stage[threadIdx.x >> 6];
   // passes of NTMAX tiles, dealt to the gridDim.y blocks
-  for (int tb = blockIdx.y * 16 * NTMAX; tb < cnt; tb += gridDim.y * 16 * NTMAX) {
-    const int nt = min(NTMAX, (cnt - tb + 15) >> 4);
-    if (NTMAX >= 4 && nt == 4) p2p_tiles<NR, (NTMAX >= 4 ? 4 : 1)>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
-    else if (NTMAX >= 3 && nt == 3) p2p_tiles<NR, (NTMAX >= 3 ? 3 : 1)>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
-    else if (NTMAX >= 2 && nt == 2) p2p_tiles<NR, (NTMAX >= 2 ? 2 : 1)>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
-    else p2p_tiles<NR, 1>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
+  for (int tb = blockIdx.y * kTile * NTMAX; tb < cnt; tb += gridDim.y * kTile * NTMAX) {
+    const int nt = min(NTMAX, (cnt - tb + kTile - 1) / kTile);
+    auto run = [&](auto k) {
+      constexpr int NT = decltype(k)::value;
+      if constexpr (NT <= NTMAX)
+        p2p_tiles<NR, NT>(a, rhs0, nv, leaf, tb, sta, cnt, nsta, ncnt, nn, st, red);
+    };
+    switch (nt) {
+    case 1: run(std::integral_constant<int, 1>()); break;
+    case 2: run(std::integral_constant<int, 2>()); break;
+    case 3: run(std::integral_constant<int, 3>()); break;
+    case 4: run(std::integral_constant<int, 4>()); break;
+    case 5: run(std::integral_constant<int, 5>()); break;
+    default: run(std::integral_constant<int, 6>()); break;
+    }
   }
 }
 
@@ -837,10 +853,11 @@ static void p2p_few_t(const P2PArgs &a, int rhs, int nv, hipStream_t s)
 //   fp32, 4 vectors: 262144 4x4 170.5, 4x1 171.9; 65536 2x1 33.6, 2x4 39.7;
 //                    50000 2x4 63.4, 2x8 65.8; 4096 2x8 15.2, 2x4 19.1
 //   fp32, 7 vectors: 1M 4x1 524, 2x1 633; 16384, 512 leaves 2x4 24.1
-//   fp64:            100003, 4096 leaves, 1 vector 2x4 67.7, 2x1 71.7, 4
-//                    vectors 2x1 109.7, 2x4 128; 8000, 64 leaves, 1 vector
-//                    2x4 62.6, 2x1 177; 40000, 512 leaves, 7 vectors 2x1 177,
-//                    2x4 222
+//   fp64:            100003, 4096 leaves, 1 vector 4x4 57.4, 4x1 57.6, 4
+//                    vectors 4x1 95.1, 4x4 134; 500000, 32768 leaves, 1
+//                    vector 4x1 191, 4x4 275; 8000, 64 leaves, 1 vector 6x4
+//                    38.6, 4x4 45.7, 4x1 111; 40000, 512 leaves, 4 vectors 6x4
+//                    97.5, 4x4 101, 4x1 117
 template <int NR>
 static void p2p_few_n(const P2PArgs &a, int rhs, int nv, hipStream_t s)
 {
@@ -856,8 +873,9 @@ static void p2p_few_n(const P2PArgs &a, int rhs, int nv, hipStream_t s)
     else p2p_few_t<NR, 2, 1>(a, rhs, nv, s);
   }
 #else
-  if (a.nleaf <= (NR == 1 ? 6144 : NR < 8 ? 1024 : 128)) p2p_few_t<NR, 2, 4>(a, rhs, nv, s);
-  else p2p_few_t<NR, 2, 1>(a, rhs, nv, s);
+  if (a.nleaf <= (NR < 8 ? 1024 : 128)) p2p_few_t<NR, NR < 8 ? 6 : 4, 4>(a, rhs, nv, s);
+  else if (NR == 1 && a.nleaf <= 6144) p2p_few_t<NR, 4, 4>(a, rhs, nv, s);
+  else p2p_few_t<NR, 4, 1>(a, rhs, nv, s);
 #endif
 }
 
