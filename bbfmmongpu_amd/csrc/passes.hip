@@ -16,6 +16,7 @@
 #include "kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace bb {
 
@@ -145,6 +146,8 @@ __host__ __device__ constexpr int row_stride()
 // P2M at the leaf level (anotherUpwardPass.c:61-330): one block per leaf and
 // group of NR vectors, one thread per Chebyshev node (n=8: two nodes per
 // thread); S = sum_j q_j Sx Sy Sz, then M = U^T (Kw .* S).
+// The weights of four particles are read at a time; an empty leaf's zeros are
+// only written (150000 particles on a surface, 4 vectors: 41 -> 26.5 us).
 // ROWS: the 16 charges of a particle are one row of a.qt (padded leaf order).
 template <int NN, int BLOCK, int NR, bool ROWS = false>
 __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
@@ -154,7 +157,8 @@ __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
   constexpr int NPT = (N3 + BLOCK - 1) / BLOCK;  // nodes per thread (the last may be past N3)
   constexpr int CH = BLOCK;
   constexpr int QS = row_stride<NR>();
-  __shared__ real sx[NN][CH], sy[NN][CH], sz[NN][CH];
+  typedef real vec4 __attribute__((ext_vector_type(4)));
+  __shared__ __align__(16) real sx[NN][CH], sy[NN][CH], sz[NN][CH];
   __shared__ __align__(16) real sq[CH * QS];
   __shared__ __align__(16) real sw[N3 * NR];
   const int leaf = blockIdx.x;
@@ -163,13 +167,21 @@ __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
   const real ih = a.leafihalf[leaf];
   const int sta = a.leafsta[leaf], cnt = a.leafcnt[leaf];
   const real4 c = a.center[A];
+  if (cnt == 0) {  // whole block
+    for (int k = 0; k < NR; k++) {
+      real *S = a.S + ((size_t)(rhs0 + k) * a.ncell + A) * N3, *M = a.M + ((size_t)(rhs0 + k) * a.ncell + A) * a.r;
+      for (int l = threadIdx.x; l < N3; l += BLOCK) S[l] = 0;
+      for (int i = threadIdx.x; i < a.r; i += BLOCK) M[i] = 0;
+    }
+    return;
+  }
   real acc[NPT][NR];
 #pragma unroll
   for (int p = 0; p < NPT; p++)
 #pragma unroll
     for (int k = 0; k < NR; k++) acc[p][k] = 0;
   for (int base = 0; base < cnt; base += CH) {
-    const int nk = min(CH, cnt - base);
+    const int nk = min(CH, cnt - base), nk4 = (nk + 3) & ~3;  // in fours, the last filled up with zeros
     if ((int)threadIdx.x < nk) {
       const real4 x = a.pos[sta + base + threadIdx.x];
       real t[NN];
@@ -182,17 +194,23 @@ __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
       cheb_row<NN>(a.Tkz, ih * (x.z - c.z), t);
 #pragma unroll
       for (int m = 0; m < NN; m++) sz[m][threadIdx.x] = t[m];
+    } else if ((int)threadIdx.x < nk4) {
+#pragma unroll
+      for (int m = 0; m < NN; m++) sx[m][threadIdx.x] = sy[m][threadIdx.x] = sz[m][threadIdx.x] = 0;
     }
     if (ROWS) {
       const real *qr = a.qt + (size_t)a.pad_of[sta] * 16;  // the leaf's rows are contiguous
       for (int o = threadIdx.x; o < 16 * CH; o += BLOCK) {
         const int j = o >> 4, k = o & 15;
-        if (j < nk) sq[j * QS + k] = qr[(size_t)(base + j) * 16 + k];
+        if (j < nk4) sq[j * QS + k] = j < nk ? qr[(size_t)(base + j) * 16 + k] : (real)0;
       }
     } else {
       for (int o = threadIdx.x; o < NR * CH; o += BLOCK) {
         const int k = o / CH, j = o % CH;
-        if (j >= nk) continue;
+        if (j >= nk) {
+          if (j < nk4) sq[j * QS + k] = 0;
+          continue;
+        }
         const size_t v = (size_t)(rhs0 + k) * a.N;
         const int i = sta + base + j;
         if (a.qin) {
@@ -210,10 +228,18 @@ __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
       const int l = threadIdx.x + p * BLOCK;
       if (N3 % BLOCK != 0 && l >= N3) break;
       const int l1 = l / (NN * NN), l2 = (l / NN) % NN, l3 = l % NN;
-      for (int j = 0; j < nk; j++) {
-        const real w = sx[l1][j] * sy[l2][j] * sz[l3][j];
+      for (int j = 0; j < nk4; j += 4) {
+        const vec4 w = *(const vec4 *)&sx[l1][j] * *(const vec4 *)&sy[l2][j] * *(const vec4 *)&sz[l3][j];
+        if (NR == 1) {
+          const vec4 q = *(const vec4 *)&sq[j];
+          acc[p][0] += (q.x * w.x + q.y * w.y) + (q.z * w.z + q.w * w.w);
+        } else {
+          const real we[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-        for (int k = 0; k < NR; k++) acc[p][k] += sq[j * QS + k] * w;
+          for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int k = 0; k < NR; k++) acc[p][k] += sq[(j + e) * QS + k] * we[e];
+        }
       }
     }
     __syncthreads();
@@ -1025,36 +1051,45 @@ __global__ void __launch_bounds__(512) k_m2m_top(PassArgs a, int off)
 
 // post-M2L (auxAnotherFMMInteraction.c:398-416, scale per level as
 // anotherFMMInteraction.cu:89-113): F = (1/L_l)^homogen Kw .* (U L), one
-// block per cell and group of NR vectors, a thread per node.
-template <int NN, int BLOCK, int NR>
-__global__ void __launch_bounds__(BLOCK) k_postm2l(PassArgs a, int Afirst)
+// block per CB cells and group of NR vectors, a thread per node: each value of
+// U is read once for all of them.
+template <int NN, int BLOCK, int NR, int CB>
+__global__ void __launch_bounds__(BLOCK) k_postm2l(PassArgs a, int count)
 {
-  constexpr int N3 = NN * NN * NN;
+  constexpr int N3 = NN * NN * NN, C = CB * NR;
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  real *sl = reinterpret_cast<real *>(smem_raw);  // [r][NR]
-  const int A = Afirst + blockIdx.x;
+  real *sl = reinterpret_cast<real *>(smem_raw);  // [r][cell][vector]
+  const int A0 = blockIdx.x * CB;
   const int rhs0 = blockIdx.y * NR;
-  const int level = a.celllev[A];
-  if (level < kMinLev) return;  // whole block, before any barrier
-  const real scale = a.scale[level];
-  for (int o = threadIdx.x; o < a.r * NR; o += BLOCK) {
-    const int k = o / a.r, i = o % a.r;
-    sl[i * NR + k] = a.L[(size_t)(rhs0 + k) * a.ncell * a.r + (size_t)A * a.r + i];
+  const int nc = min(CB, count - A0);
+  bool any = false;
+  for (int c = 0; c < nc; c++) any |= a.celllev[A0 + c] >= kMinLev;
+  if (!any) return;  // whole block, before any barrier
+  for (int k = 0; k < NR; k++) {
+    const real *L = a.L + (size_t)(rhs0 + k) * a.ncell * a.r + (size_t)A0 * a.r;
+    for (int o = threadIdx.x; o < nc * a.r; o += BLOCK) sl[(o % a.r) * C + o / a.r * NR + k] = L[o];
   }
   __syncthreads();
   for (int l = threadIdx.x; l < N3; l += BLOCK) {
-    real s[NR];
+    real s[C];
 #pragma unroll
-    for (int k = 0; k < NR; k++) s[k] = 0;
-#pragma unroll 4
+    for (int k = 0; k < C; k++) s[k] = 0;
+#pragma unroll(C > 4 ? 4 : 8)
     for (int i = 0; i < a.r; i++) {
       const real u = a.Ucm[l + (size_t)N3 * i];
 #pragma unroll
-      for (int k = 0; k < NR; k++) s[k] += u * sl[i * NR + k];
+      for (int k = 0; k < C; k++) s[k] += u * sl[i * C + k];
     }
-    const real f = scale * a.Kw[l];
+    const real kw = a.Kw[l];
 #pragma unroll
-    for (int k = 0; k < NR; k++) a.F[(size_t)(rhs0 + k) * a.ncell * N3 + (size_t)A * N3 + l] = f * s[k];
+    for (int c = 0; c < CB; c++) {
+      if (c >= nc) break;
+      const int level = a.celllev[A0 + c];
+      if (level < kMinLev) continue;
+      const real f = a.scale[level] * kw;
+#pragma unroll
+      for (int k = 0; k < NR; k++) a.F[(size_t)(rhs0 + k) * a.ncell * N3 + (size_t)(A0 + c) * N3 + l] = f * s[c * NR + k];
+    }
   }
 }
 
@@ -1643,20 +1678,28 @@ int launch_m2m(const PassArgs &a, const int *h_ploff, hipStream_t s, int nrhs)
   return BBFMM_OK;
 }
 
-// every cell; blocks of cells above level 2 return at once
+// Every cell; what lies above level 2 is not written.  Cells of a block, in us
+// (post-M2L of one vector): 37449 cells, n = 4, 1 cell 18.2, 2 13.4, 4 11.7, 8
+// 12.2; 4681 cells, n = 4 7.3, 6.8, 7.2, n = 6 23.1, 16.3, 12.8, 16.4, n = 8
+// 83.6, 52.0, 34.8, 49.9; 4 vectors, 37449 cells 26.9, 22.5, 23.3, 4681 9.3,
+// 10.2, 12.1.
+template <int NN, int BLOCK, int NR, int CB>
+static void postm2l_c(const PassArgs &a, hipStream_t s, int nrhs)
+{
+  hipLaunchKernelGGL((k_postm2l<NN, BLOCK, NR, CB>), dim3((a.ncell + CB - 1) / CB, nrhs / NR), dim3(BLOCK),
+                     sizeof(real) * a.r * NR * CB, s, a, a.ncell);
+}
+
 template <int NN, int BLOCK>
 static int postm2l_t(const PassArgs &a, hipStream_t s, int nrhs)
 {
-  const int first = 0, count = a.ncell;
-  if (count <= 0) return BBFMM_OK;
+  if (a.ncell <= 0) return BBFMM_OK;
   const int nr = vec_group(nrhs);
-  const size_t sh = sizeof(real) * a.r * nr;
-  if (nr == 16)
-    hipLaunchKernelGGL((k_postm2l<NN, BLOCK, 16>), dim3(count, nrhs / 16), dim3(BLOCK), sh, s, a, first);
-  else if (nr == 4)
-    hipLaunchKernelGGL((k_postm2l<NN, BLOCK, 4>), dim3(count, nrhs / 4), dim3(BLOCK), sh, s, a, first);
-  else
-    hipLaunchKernelGGL((k_postm2l<NN, BLOCK, 1>), dim3(count, nrhs), dim3(BLOCK), sh, s, a, first);
+  if (nr == 16) postm2l_c<NN, BLOCK, 16, 1>(a, s, nrhs);
+  else if (nr == 4 && a.ncell > 8192) postm2l_c<NN, BLOCK, 4, 2>(a, s, nrhs);
+  else if (nr == 4) postm2l_c<NN, BLOCK, 4, 1>(a, s, nrhs);
+  else if (a.ncell > 8192 || NN > 5) postm2l_c<NN, BLOCK, 1, 4>(a, s, nrhs);
+  else postm2l_c<NN, BLOCK, 1, 2>(a, s, nrhs);
   BB_HIP(hipGetLastError());
   return BBFMM_OK;
 }
