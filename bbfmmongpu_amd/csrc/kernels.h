@@ -164,7 +164,12 @@ void grid_m2l_set_flat(GridM2L *g, int flat);
 // deep_in_grid: the deepest level's multipoles are already in the grids
 // (written by the fused first upward level), so only the levels above are
 // scattered from M
-int grid_m2l_run(GridM2L *g, const real *M, real *L, int ncell, hipStream_t s, hipEvent_t mid, int deep_in_grid = 0);
+// zero_empty: the M of cells without particles is zero (as a solve's P2M and
+// M2M leave it); the offsets that see only those may be left out
+int grid_m2l_run(GridM2L *g, const real *M, real *L, int ncell, hipStream_t s, hipEvent_t mid, int deep_in_grid = 0,
+                 bool zero_empty = false);
+// marks the cells with particles (leafcnt: the leaves' counts), for zero_empty
+int grid_m2l_occupied(GridM2L *g, const int *d_leafcnt, int nleaf, hipStream_t s);
 // the split-BF16 grids of the deepest level, for the fused first upward
 // level to write into: returns 1 and sets hi, lo and the level's first slot
 // when the grid is split-BF16 with 16 vectors and covers that level, else 0
