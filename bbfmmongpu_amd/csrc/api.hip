@@ -292,7 +292,8 @@ static inline hipEvent_t stage_event(bbfmm_amd_plan *p, int st)
 // file layouts.
 static int plan_init_forest(bbfmm_amd_plan *p, const HostForest &f, const real3 *pos, int n, int r,
                             const real *K, const real *U, const real *Tkz, const real *Kw, const real *Cw,
-                            real homogen, int nrhs, hipStream_t stream)
+                            real homogen, int nrhs, hipStream_t stream,
+                            bool lists = true)
 {
   BB_TRY(check_device());
   if (n < kMinOrder || n > kMaxOrder)
@@ -337,7 +338,7 @@ static int plan_init_forest(bbfmm_amd_plan *p, const HostForest &f, const real3 
   // operators: K4 (four consecutive columns of a row; r = 32 and 256, the
   // ranks with compiled-in kernels), column-major as given (other ranks), U
   // both ways
-  const bool k4 = r == 32 || r == 256;
+  const bool k4 = lists && (r == 32 || r == 256);
   std::vector<real4> K4(k4 ? (size_t)kNumOps * r * r / 4 : 0);
   for (int k = 0; k < (k4 ? kNumOps : 0); k++)
     for (int jb = 0; jb < r / 4; jb++)
@@ -375,8 +376,8 @@ static int plan_init_forest(bbfmm_amd_plan *p, const HostForest &f, const real3 
   BB_TRY(upload(&p->d_leafof, f.leafof.data(), (size_t)N, stream));
   BB_TRY(upload(&p->d_nbr, f.nbr.data(), f.nbr.size(), stream));
   BB_TRY(upload(&p->d_nnbr, f.nnbr.data(), f.nnbr.size(), stream));
-  BB_TRY(upload(&p->d_iinter, f.iinter.data(), f.iinter.size(), stream));
-  if (f.complete) {
+  if (lists) BB_TRY(upload(&p->d_iinter, f.iinter.data(), f.iinter.size(), stream));
+  if (f.complete && lists) {
     BB_TRY(upload(&p->d_inter, f.inter.data(), f.inter.size(), stream));
     BB_TRY(upload(&p->d_kidx, f.kidx.data(), f.kidx.size(), stream));
   }
@@ -424,8 +425,9 @@ static int plan_init_forest(bbfmm_amd_plan *p, const HostForest &f, const real3 
     p->h_leafdepth.resize(nleaf);
     for (int k = 0; k < nleaf; k++) p->h_leafdepth[k] = f.celllev[f.leafcell[k]];
   }
-  {
-    // padded copy for P2P: leaf ranges start at multiples of 4, dummies far away with q = 0
+  if (p->width >= 16) {
+    // padded copy for the 16-vector P2P: leaf ranges start at multiples of 4,
+    // dummies far away with q = 0
     const std::vector<int> &lsta = f.leafsta, &lcnt = f.leafcnt, &nbr = f.nbr, &nnbr = f.nnbr;
     std::vector<int> psta((size_t)nleaf), pcnt((size_t)nleaf), pad_of((size_t)N);
     int run = 0;
@@ -444,7 +446,7 @@ static int plan_init_forest(bbfmm_amd_plan *p, const HostForest &f, const real3 
     }
     for (int i = 0; i < N; i++) ppos[pad_of[i]] = hpos[i];
     BB_TRY(upload(&p->d_ppos, ppos.data(), ppos.size(), stream));
-    if (p->width >= 16) {  // segment tables of the 16-vector P2P kernels
+    {  // segment tables
       std::vector<int2> seg((size_t)nleaf * 27, make_int2(0, 0));
       std::vector<int> nseg((size_t)nleaf, 0);
       for (int k = 0; k < nleaf; k++) {
@@ -563,12 +565,12 @@ static int plan_init_forest(bbfmm_amd_plan *p, const HostForest &f, const real3 
 
 static int plan_init(bbfmm_amd_plan *p, const anotherTree *t, const real3 *pos, int n, int r, const real *K,
                      const real *U, const real *Tkz, const real *Kw, const real *Cw, real homogen, int nrhs,
-                     hipStream_t stream)
+                     hipStream_t stream, bool lists = true)
 {
   if (t->maxlev < kMinLev) return set_error(BBFMM_E_ARG, "maxlev=%d < %d", t->maxlev, kMinLev);
   HostForest f;
-  BB_TRY(forest_from_tree(f, t));
-  return plan_init_forest(p, f, pos, n, r, K, U, Tkz, Kw, Cw, homogen, nrhs, stream);
+  BB_TRY(forest_from_tree(f, t, lists));
+  return plan_init_forest(p, f, pos, n, r, K, U, Tkz, Kw, Cw, homogen, nrhs, stream, lists);
 }
 
 // Particle-row form of a solve: 16 vectors in an MFMA form (fp32 build); the
@@ -1372,10 +1374,11 @@ extern "C" int bbfmm_amd_plan_update_positions(bbfmm_amd_plan *p, const real3 *p
     if (ix != c[0] || iy != c[1] || iz != c[2])
       return set_error(BBFMM_E_RANGE, "particle %d moved to another leaf: build a new plan", p->h_perm[i]);
     hpos[i] = real4{x.x, x.y, x.z, 0};
-    ppos[p->h_pad_of[i]] = hpos[i];
+    if (p->npad > 0) ppos[p->h_pad_of[i]] = hpos[i];
   }
   BB_HIP(hipMemcpyAsync(p->d_pos, hpos.data(), sizeof(real4) * (size_t)N, hipMemcpyHostToDevice, p->stream));
-  BB_HIP(hipMemcpyAsync(p->d_ppos, ppos.data(), sizeof(real4) * ppos.size(), hipMemcpyHostToDevice, p->stream));
+  if (p->npad > 0)
+    BB_HIP(hipMemcpyAsync(p->d_ppos, ppos.data(), sizeof(real4) * ppos.size(), hipMemcpyHostToDevice, p->stream));
   BB_HIP(hipStreamSynchronize(p->stream));
   return BBFMM_OK;
 }
@@ -1638,9 +1641,13 @@ int dropin_plan(DropInPlan &d, anotherTree *t, const real3 *field, real *K, real
                 real *Cw, real homogen, int cutoff, int n)
 {
   d.p = new bbfmm_amd_plan();
-  const int rc = plan_init(d.p, t, field, n, cutoff, K, U, Tkz, Kw, Cw, homogen, 1, nullptr);
+  // the dense-grid M2L reads neither the interaction lists nor the list
+  // kernels' operators: building them took 1.2 of a call's 2.6 ms at 65536
+  // particles (0.84 without, and without the padded copy of the particles)
+  const int scheme = g_default_scheme;
+  const int rc = plan_init(d.p, t, field, n, cutoff, K, U, Tkz, Kw, Cw, homogen, 1, nullptr, scheme != M2L_SCHEME_IJ);
   if (rc != BBFMM_OK) return rc;
-  d.p->scheme = g_default_scheme;
+  d.p->scheme = scheme;
   d.p->form = BBFMM_M2L_PLAIN;
   d.p->l2p_ref = 1;  // the drop-in reproduces the reference's field output, quirks included
   return BBFMM_OK;

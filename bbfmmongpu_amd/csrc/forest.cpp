@@ -39,7 +39,7 @@ static inline void morton_coords(uint32_t m, int bits, int &x, int &y, int &z)
   }
 }
 
-int forest_from_tree(HostForest &f, const anotherTree *t)
+int forest_from_tree(HostForest &f, const anotherTree *t, bool lists)
 {
   const cell *c = t->c;
   const int maxlev = t->maxlev;
@@ -99,22 +99,25 @@ int forest_from_tree(HostForest &f, const anotherTree *t)
     }
   }
   f.iinter.assign(c->iinter, c->iinter + ncell);
-  f.inter.assign((size_t)ncell * kPitchInteraction, 0);
-  f.kidx.assign((size_t)ncell * kPitchInteraction, 0);
   for (int A = 0; A < ncell; A++) {
     if (f.iinter[A] > kPitchInteraction) return set_error(BBFMM_E_ARG, "cell %d has %d interactions", A, f.iinter[A]);
-    for (int i = 0; i < f.iinter[A]; i++)
-      f.inter[(size_t)kPitchInteraction * A + i] = c->interaction[(size_t)c->pitch_interaction * A + i];
     if (A >= f.levsta[kMinLev]) f.ninter += f.iinter[A];
   }
-  int Kt[343];
-  ktable(Kt);
-  anotherTree tv = *t;
-  cell cv = *c;
-  cv.interaction = f.inter.data();
-  cv.pitch_interaction = kPitchInteraction;
-  tv.c = &cv;
-  kindex(&tv, Kt, f.kidx.data());
+  if (lists) {
+    f.inter.assign((size_t)ncell * kPitchInteraction, 0);
+    f.kidx.assign((size_t)ncell * kPitchInteraction, 0);
+    for (int A = 0; A < ncell; A++)
+      for (int i = 0; i < f.iinter[A]; i++)
+        f.inter[(size_t)kPitchInteraction * A + i] = c->interaction[(size_t)c->pitch_interaction * A + i];
+    int Kt[343];
+    ktable(Kt);
+    anotherTree tv = *t;
+    cell cv = *c;
+    cv.interaction = f.inter.data();
+    cv.pitch_interaction = kPitchInteraction;
+    tv.c = &cv;
+    kindex(&tv, Kt, f.kidx.data());
+  }
   f.inst_N.assign(1, f.N);
   f.inst_depth.assign(1, maxlev);
   f.inst_p0.assign(1, 0);

@@ -86,8 +86,9 @@ struct HostForest {
   std::vector<int> cellcls;                   // sparse forests: sibling class of each cell [ncell]
 };
 
-// The reference's complete tree (anotherTree after build_tree).
-int forest_from_tree(HostForest &f, const anotherTree *t);
+// The reference's complete tree (anotherTree after build_tree).  lists: with
+// inter and kidx, which only the list-driven M2L schemes read.
+int forest_from_tree(HostForest &f, const anotherTree *t, bool lists = true);
 
 // ninst instances: N[i] points each, concatenated in pos; depth[i] the
 // uniform depth of instance i, or (depth == NULL or depth[i] <= 0) the
