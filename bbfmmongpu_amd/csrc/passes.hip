@@ -1511,72 +1511,82 @@ __global__ void __launch_bounds__(256) k_down_cols(PassArgs a, int w0, int w1, i
   }
 }
 
-// M2M of sparse forests, one level (n = 4, r = 32): 32 parents per wave, in
+// M2M of sparse forests, one level (n = 4, r = 32): 32 parents per block, in
 // the order of mplist (parents with the same set of children together);
 // S_parent = sum_c T_c^T S_child(c) (anotherUpwardPass.c, as k_m2m) as
-// products over the child classes some parent of the wave has
+// products over the child classes some parent of the block has
 // (v_mfma_f32_32x32x2_f32, A = T_c^T, B = the children's S, zero for absent
-// children; k-step k pairs child nodes k and 32 + k), then M = U^T (Kw .* S_parent) on the matrix unit with the
-// contraction ordered as the accumulators hold the nodes: lane (j, h) owns
-// nodes 32 t + 8 q + 4 h + e of parent j, so k-step (t, q, e) pairs node
-// 32 t + 8 q + e (h = 0) with node 32 t + 8 q + 4 + e (h = 1).
+// children; k-step k pairs child nodes k and 32 + k), wave w taking the
+// classes w and w + 4 (one wave for all eight spent its time on their loads in
+// turn: 34 us at least a level).  The waves' sums are added through LDS, in
+// wave order, and M = U^T (Kw .* S_parent) follows, a 16 x 16 tile a wave.
+// A batch of 1.65M cells, 6 levels: 520 -> 426 us; 16 instances 213 -> 100; 8
+// of up to 16384 points 170 -> 60.
 __global__ void __launch_bounds__(256) k_m2m_cols(PassArgs a, int off, int count)
 {
+  constexpr int LP = 33;  // padded row of 32 parents
+  __shared__ float part[4][64 * LP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int j = lane & 31, h = lane >> 5;
-  const int base = (blockIdx.x * 4 + wave) * 32;
-  if (base >= count) return;  // whole wave; no block-wide barrier below
+  const int base = blockIdx.x * 32;
+  const size_t rs = (size_t)blockIdx.y * a.ncell;
   const bool valid = base + j < count;
   const int P = a.mplist[off + (valid ? base + j : base)];
-  const size_t rs = (size_t)blockIdx.y * a.ncell;
+  int ch[2];
+#pragma unroll
+  for (int k = 0; k < 2; k++) ch[k] = valid ? a.child[(size_t)8 * P + wave + 4 * k] : -1;
+  f32x4 sv[2][8];  // k-step k pairs child node k (h = 0) with 32 + k (h = 1): contiguous rows
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+#pragma unroll
+    for (int q = 0; q < 8; q++) sv[k][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (ch[k] >= 0) {
+      const f32x4 *Sr = reinterpret_cast<const f32x4 *>(a.S + (rs + ch[k]) * 64 + 32 * h);
+#pragma unroll
+      for (int q = 0; q < 8; q++) sv[k][q] = Sr[q];
+    }
+  }
   f32x16 d0, d1;
 #pragma unroll
   for (int e = 0; e < 16; e++) d0[e] = d1[e] = 0.0f;
-  for (int c = 0; c < 8; c++) {
-    const int ch = valid ? a.child[(size_t)8 * P + c] : -1;
-    if (__ballot(ch >= 0) == 0) continue;  // no parent of the wave has this child
-    // k-step k pairs child node k (h = 0) with 32 + k (h = 1): contiguous rows
-    const f32x4 *Sr = reinterpret_cast<const f32x4 *>(a.S + (rs + (ch >= 0 ? ch : P)) * 64 + 32 * h);
-    float sv[32];
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const f32x4 v = Sr[q];
+  for (int k = 0; k < 2; k++) {
+    if (__ballot(ch[k] >= 0) == 0) continue;  // no parent of the block has this child
+    const float *Tm = a.T8m + (size_t)(wave + 4 * k) * 64 * 64 + 64 * 32 * h + j;
 #pragma unroll
-      for (int e = 0; e < 4; e++) sv[4 * q + e] = ch >= 0 ? v[e] : 0.0f;
-    }
-    const float *Tm = a.T8m + (size_t)c * 64 * 64;
+    for (int q = 0; q < 8; q++)
 #pragma unroll
-    for (int k = 0; k < 32; k++) {
-      const float *Tc = Tm + 64 * (32 * h + k);
-      d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(Tc[j], sv[k], d0, 0, 0, 0);
-      d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(Tc[32 + j], sv[k], d1, 0, 0, 0);
-    }
+      for (int e = 0; e < 4; e++) {
+        const float *Tc = Tm + 64 * (4 * q + e);
+        d0 = __builtin_amdgcn_mfma_f32_32x32x2f32(Tc[0], sv[k][q][e], d0, 0, 0, 0);
+        d1 = __builtin_amdgcn_mfma_f32_32x32x2f32(Tc[32], sv[k][q][e], d1, 0, 0, 0);
+      }
   }
-  if (valid) {
-    float *Sp = a.S + (rs + P) * 64 + 4 * h;
+  // lane: nodes 8 (e / 4) + 4 h + e % 4 (and 32 more) of parent j
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      *reinterpret_cast<f32x4 *>(Sp + 8 * q) = f32x4{d0[4 * q], d0[4 * q + 1], d0[4 * q + 2], d0[4 * q + 3]};
-      *reinterpret_cast<f32x4 *>(Sp + 32 + 8 * q) = f32x4{d1[4 * q], d1[4 * q + 1], d1[4 * q + 2], d1[4 * q + 3]};
-    }
+  for (int e = 0; e < 16; e++) {
+    const int node = 8 * (e >> 2) + 4 * h + (e & 3);
+    part[wave][node * LP + j] = d0[e];
+    part[wave][(32 + node) * LP + j] = d1[e];
   }
-  f32x16 mc;
+  __syncthreads();
+  // S of the parents: a wave's lanes take the 64 nodes of a parent
+  for (int i = wave; i < 32; i += 4) {
+    const int o = lane * LP + i;
+    const float s = (part[0][o] + part[1][o]) + (part[2][o] + part[3][o]);
+    const int Pi = __shfl(P, i);
+    if (base + i < count) a.S[(rs + Pi) * 64 + lane] = s;
+    part[0][o] = a.Kw[lane] * s;
+  }
+  __syncthreads();
+  const int c = lane & 15, q = lane >> 4, row0 = 16 * (wave >> 1), col0 = 16 * (wave & 1);
+  f32x4 m = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int e = 0; e < 16; e++) mc[e] = 0.0f;
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const int node = 8 * q + 4 * h + e;
-      mc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.Urm[node * 32 + j], a.Kw[node] * d0[4 * q + e], mc, 0, 0, 0);
-      mc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.Urm[(32 + node) * 32 + j], a.Kw[32 + node] * d1[4 * q + e], mc,
-                                                0, 0, 0);
-    }
-  if (!valid) return;
-  float *Mp = a.M + (rs + P) * 32 + 4 * h;
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-    *reinterpret_cast<f32x4 *>(Mp + 8 * q) = f32x4{mc[4 * q], mc[4 * q + 1], mc[4 * q + 2], mc[4 * q + 3]};
+  for (int k = 0; k < 64; k += 4)
+    m = __builtin_amdgcn_mfma_f32_16x16x4f32(a.Urm[(k + q) * 32 + row0 + c], part[0][(k + q) * LP + col0 + c], m, 0, 0,
+                                             0);
+  const int Pm = __shfl(P, col0 + c);
+  if (base + col0 + c < count) *reinterpret_cast<f32x4 *>(a.M + (rs + Pm) * 32 + row0 + 4 * q) = m;
 }
 #endif
 
@@ -1668,7 +1678,7 @@ int launch_m2m(const PassArgs &a, const int *h_ploff, hipStream_t s, int nrhs)
       hipLaunchKernelGGL(k_m2m_v16, dim3(count), dim3(1024), 0, s, a, off);
 #ifdef SINGLE
     else if (a.mplist && a.T8m && a.n == 4 && a.r == 32)
-      hipLaunchKernelGGL(k_m2m_cols, dim3((count + 127) / 128, nrhs), dim3(256), 0, s, a, off, count);
+      hipLaunchKernelGGL(k_m2m_cols, dim3((count + 31) / 32, nrhs), dim3(256), 0, s, a, off, count);
 #endif
     else
       BB_WITH_ORDER(a.n, hipLaunchKernelGGL((k_m2m<NN, node_block(NN)>), dim3(count, nrhs), dim3(node_block(NN)),
