@@ -10,7 +10,7 @@ M2L, post-M2L, L2L, L2P, P2P) on data already resident in HBM:
   chosen form : 16 charge vectors per solve on one geometry, M2L on MFMA with
                 split-BF16 operands (hi + lo, 3 products) and fp32 accumulate,
                 P2P in fp32 (1/r and the sum over sources);
-  plain form  : the fp32 drop-in (one vector, dense-grid M2L in fp32 FMAs).
+  plain form  : the fp32 drop-in (one vector, dense-grid M2L in fp32 products).
 
 value = per-vector solves per second of the chosen form (whole job).  Errors
 are relative L2 of q*phi against the FP64 direct sum (GPU) on 4,096 sampled
@@ -42,7 +42,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "pmc_traffic_c2.txt")
 CSRC = os.path.join(ROOT, "bbfmmongpu_amd", "csrc")
 # source file of each kernel whose HBM traffic the bench reports
 KERNEL_SOURCE = {"k_m2l_mfma_ss<4,1,true>": "m2l_grid.hip", "k_m2l_mfma_ss_pair<true>": "m2l_grid.hip",
-                 "k_m2l_add_parts": "m2l_grid.hip", "k_p2p_seg16<true>": "p2p.hip", "k_p2p_seg16x<3>": "p2p.hip"}
+                 "k_m2l_add_parts": "m2l_grid.hip", "k_p2p_seg16<true,1>": "p2p.hip", "k_p2p_seg16x<3>": "p2p.hip"}
 # the launches of the split-BF16 M2L stage at C2 (automatic configuration):
 # the deepest level with two 32-column tiles per wave and both class groups
 # in one block, the levels above with one tile and 4 classes per wave and
@@ -321,7 +321,7 @@ def run_c3(args):
         d = B.direct(pos, Q[j], tg)
         errs.append(rel_l2(d, phi[j, tg]))
     log(f"c3: errors vs FP64 direct {errs}")
-    # the fp64 plain solve of vector 0 (dense-grid M2L in fp64 FMAs), kept for
+    # the fp64 plain solve of vector 0 (dense-grid M2L in fp64 products), kept for
     # error comparison: its own error against the direct sum and the chosen
     # form's distance from it
     p64 = B.Plan(pos, 8, U64, K64, nrhs=1, prec="d", stream=stream.cuda_stream).set(
@@ -730,7 +730,7 @@ def main():
                 "issued_mfma_frac": issued / (st_chosen["m2l"] * 1e-3) / (PEAK_BF16_TFLOPS * 1e12),
                 "traffic": tr_m2l, "traffic_source": tr_m2l_src}
     roof_m2l["frac"] = roof_m2l["achieved"] / roof_m2l["peak"]
-    p2p_kernel = "k_p2p_seg16<true>"
+    p2p_kernel = "k_p2p_seg16<true,1>"
     tr_p2p, tr_p2p_src = measured_traffic(p2p_kernel)
     roof_p2p = {"kernel": p2p_kernel, "bound": "valu", "unit": "TFLOP/s",
                 "achieved": p2p_flop / (st_chosen["p2p"] * 1e-3) / 1e12, "peak": PEAK_FP32_TFLOPS,

@@ -148,7 +148,7 @@ int bbfmm_amd_set_default_scheme(int scheme);
 typedef struct bbfmm_amd_plan bbfmm_amd_plan;
 
 /* M2L arithmetic forms */
-#define BBFMM_M2L_PLAIN 0     /* real-precision FMAs (drop-in parity) */
+#define BBFMM_M2L_PLAIN 0     /* real precision (drop-in parity): fp32 or fp64 products */
 #define BBFMM_M2L_BF16X2 1    /* split BF16 hi/lo operands, 3 MFMA products, FP32 accumulate */
 #define BBFMM_M2L_FP32MFMA 2  /* FP32 MFMA */
 #define BBFMM_M2L_FP16X3 3    /* split FP16 operands in three terms (K and each level's M
@@ -172,7 +172,11 @@ typedef struct bbfmm_amd_plan bbfmm_amd_plan;
                                     two 32-column tiles per wave, 8 as 7 with both class
                                     groups in one block sharing the source tiles through
                                     LDS (the 8-class step list), 2/3 class-stationary
-                                    with one/two 32-column tiles per wave */
+                                    with one/two 32-column tiles per wave (FP32 MFMA:
+                                    blocks of 32/64 columns).  0 takes, by the columns
+                                    of the deepest level, 16-column tiles with the
+                                    offsets in slices (full precision; split-BF16 below
+                                    8192 columns) or a source-stationary kernel */
 #define BBFMM_OPT_NEAR_STREAM 8  /* 16-vector MFMA solves: 1 runs P2P on a side stream
                                     beside the downward pass (forked after the M2L, joined
                                     before the scatter), 0 (default) after it; the results
@@ -212,8 +216,9 @@ typedef struct bbfmm_amd_plan bbfmm_amd_plan;
 #define BBFMM_OPT_ADDRESSING 11 /* 0 (default): kernels with two forms read through
                                    scalar-offset buffer loads while their arrays are
                                    below 2 GB and through pointers beyond; 1: through
-                                   pointers always (the split-BF16 source-stationary
-                                   and list M2L, the fp32 16-vector P2P).  Same results */
+                                   pointers always (the split-BF16 source-stationary,
+                                   the list and the full-precision dense-grid M2L, the
+                                   fp32 16-vector P2P).  Same results */
 
 /* Create a plan for N particles at host positions pos (N real3, inside the
    root cell [-L/2,L/2]^3), Chebyshev order n, level modifier lmod (the -d
