@@ -147,7 +147,10 @@ __host__ __device__ constexpr int row_stride()
 // group of NR vectors, one thread per Chebyshev node (n=8: two nodes per
 // thread); S = sum_j q_j Sx Sy Sz, then M = U^T (Kw .* S).
 // The weights of four particles are read at a time; an empty leaf's zeros are
-// only written (150000 particles on a surface, 4 vectors: 41 -> 26.5 us).
+// only written (150000 particles on a surface, 4 vectors: 41 -> 26.5 us).  High
+// orders are bound by LDS, its size (64 particles staged instead of a block's
+// 256) and its reads (two rows of U to each of sw): n = 8, 16 vectors 509 ->
+// 323 us, n = 6 38 -> 30, n = 5 25 -> 19.
 // ROWS: the 16 charges of a particle are one row of a.qt (padded leaf order).
 template <int NN, int BLOCK, int NR, bool ROWS = false>
 __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
@@ -155,7 +158,7 @@ __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
   static_assert(!ROWS || NR == 16, "particle rows hold 16 vectors");
   constexpr int N3 = NN * NN * NN;
   constexpr int NPT = (N3 + BLOCK - 1) / BLOCK;  // nodes per thread (the last may be past N3)
-  constexpr int CH = BLOCK;
+  constexpr int CH = 64;  // particles staged at a time (BLOCK of them held LDS that blocks in flight need)
   constexpr int QS = row_stride<NR>();
   typedef real vec4 __attribute__((ext_vector_type(4)));
   __shared__ __align__(16) real sx[NN][CH], sy[NN][CH], sz[NN][CH];
@@ -257,22 +260,35 @@ __global__ void __launch_bounds__(BLOCK) k_p2m(PassArgs a)
     }
   }
   __syncthreads();
-  // M[k][i] = sum_l U[l][i] sw[l][k]; a thread per (i, group of RS vectors)
-  constexpr int RS = NR >= 8 ? NR / 2 : NR, NG = NR / RS;
-  for (int o = threadIdx.x; o < a.r * NG; o += BLOCK) {
-    const int i = o % a.r, g = o / a.r;
-    real m[RS];
+  // M[k][i] = sum_l U[l][i] sw[l][k]; a thread per (NI rows i, group of RS
+  // vectors): two rows share what is read of sw, which bounds 16 vectors, where
+  // one left the block more than a round of them (n = 7, 8)
+  constexpr int RS = NR >= 8 ? NR / 2 : NR, NG = NR / RS, NI = NR >= 8 && NN >= 7 ? 2 : 1;
+  const int rh = (a.r + NI - 1) / NI;
+  for (int o = threadIdx.x; o < rh * NG; o += BLOCK) {
+    const int i = o % rh, g = o / rh;
+    const int i1 = NI == 2 ? min(i + rh, a.r - 1) : i;
+    real m[NI][RS];
 #pragma unroll
-    for (int k = 0; k < RS; k++) m[k] = 0;
-#pragma unroll 4
+    for (int h = 0; h < NI; h++)
+#pragma unroll
+      for (int k = 0; k < RS; k++) m[h][k] = 0;
+#pragma unroll 8
     for (int l = 0; l < N3; l++) {
-      const real u = a.Urm[(size_t)l * a.r + i];
+      const real u0 = a.Urm[(size_t)l * a.r + i], u1 = NI == 2 ? a.Urm[(size_t)l * a.r + i1] : u0;
 #pragma unroll
-      for (int k = 0; k < RS; k++) m[k] += u * sw[l * NR + g * RS + k];
+      for (int k = 0; k < RS; k++) {
+        const real w = sw[l * NR + g * RS + k];
+        m[0][k] += u0 * w;
+        if (NI == 2) m[NI - 1][k] += u1 * w;
+      }
     }
 #pragma unroll
-    for (int k = 0; k < RS; k++)
-      a.M[(size_t)(rhs0 + g * RS + k) * a.ncell * a.r + (size_t)A * a.r + i] = m[k];
+    for (int k = 0; k < RS; k++) {
+      real *M = a.M + ((size_t)(rhs0 + g * RS + k) * a.ncell + A) * a.r;
+      M[i] = m[0][k];
+      if (NI == 2 && i + rh < a.r) M[i + rh] = m[NI - 1][k];
+    }
   }
 }
 
@@ -1070,25 +1086,41 @@ __global__ void __launch_bounds__(BLOCK) k_postm2l(PassArgs a, int count)
     for (int o = threadIdx.x; o < nc * a.r; o += BLOCK) sl[(o % a.r) * C + o / a.r * NR + k] = L[o];
   }
   __syncthreads();
-  for (int l = threadIdx.x; l < N3; l += BLOCK) {
-    real s[C];
+  // (n = 7, 8: a thread takes both of its nodes at once, sharing the reads of L,
+  // which bound it: n = 8, 16 vectors 330 -> 260 us)
+  constexpr int NPT = (N3 + BLOCK - 1) / BLOCK;
+  int l[NPT];
+  real s[NPT][C];
 #pragma unroll
-    for (int k = 0; k < C; k++) s[k] = 0;
-#pragma unroll(C > 4 ? 4 : 8)
-    for (int i = 0; i < a.r; i++) {
-      const real u = a.Ucm[l + (size_t)N3 * i];
+  for (int p = 0; p < NPT; p++) {
+    l[p] = min((int)threadIdx.x + p * BLOCK, N3 - 1);
 #pragma unroll
-      for (int k = 0; k < C; k++) s[k] += u * sl[i * C + k];
+    for (int k = 0; k < C; k++) s[p][k] = 0;
+  }
+#pragma unroll 8
+  for (int i = 0; i < a.r; i++) {
+    real u[NPT];
+#pragma unroll
+    for (int p = 0; p < NPT; p++) u[p] = a.Ucm[l[p] + (size_t)N3 * i];
+#pragma unroll
+    for (int k = 0; k < C; k++) {
+      const real v = sl[i * C + k];
+#pragma unroll
+      for (int p = 0; p < NPT; p++) s[p][k] += u[p] * v;
     }
-    const real kw = a.Kw[l];
+  }
 #pragma unroll
-    for (int c = 0; c < CB; c++) {
-      if (c >= nc) break;
-      const int level = a.celllev[A0 + c];
-      if (level < kMinLev) continue;
-      const real f = a.scale[level] * kw;
+  for (int c = 0; c < CB; c++) {
+    if (c >= nc) break;
+    const int level = a.celllev[A0 + c];
+    if (level < kMinLev) continue;
 #pragma unroll
-      for (int k = 0; k < NR; k++) a.F[(size_t)(rhs0 + k) * a.ncell * N3 + (size_t)(A0 + c) * N3 + l] = f * s[c * NR + k];
+    for (int p = 0; p < NPT; p++) {
+      if (N3 % BLOCK != 0 && (int)threadIdx.x + p * BLOCK >= N3) continue;
+      const real f = a.scale[level] * a.Kw[l[p]];
+#pragma unroll
+      for (int k = 0; k < NR; k++)
+        a.F[(size_t)(rhs0 + k) * a.ncell * N3 + (size_t)(A0 + c) * N3 + l[p]] = f * s[p][c * NR + k];
     }
   }
 }
@@ -1220,19 +1252,26 @@ __global__ void __launch_bounds__(256) k_l2p(PassArgs a)
 // ROWS: the potentials go to rows of a.phit (padded leaf order) without the
 // output's q factor, which P2P applies; vector 0's far field with that factor
 // goes to a.farfield.
+// n >= 6 and 16 vectors: 4 vectors a lane and 128 lanes a block, as the 14 to
+// 33 KB of F that a block holds leave a CU few blocks (n = 8 289 -> 183 us).
+template <int NN, int NR>
+__host__ __device__ constexpr int l2p_block()
+{
+  return NN >= 6 && NR == 16 ? 128 : 64;
+}
 template <int NN, int NR, bool ROWS = false>
-__global__ void __launch_bounds__(64) k_l2p_leaf(PassArgs a)
+__global__ void __launch_bounds__((l2p_block<NN, NR>())) k_l2p_leaf(PassArgs a)
 {
   static_assert(!ROWS || NR == 16, "particle rows hold 16 vectors");
   constexpr int N3 = NN * NN * NN;
-  constexpr int RS = NR >= 8 ? NR / 2 : NR, NG = NR / RS, PT = 64 / NG;
+  constexpr int BL = l2p_block<NN, NR>(), RS = BL > 64 ? NR / 4 : NR >= 8 ? NR / 2 : NR, NG = NR / RS, PT = BL / NG;
   __shared__ __align__(16) real sf[N3 * NR];
   const int leaf = blockIdx.x;
   const int rhs0 = blockIdx.y * NR;
   const int A = a.leafcell[leaf];
   const real ih = a.leafihalf[leaf];
   const int sta = a.leafsta[leaf], cnt = a.leafcnt[leaf];
-  for (int o = threadIdx.x; o < N3 * NR; o += 64) {
+  for (int o = threadIdx.x; o < N3 * NR; o += BL) {
     const int k = o / N3, l = o % N3;
     sf[l * NR + k] = a.F[(size_t)(rhs0 + k) * a.ncell * N3 + (size_t)A * N3 + l];
   }
@@ -1768,9 +1807,9 @@ static void l2p_t(const PassArgs &a, hipStream_t s, int nrhs)
   }
 #endif
   if (a.rows)
-    hipLaunchKernelGGL((k_l2p_leaf<NN, 16, true>), dim3(a.nleaf, 1), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((k_l2p_leaf<NN, 16, true>), dim3(a.nleaf, 1), dim3(l2p_block<NN, 16>()), 0, s, a);
   else if (nr == 16)
-    hipLaunchKernelGGL((k_l2p_leaf<NN, 16>), dim3(a.nleaf, nrhs / 16), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((k_l2p_leaf<NN, 16>), dim3(a.nleaf, nrhs / 16), dim3(l2p_block<NN, 16>()), 0, s, a);
   else if (nr == 4)
     hipLaunchKernelGGL((k_l2p_leaf<NN, 4>), dim3(a.nleaf, nrhs / 4), dim3(64), 0, s, a);
   else
