@@ -286,6 +286,20 @@ static inline hipEvent_t stage_event(bbfmm_amd_plan *p, int st)
   return p->ev[(size_t)(p->solves % p->nsets) * kEvPerSet + st];
 }
 
+// The padded copy of the particles: every leaf's range filled up to a multiple
+// of 4 with its last particle.
+static void fill_padded(std::vector<real4> &ppos, const std::vector<real4> &hpos, const std::vector<int> &leafof,
+                        const std::vector<int> &pad_of)
+{
+  const size_t N = hpos.size();
+  for (size_t i = 0; i < N; i++) {
+    size_t k = pad_of[i];
+    ppos[k++] = hpos[i];
+    if (i + 1 == N || leafof[i + 1] != leafof[i])
+      for (; k & 3; k++) ppos[k] = hpos[i];
+  }
+}
+
 // Upload everything a solve needs from a forest (one complete tree in the
 // reference's layout, or a batch of sparse instances).  Tkz/Kw/Cw are the
 // caller's Chebyshev weights; K and U are in the reference's column-major
@@ -427,7 +441,7 @@ static int plan_init_forest(bbfmm_amd_plan *p, const HostForest &f, const real3 
   }
   if (p->width >= 16) {
     // padded copy for the 16-vector P2P: leaf ranges start at multiples of 4,
-    // dummies far away with q = 0
+    // filled up with copies of their last particle (q = 0)
     const std::vector<int> &lsta = f.leafsta, &lcnt = f.leafcnt, &nbr = f.nbr, &nnbr = f.nnbr;
     std::vector<int> psta((size_t)nleaf), pcnt((size_t)nleaf), pad_of((size_t)N);
     int run = 0;
@@ -440,11 +454,7 @@ static int plan_init_forest(bbfmm_amd_plan *p, const HostForest &f, const real3 
     p->npad = run;
     p->h_pad_of = pad_of;
     std::vector<real4> ppos((size_t)run);
-    for (auto &x : ppos) {
-      x.x = x.y = x.z = (real)1e6;
-      x.w = 0;
-    }
-    for (int i = 0; i < N; i++) ppos[pad_of[i]] = hpos[i];
+    fill_padded(ppos, hpos, f.leafof, pad_of);
     BB_TRY(upload(&p->d_ppos, ppos.data(), ppos.size(), stream));
     {  // segment tables
       std::vector<int2> seg((size_t)nleaf * 27, make_int2(0, 0));
@@ -828,6 +838,7 @@ static P2PArgs p2p_args(const bbfmm_amd_plan *p)
   pp.nnbr = p->d_nnbr;
   pp.q = p->d_q;
   pp.phi = p->d_phi;
+  pp.beyond = 2 * std::max((real)1, p->L);  // (at least 2: r^2 from there does not vanish in a small root cell)
   pp.use_mfma = p->form != BBFMM_M2L_PLAIN;
   pp.potential = p->potential;
   pp.ppos = p->d_ppos;
@@ -1354,11 +1365,7 @@ extern "C" int bbfmm_amd_plan_update_positions(bbfmm_amd_plan *p, const real3 *p
   if (!p || !pos) return set_error(BBFMM_E_ARG, "null argument");
   const int N = p->N;
   const real half = p->L / 2;
-  std::vector<real4> hpos((size_t)N), ppos((size_t)(p->npad > 0 ? p->npad : 1));
-  for (auto &x : ppos) {
-    x.x = x.y = x.z = (real)1e6;
-    x.w = 0;
-  }
+  std::vector<real4> hpos((size_t)N), ppos((size_t)p->npad);
   for (int i = 0; i < N; i++) {
     const real3 x = pos[p->h_perm[i]];
     const int k = p->h_leafof[i];
@@ -1374,11 +1381,12 @@ extern "C" int bbfmm_amd_plan_update_positions(bbfmm_amd_plan *p, const real3 *p
     if (ix != c[0] || iy != c[1] || iz != c[2])
       return set_error(BBFMM_E_RANGE, "particle %d moved to another leaf: build a new plan", p->h_perm[i]);
     hpos[i] = real4{x.x, x.y, x.z, 0};
-    if (p->npad > 0) ppos[p->h_pad_of[i]] = hpos[i];
   }
   BB_HIP(hipMemcpyAsync(p->d_pos, hpos.data(), sizeof(real4) * (size_t)N, hipMemcpyHostToDevice, p->stream));
-  if (p->npad > 0)
+  if (p->npad > 0) {
+    fill_padded(ppos, hpos, p->h_leafof, p->h_pad_of);
     BB_HIP(hipMemcpyAsync(p->d_ppos, ppos.data(), sizeof(real4) * ppos.size(), hipMemcpyHostToDevice, p->stream));
+  }
   BB_HIP(hipStreamSynchronize(p->stream));
   return BBFMM_OK;
 }
@@ -1767,18 +1775,7 @@ extern "C" void anotherDownwardPass(anotherTree **atree, real3 *field, real3 *so
   const PassArgs a = pass_args(p);
   if (launch_l2l(a, p->h_ploff.data(), s, 1) != BBFMM_OK) return;
   if (launch_l2p(a, s, 1) != BBFMM_OK) return;
-  P2PArgs pp;
-  pp.N = p->N;
-  pp.nleaf = p->nleaf;
-  pp.nrhs = 1;
-  pp.pos = p->d_pos;
-  pp.leafsta = p->d_leafsta;
-  pp.leafcnt = p->d_leafcnt;
-  pp.nbr = p->d_nbr;
-  pp.nnbr = p->d_nnbr;
-  pp.q = p->d_q;
-  pp.phi = p->d_phi;
-  if (launch_p2p(pp, s) != BBFMM_OK) return;
+  if (launch_p2p(p2p_args(p), s) != BBFMM_OK) return;
   if (launch_scatter(p->d_iperm, p->d_phi, p->d_phiout, p->N, 1, s) != BBFMM_OK) return;
   if (hipMemcpy(phi, p->d_phiout, sizeof(real) * p->N, hipMemcpyDeviceToHost) != hipSuccess) {
     set_error(BBFMM_E_HIP, "copy of phi failed");

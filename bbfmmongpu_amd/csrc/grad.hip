@@ -147,8 +147,8 @@ __global__ void __launch_bounds__(BLOCK) k_l2p_grad(GradArgs a)
 // Lanes are 16 targets (l % 16) by 4 source groups (l / 16), NT tiles of
 // targets share the sources that a wave stages in LDS, kStage at a time across
 // leaves (a lane finds its source's leaf by bisection), the next chunk's loads
-// in flight during a chunk's sums, padded to a multiple of 16 with far sources
-// of zero charge.  The W waves of a block take the chunks in turn, their sums
+// in flight during a chunk's sums, padded to a multiple of 16 with copies of its
+// last source that carry no charge.  The W waves of a block take the chunks in turn, their sums
 // added through LDS; the passes over target tiles go to gridDim.y blocks.
 // Bound by the matrix unit and the vector ALUs, which do not overlap in fp32
 // (8 vectors: 8 products of 32 cycles and about 190 cycles of 1/r per 256
@@ -275,16 +275,15 @@ __device__ __forceinline__ void grad_tiles(const GradArgs &a, int tb, int sta, i
       for (int v = 0; v < NR; v++) u.phi[t][v] = 0;
     }
   }
-  // a chunk of kStage sources: a lane's is loaded into registers (one past
-  // the end: far away, without charge), later moved into LDS
+  // a chunk of kStage sources: a lane's is loaded into registers (past the
+  // end, on = false: the last one, without charge), later moved into LDS
   rx4 rp;
   real rc[2 * NR];
   auto load = [&](bool on, int j) {
-    rp = rx4{(real)1e6, (real)1e6, (real)1e6, 0};
+    rp = pos[j];
 #pragma unroll
     for (int k = 0; k < 2 * NR; k++) rc[k] = 0;
     if (on) {
-      rp = pos[j];
 #pragma unroll
       for (int k = 0; k < 2 * NR; k++) rc[k] = charge(k, j);
     }
@@ -296,15 +295,16 @@ __device__ __forceinline__ void grad_tiles(const GradArgs &a, int tb, int sta, i
   };
   // source n of the other leaves, one after the other
   auto load_other = [&](int n) {
+    const int m = min(n, total - 1);
     int b = 0;
 #pragma unroll
     for (int d = 16; d > 0; d >>= 1)
-      if (end[b + d - 1] <= n) b += d;
-    load(n < total, n + delta[b]);
+      if (end[b + d - 1] <= m) b += d;
+    load(n < total, m + delta[b]);
   };
   if (wave == 0)  // the leaf itself
     for (int j = 0; j < cnt; j += kStage) {
-      load(j + lane < cnt, sta + j + lane);
+      load(j + lane < cnt, sta + min(j + lane, cnt - 1));
       put();
       grad_sweep<NR, MFMA, NT, true>(st, min(kStage, (cnt - j + 15) & ~15), ti, h, u);
     }

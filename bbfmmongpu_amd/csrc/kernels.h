@@ -204,10 +204,11 @@ struct P2PArgs {
   // here, in the user's order (perm: leaf order -> user), and phi is only read
   real *out = nullptr;
   const int *perm = nullptr;
+  real beyond;             // (beyond, beyond, beyond): outside the root cell, no particle near it
   int use_mfma = 0;        // fp32: 16 vectors at a time on MFMA
   int potential = 0;       // 1: add the potential, 0: q * potential (the reference's output)
-  // padded particle copy (every leaf padded to a multiple of 4 with far-away,
-  // zero-charge dummies); kernels fall back to the unpadded ones when null
+  // padded particle copy (every leaf padded to a multiple of 4 with zero-charge
+  // copies of its last particle); kernels fall back to the unpadded ones when null
   const real4 *ppos = nullptr;  // [Npad]
   const int2 *seg = nullptr;    // [nleaf][27] (padded start, padded count), self first, empties dropped
   const int *nseg = nullptr;    // [nleaf]

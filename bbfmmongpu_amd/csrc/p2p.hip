@@ -127,11 +127,12 @@ __global__ void k_pack_pq(int N, const real4 *__restrict__ pos, const real *__re
 // added through LDS; the target tiles of a leaf go to gridDim.y blocks, so
 // that few large leaves fill the chip too.  Each wave stages up to kP2PLeaves
 // leaves (64 sources of each) at a time in its own part of LDS, their loads
-// in flight together, padded to a multiple of 8 (16) with far sources of zero
-// charge (no tail masks).  The r != 0 test is applied in the self leaf, which
-// wave 0 stages by itself.
+// in flight together, padded to a multiple of 8 (16) with sources of zero charge
+// outside the root cell (no tail masks; copies of a leaf's last particle, as the
+// 16-vector layout has, cost 64K particles 1.5 us here).  The r != 0 test is
+// applied in the self leaf, which wave 0 stages by itself.
 // Bound by the vector ALUs (7 + NR fp32 operations and a reciprocal square
-// root a pair; fp64: the library rsqrt).  N = 1M, depth 5, one vector: 467 -> 244
+// root a pair; fp64: rsqrt_r).  N = 1M, depth 5, one vector: 467 -> 244
 // us (45 cycles of a SIMD per 64 pairs of whole tiles; the operations alone
 // measure 37); 4096, depth 2 (64 leaves of 64): 192 -> 11.7 us; 65536, depth
 // 4: 33 -> 21.5 us; fp64 100003, depth 4: 117 -> 57.6 us; 4 vectors of 150001
@@ -217,7 +218,7 @@ __device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, in
   auto pad = [&](int n) {  // to a multiple of 2 kGroups
     const int n2 = (n + 2 * kGroups - 1) & ~(2 * kGroups - 1);
     if (lane < n2 - n) {
-      st.s[n + lane] = realx4{(real)1e6, (real)1e6, (real)1e6, 0};
+      st.s[n + lane] = realx4{a.beyond, a.beyond, a.beyond, 0};
       if (NR > 1)
 #pragma unroll
         for (int r = 0; r < NR; r++) st.q[n + lane][r] = 0;
@@ -343,8 +344,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------- padded layout
 // The kernel below reads a private copy of the particles in which every
 // leaf's range starts at a multiple of 4 and is padded to a multiple of 4
-// with dummy sources far outside the root cell and of zero charge, so that
-// its source loops need no tail masks.  seg[leaf][0..nseg) lists the
+// with copies of its last particle of zero charge, so that its source loops
+// need no tail masks.  seg[leaf][0..nseg) lists the
 // (padded start, padded count) of the leaf's non-empty neighbours, the leaf
 // itself first.  Targets are read from the same copy; dummy targets are
 // never written.
