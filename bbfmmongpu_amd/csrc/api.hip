@@ -1247,8 +1247,10 @@ extern "C" int bbfmm_amd_plan_tune(bbfmm_amd_plan *p, int reps, double *table, i
       if (p->r <= kClusterMaxRank) cands.push_back({M2L_SCHEME_CL, 0, kMinLev, 0});
       for (int sw : sws) cands.push_back({M2L_SCHEME_IJ, 0, sw, 0});
     } else if (p->form == BBFMM_M2L_BF16X2) {
+      // 0: the automatic choice, which none of the others is on few columns
+      // (k_m2l_bf16_few) or many (variant 8 below levels of variant 4)
       for (int sw : sws)
-        for (int v = 1; v <= 5; v++) cands.push_back({M2L_SCHEME_IJ, v, sw, 0});
+        for (int v = 0; v <= 5; v++) cands.push_back({M2L_SCHEME_IJ, v, sw, 0});
       // source-stationary with a class-group size of its own above the deepest level
       if (p->maxlev > kMinLev)
         for (int v : {1, 4, 5})

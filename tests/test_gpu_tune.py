@@ -237,6 +237,30 @@ def test_tuned_plan_solves_like_oracle(form, nrhs, ops4, cuda):
     plan.close()
 
 
+@pytest.mark.parametrize("form", [0, 1, 2, 3])
+@pytest.mark.parametrize("N,nrhs", [(4096, 16), (50_021, 12), (65_536, 1), (262_144, 16)])
+def test_tuner_considers_the_automatic_configuration(form, N, nrhs, ops4, cuda):
+    """The configuration that a plan has before it is tuned is one of those
+    timed, so that tuning never leaves a slower one: a row of variant 0 (or,
+    for the split-FP16 form, of variant 2 or 3, one of which it is), and the
+    tuned plan has the fastest row's M2L."""
+    import torch
+    import bbfmmongpu_amd as B
+    U, K, _ = ops4
+    pos, Q = O.uniform_inputs(N, seed=5, nrhs=nrhs)
+    q = torch.from_numpy(np.ascontiguousarray(np.atleast_2d(Q).astype(np.float32))).to(cuda)
+    plan = B.Plan(pos, 4, U, K, prec="s", nrhs=nrhs).set(scheme=B.SCHEME_IJ, form=form)
+    phi0 = plan.solve(q).cpu().numpy()
+    table = plan.tune(reps=3)
+    rows = {(int(t[0]), int(t[1]), int(t[2]), int(t[3])): t[4] for t in table}
+    default = [rows[k] for k in ((3, v, 0, 2) for v in ((2, 3) if form == 3 else (0,))) if k in rows]
+    assert default
+    assert min(rows.values()) <= min(default)
+    phi1 = plan.solve(q).cpu().numpy()
+    plan.close()
+    assert O.rel_l2(phi0, phi1) < (3e-5 if form == 1 else 1e-5)
+
+
 def test_tuned_batch_plan(ops4, cuda):
     import bbfmmongpu_amd as B
     from bbfmmongpu_amd import workloads as W
