@@ -1487,11 +1487,12 @@ constexpr int real_max_waves(int rt, int ct) { return rt * ct <= 4 ? 16 : 8; }
 //            fp64 147 x 7: 4 x 2 1291, 2 x 2 1657
 // Slices: 8 (64K one vector 32 us, 2 slices 61), 4 once the blocks alone give
 // several rounds (1M, 4 vectors: 4 slices 426, 8 442), 16 at the smallest.
+// The pointer form takes the same column tiles and slices, so that its sums are
+// the same to the bit, and one row tile a block (n = 8, 16 vectors, 131072
+// particles 15.8 ms, with blocks of 1 x 1 35.8; 1M, one vector 180 us and 191).
 static void real_shape(GridM2L *g)
 {
   GridArgs &a = g->args;
-  // the planes of a k chunk within the 32-bit offsets of the buffer loads
-  a.buf = !g->flat && a.plane * sizeof(real) * (16 / kVW) < ((size_t)1 << 32);
   long long t16 = 0;  // tiles of 16 columns of one class
   for (int l = a.minlev; l <= a.maxlev; l++) t16 += ((1LL << (3 * (l - 1))) * a.nrhs + 15) / 16;
   const long long u = 8 * t16 * a.kt;
@@ -1500,8 +1501,7 @@ static void real_shape(GridM2L *g)
     a.ct = ct;
   };
   constexpr bool f64 = sizeof(real) == 8;
-  if (!a.buf) take(1, 1);
-  else if (g->variant == 2) take(2, 2);  // 32 columns of r = 32
+  if (g->variant == 2) take(2, 2);  // 32 columns of r = 32
   else if (g->variant == 3) take(2, 4);  // 64
   else if (a.kt <= 2) {
     if (f64 && a.kt == 2 && u >= 2 * 1024) take(2, 1);
@@ -1522,6 +1522,13 @@ static void real_shape(GridM2L *g)
   a.blk0[a.maxlev + 1] = groups;
   g->nblocks = 8 * groups * a.nrg;
   a.ws = std::min(g->nblocks >= 2048 ? 4 : g->nblocks >= 128 ? 8 : 16, real_max_waves(a.rt, a.ct));
+  // buffer loads: the planes of a k chunk within their 32-bit offsets
+  a.buf = !g->flat && a.plane * sizeof(real) * (16 / kVW) < ((size_t)1 << 32);
+  if (!a.buf) {
+    a.rt = 1;
+    a.nrg = a.kt;
+    g->nblocks = 8 * groups * a.nrg;
+  }
 }
 
 // Split-BF16 on fewer columns of the deepest level than this runs
@@ -1919,7 +1926,8 @@ void grid_m2l_destroy(GridM2L *g)
 template <int RT, int CT, int KC, bool BUF = true>
 static int launch_real_t(const GridArgs &a, int nblocks, hipStream_t s)
 {
-  constexpr int MAXW = real_max_waves(RT, CT);
+  // (4 column tiles never come with more than 8 slices)
+  constexpr int MAXW = !BUF && CT == 4 ? 8 : real_max_waves(RT, CT);
   const int lds = a.ws > 1 ? (int)(a.ws * RT * CT * 64 * sizeof(realx4)) : 0;
   const auto kernel = k_m2l_real<RT, CT, KC, MAXW, BUF>;
   hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(64 * a.ws), lds, s, a);
@@ -1932,7 +1940,11 @@ static int launch_real_t(const GridArgs &a, int nblocks, hipStream_t s)
 static int launch_real(const GridArgs &a, int nb, hipStream_t s)
 {
   const bool two = a.kt % 2 == 0;
-  if (!a.buf) return launch_real_t<1, 1, 1, false>(a, nb, s);
+  if (!a.buf) {
+    if (a.ct == 1) return launch_real_t<1, 1, 1, false>(a, nb, s);
+    if (a.ct == 2) return launch_real_t<1, 2, 1, false>(a, nb, s);
+    return launch_real_t<1, 4, 1, false>(a, nb, s);
+  }
   switch (a.rt * 10 + a.ct) {
   case 11: return two ? launch_real_t<1, 1, 2>(a, nb, s) : launch_real_t<1, 1, 1>(a, nb, s);
   case 12: return two ? launch_real_t<1, 2, 2>(a, nb, s) : launch_real_t<1, 2, 1>(a, nb, s);

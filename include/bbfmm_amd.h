@@ -218,7 +218,8 @@ typedef struct bbfmm_amd_plan bbfmm_amd_plan;
                                    below 2 GB and through pointers beyond; 1: through
                                    pointers always (the split-BF16 source-stationary,
                                    the list and the full-precision dense-grid M2L, the
-                                   fp32 16-vector P2P).  Same results */
+                                   fp32 16-vector P2P).  Same results, to the bit but
+                                   for the P2P, whose two forms agree to rounding */
 
 /* Create a plan for N particles at host positions pos (N real3, inside the
    root cell [-L/2,L/2]^3), Chebyshev order n, level modifier lmod (the -d

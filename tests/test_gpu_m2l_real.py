@@ -59,6 +59,41 @@ def test_against_list_kernel(prec, r, depth, nrhs, flat, cuda):
     assert err < TOL[prec]
 
 
+@pytest.mark.parametrize("prec,r,depth,nrhs,opts", [c + (dict(form=0),) for c in CASES] + [
+    ("s", 32, 2, 1, dict(form=2, variant=2)), ("s", 32, 3, 16, dict(form=2)), ("s", 32, 3, 16, dict(form=2, variant=2)),
+    ("s", 32, 3, 5, dict(form=2, variant=3)), ("s", 32, 4, 16, dict(form=2, variant=3)), ("s", 256, 3, 16, dict(form=2)),
+])
+def test_pointer_form_same_bits(prec, r, depth, nrhs, opts, cuda):
+    """Only the addressing differs: the same column tiles, offset slices and order of the sums."""
+    import bbfmmongpu_amd as B
+    ncell = (8 ** (depth + 1) - 1) // 7
+    rng = np.random.default_rng(r + nrhs)
+    K = rng.standard_normal(316 * r * r, dtype=np.float32)
+    M = rng.standard_normal((nrhs, ncell, r), dtype=np.float32)
+    out = [_m2l(B, prec, ORDER[r], r, depth, nrhs, K, M, cuda, 0, scheme=B.SCHEME_IJ, flat_loads=flat, **opts)
+           for flat in (False, True)]
+    assert np.abs(out[0]).max() > 0
+    assert np.array_equal(out[0], out[1])
+
+
+def test_pointer_form_same_bits_many_empty_leaves(ops4, cuda):
+    """The same where offsets without particles are left out."""
+    import torch
+    import bbfmmongpu_amd as B
+    from bbfmmongpu_amd import workloads as W
+    U, K, _ = ops4
+    rng = np.random.default_rng(2)
+    pos = W.sphere_surface(20_001, rng)
+    for nrhs in (1, 4):
+        q = torch.from_numpy(rng.uniform(-1, 1, (nrhs, 20_001)).astype(np.float32)).to(cuda)
+        out = []
+        for flat in (False, True):
+            plan = B.Plan(pos, 4, U, K, nrhs=nrhs, lmod=1).set(scheme=B.SCHEME_IJ, flat_loads=flat)
+            out.append(plan.solve(q).cpu().numpy())
+            plan.close()
+        assert np.array_equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("variant,nrhs", [(0, 16), (2, 16), (3, 16), (2, 3), (3, 5)])
 def test_fp32_form_variants(variant, nrhs, cuda):
     import bbfmmongpu_amd as B
