@@ -306,14 +306,18 @@ __device__ __forceinline__ void grad_tiles(const GradArgs &a, int tb, int sta, i
     for (int j = 0; j < cnt; j += kStage) {
       load(j + lane < cnt, sta + min(j + lane, cnt - 1));
       put();
+      wave_sync();
       grad_sweep<NR, MFMA, NT, true>(st, min(kStage, (cnt - j + 15) & ~15), ti, h, u);
+      wave_sync();
     }
   int n = kStage * wave;
   if (n < total) load_other(n + lane);
   for (; n < total; n += kStage * W) {
     put();
     if (n + kStage * W < total) load_other(n + kStage * W + lane);  // in flight during the sums
+    wave_sync();
     grad_sweep<NR, MFMA, NT, false>(st, min(kStage, (total - n + 15) & ~15), ti, h, u);
+    wave_sync();
   }
   // sums over the lane groups (the MFMA potentials are whole already)
   auto groups = [&](real v) {

@@ -16,6 +16,17 @@ __device__ __forceinline__ int xcd_leaf(int b, int nleaf)
   return (b & 7) * (nleaf >> 3) + (b >> 3);
 }
 
+// Between the LDS accesses of one wavefront's lanes: what lanes stored before
+// it, other lanes read after it, and what they read before it, others overwrite
+// after it.  It orders the compiler's code (a wavefront's LDS instructions run
+// in their order) and emits nothing.
+__device__ __forceinline__ void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Everything the pass kernels read, by value (device pointers).
 struct PassArgs {
   int N, n, r, ncell, maxlev, nleaf;

@@ -2455,7 +2455,7 @@ __global__ void __launch_bounds__(256) k_m2l_list_packed(ListArgs g)
       acc[a[i]] = C[i][0];
       acc[a[i] + 4 * ts] = C[i][1];
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
   };
   // the units of R columns
   auto phase = [&](auto rc) {

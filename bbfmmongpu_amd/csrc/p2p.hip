@@ -232,7 +232,10 @@ __device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, in
       real q[NR];
       load(sta + j, n, p, q);
       put(0, n, p, q);
-      p2p_sweep<NR, NT, true>(st, pad(n), h, x, acc);
+      const int n2 = pad(n);
+      wave_sync();
+      p2p_sweep<NR, NT, true>(st, n2, h, x, acc);
+      wave_sync();
     }
   }
   // the other leaves: items (leaf b, 64 sources from j) of this wave
@@ -263,7 +266,12 @@ __device__ __forceinline__ void p2p_tiles(const P2PArgs &a, int rhs0, int nv, in
         put(at, n[g], p[g], q[g]);
         at += n[g];
       }
-    if (at > 0) p2p_sweep<NR, NT, false>(st, pad(at), h, x, acc);
+    if (at > 0) {
+      const int n2 = pad(at);
+      wave_sync();
+      p2p_sweep<NR, NT, false>(st, n2, h, x, acc);
+      wave_sync();
+    }
   }
 #pragma unroll
   for (int t = 0; t < NT; t++)

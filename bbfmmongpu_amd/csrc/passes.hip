@@ -47,14 +47,6 @@ __device__ __forceinline__ void l2p_reference_z(real *sz, int on)
   if (NN % 4 == 3 && on) sz[NN - 1] = sz[NN - 2];
 }
 
-// LDS writes of a wave visible to its other lanes
-__device__ __forceinline__ void wave_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __global__ void k_gather(int N, const int *__restrict__ perm, const real *__restrict__ src,
                          real *__restrict__ dst)
 {
