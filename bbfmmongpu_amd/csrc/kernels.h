@@ -211,8 +211,9 @@ struct P2PArgs {
   const int *nnbr;         // [nleaf]
   const real *q;           // [rhs][N]
   real *phi;               // [rhs][N] (accumulated into)
-  // not null (fewer than 16 vectors, a leaf per wave or block): the sums go
-  // here, in the user's order (perm: leaf order -> user), and phi is only read
+  // not null (vectors by eights or fewer, a leaf per wave or block; refused
+  // otherwise): the sums go here, in the user's order (perm: leaf order ->
+  // user), and phi is only read
   real *out = nullptr;
   const int *perm = nullptr;
   real beyond;             // (beyond, beyond, beyond): outside the root cell, no particle near it

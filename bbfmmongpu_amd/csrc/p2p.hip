@@ -928,7 +928,15 @@ int launch_p2p(const P2PArgs &a, hipStream_t s)
 {
   if (a.nleaf <= 0 || a.N <= 0) return BBFMM_OK;
   int rhs = 0;
-  if (a.leafof && !a.phit && !a.phin) {
+  const bool lane = a.leafof && !a.phit && !a.phin;  // a lane per target particle
+#ifdef SINGLE
+  const bool mfma = a.use_mfma && a.qt && a.ppos && a.seg;  // 16 vectors at a time
+#else
+  const bool mfma = false;
+#endif
+  if (a.out && (lane || (mfma && a.nrhs >= 16)))  // these leave the sums in phi
+    return set_error(BBFMM_E_ARG, "internal: near field asked to scatter by a kernel that does not");
+  if (lane) {
     const int nb = (a.N + 255) / 256;
     while (rhs < a.nrhs) {
       const int left = a.nrhs - rhs;
@@ -952,7 +960,7 @@ int launch_p2p(const P2PArgs &a, hipStream_t s)
     const int left = a.nrhs - rhs;
     if (left >= 16) {
 #ifdef SINGLE
-      if (a.use_mfma && a.qt && a.ppos && a.seg) {
+      if (mfma) {
         if (!a.phit && !a.phin) {  // particle rows arrive filled
           hipLaunchKernelGGL(k_pad_charges16, dim3((a.N + 255) / 256), dim3(256), 0, s, a.N, a.pad_of,
                              a.q + (size_t)rhs * a.N, a.qt);
