@@ -142,7 +142,11 @@ __global__ void __launch_bounds__(BLOCK) k_l2p_grad(GradArgs a)
 // over the particles j of the neighbour leaves with r_kj != 0: the gradient
 // and the near field of the potentials it returns share 1/r (as two kernels,
 // a lane a target and the 16-vector P2P of q and g, they took 818 + 233 us at
-// N = 262144, depth 4, 8 vectors; this one 525).
+// N = 262144, depth 4, 8 vectors; this one 525).  r != 0 is tested in the leaf
+// itself only: coordinates that fall into different leaves differ by an ulp of
+// x + L/2 or more, 3e-8 of a leaf in fp32, so that r^2 between two leaves
+// vanishes only in root cells so small (1e-15 fp32, 3e-146 fp64, twice as
+// large with each level) that 1 / r^3 overflows for every pair.
 //
 // Lanes are 16 targets (l % 16) by 4 source groups (l / 16), NT tiles of
 // targets share the sources that a wave stages in LDS, kStage at a time across

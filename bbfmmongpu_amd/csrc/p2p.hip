@@ -22,8 +22,8 @@ __device__ __forceinline__ real rsqrt_r(real x)
 #else
   // the hardware's estimate (5e-8) and one third-order step: as exact as the
   // library's rsqrt (1.4e-16 at most over 1e-12 .. 100) without its special
-  // cases (x is positive and finite here, or the result is not used), 47
-  // against 60 cycles a wavefront
+  // cases, 47 against 60 cycles a wavefront: x is positive and finite here, or
+  // the result is not used (r^2 overflows in root cells of 1e154: NaN, not 0)
   const double y = __builtin_amdgcn_rsq(x);
   const double e = __builtin_fma(-x * y, y, 1.0);
   return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
@@ -862,6 +862,9 @@ static void p2p_few_t(const P2PArgs &a, int rhs, int nv, hipStream_t s)
 //   fp32, 4 vectors: 262144 4x4 170.5, 4x1 171.9; 65536 2x1 33.6, 2x4 39.7;
 //                    50000 2x4 63.4, 2x8 65.8; 4096 2x8 15.2, 2x4 19.1
 //   fp32, 7 vectors: 1M 4x1 524, 2x1 633; 16384, 512 leaves 2x4 24.1
+//   fp32, 16 vectors of the plain form, as two times 8 (all 16 at once, a lane
+//                    a target: in brackets): 4096 51 (547), 65536 114 (109),
+//                    262144 490 (1082), 1M 1112 (1585)
 //   fp64:            100003, 4096 leaves, 1 vector 4x4 57.4, 4x1 57.6, 4
 //                    vectors 4x1 95.1, 4x4 134; 500000, 32768 leaves, 1
 //                    vector 4x1 191, 4x4 275; 8000, 64 leaves, 1 vector 6x4

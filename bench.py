@@ -760,7 +760,7 @@ def main():
                    "N": N, "n": 4, "r": 32, "maxlev": chosen.maxlev, "nrhs": nrhs,
                    "m2l_scheme": "dense grid (IJ)", "m2l_form": "split-BF16 MFMA (hi+lo, 3 products), fp32 accumulate",
                    "p2p_form": "fp32 (1/r on the vector ALUs, the sum over sources on FP32 MFMA)",
-                   "plain_form": "fp32 drop-in, dense-grid M2L in fp32 FMAs, one vector"},
+                   "plain_form": "fp32 drop-in, dense-grid M2L in fp32 products (matrix unit), one vector"},
         "s_per_solve": s_per_solve_chosen,
         "m2l_gflops": m2l_gflops_chosen,
         "p2p_ginteractions_per_s": p2p_gips_chosen,
